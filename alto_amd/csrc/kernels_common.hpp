@@ -269,7 +269,9 @@ inline int fill_value(T* p, uint64_t n, T v, hipStream_t s)
 template <typename T>
 inline int fill_zero(T* p, uint64_t n, hipStream_t s) { return fill_value<T>(p, n, (T)0, s); }
 
-// entry points implemented in mttkrp.hip
+// entry points implemented in mttkrp.hip and phi.hip
+int check_offsets(const alto_tensor* t, int R);
+int phi_variant();
 int mttkrp_device(alto_tensor* t, int mode, int R, const void* const* U, void* out, int precision, int accumulate,
                   hipStream_t s, int seg);
 int phi_device(alto_tensor* t, int mode, int R, const double* const* U, double* phi, double eps, hipStream_t s, int seg);

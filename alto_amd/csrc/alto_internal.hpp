@@ -177,7 +177,6 @@ namespace alto {
 int build_luts(alto_tensor* t, hipStream_t s);
 size_t pool_in_use(int dev);
 int compute_masks(int nmode, const uint64_t* dims, int W, uint64_t* masks, uint64_t* alto_mask);
-int radix_sort_pairs(uint64_t* keys, int W, uint32_t* payload, uint64_t n, int bits, hipStream_t s);
 int delinearize_all(const alto_tensor* t, uint64_t* coords_dev, hipStream_t s);
 int prepare_mode_streams(alto_tensor* t, int need64, int need32, hipStream_t s);
 int tuned_chunk_log2();

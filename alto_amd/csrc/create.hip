@@ -1,7 +1,6 @@
 // ALTO format construction on gfx950: linearization (bit deposit) and
-// delinearization (bit extract) as byte-LUT bit permutations, a stable LSD
-// radix sort written for wave64, line-balanced partition pointers,
-// partition intervals, conflict-resolution (CR) bits, and the per-mode
+// delinearization (bit extract) as byte-LUT bit permutations, the sort by key
+// (sort.hip), line-balanced partition pointers, partition intervals, conflict-resolution (CR) bits, and the per-mode
 // chunk-ordered nonzero streams consumed by MTTKRP / Phi.
 //
 // Reference behaviour followed: create_alto (include/alto.hpp:108-294),
@@ -17,6 +16,7 @@
 
 #include "alto_internal.hpp"
 #include "kernels_common.hpp"
+#include "sort.hpp"
 
 namespace alto {
 
@@ -231,8 +231,8 @@ int build_luts(alto_tensor* t, hipStream_t s)
                 }
             }
         ALTO_TRY(lut.dev.alloc(lut.host.size() * 8));
+        // (the table stays in `host`: no wait for the copy)
         HIP_TRY(hipMemcpyAsync(lut.dev.p, lut.host.data(), lut.host.size() * 8, hipMemcpyHostToDevice, s));
-        HIP_TRY(hipStreamSynchronize(s));
         return ALTO_OK;
     };
     int map_delin[128], map_lin[128];
@@ -287,21 +287,23 @@ struct DimArr {
 };
 
 // linearize (include/alto.hpp:184-204): pack the coordinates, then permute
-// the packed bits into ALTO key order; vals cast to ValType.
+// the packed bits into ALTO key order.  Coordinates must lie inside dims (the
+// reference asserts it in CreateSparseTensor, src/sptensor.cpp:276-281); a
+// violation sets *bad.
 template <int PW, int W>
-__global__ void __launch_bounds__(256) k_linearize(CoordPtrs cp, int nmode, PackLayout L, const double* __restrict__ vin,
-                                                   int val_u64, LutRef g_lut, uint64_t n,
-                                                   uint64_t* __restrict__ keys, double* __restrict__ vout,
-                                                   uint32_t* __restrict__ payload)
+__global__ void __launch_bounds__(256) k_linearize(CoordPtrs cp, int nmode, DimArr dims, PackLayout L, LutRef g_lut,
+                                                   uint64_t n, uint64_t* __restrict__ keys, int* __restrict__ bad)
 {
     extern __shared__ uint64_t s_lut[];
     const uint64_t* lut = stage_lut<W>(s_lut, g_lut);
+    int out = 0;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
         uint64_t pk[PW];
 #pragma unroll
         for (int w = 0; w < PW; ++w) pk[w] = 0;
         for (int m = 0; m < nmode; ++m) {
             uint64_t c = cp.c[m][i];
+            out |= c >= dims.d[m];
             int o = L.off[m];
             if (PW == 1) {
                 pk[0] |= c << o;
@@ -318,21 +320,8 @@ __global__ void __launch_bounds__(256) k_linearize(CoordPtrs cp, int nmode, Pack
         lut_apply<PW, W>(lut, g_lut.nb, pk, k);
 #pragma unroll
         for (int w = 0; w < W; ++w) keys[i * W + w] = k[w];
-        if (vout) {
-            double v = vin[i];
-            vout[i] = val_u64 ? (double)(unsigned long long)v : v;
-        }
-        if (payload) payload[i] = (uint32_t)i;
     }
-}
-
-// coordinates must lie inside dims (the reference asserts it in
-// CreateSparseTensor, src/sptensor.cpp:276-281); a violation sets *bad
-__global__ void __launch_bounds__(256) k_validate(CoordPtrs cp, int nmode, DimArr dims, uint64_t n, int* __restrict__ bad)
-{
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-        for (int m = 0; m < nmode; ++m)
-            if (cp.c[m][i] >= dims.d[m]) atomicOr(bad, 1);
+    if (out) atomicOr(bad, 1);
 }
 
 // generic bit permutation of an array of keys (pdep / pext of all modes)
@@ -417,248 +406,80 @@ static size_t lut_smem(const BitPermLut& L)
     return b <= 48 * 1024 ? b : 0;
 }
 
-// ------------------------------------------------------------------ radix sort
-// Stable LSD radix sort, 8-bit digits, tiles of 256 threads x 16 keys with a
-// striped layout (key j*256+t of a tile belongs to round j, lane order t):
-// per-round wave ranks come from 8 ballots (match on the digit), cross-wave
-// offsets from per-wave digit counts in LDS.
-constexpr int RS_THREADS = 256;
-constexpr int RS_ITEMS = 16;
-constexpr int RS_TILE = RS_THREADS * RS_ITEMS;
-constexpr int RS_WAVES = RS_THREADS / 64;
-
-template <int W>
-__device__ inline unsigned digit_of(const uint64_t* keys, uint64_t i, int shift)
-{
-    uint64_t w = keys[i * W + (shift >> 6)];
-    return (unsigned)(w >> (shift & 63)) & 0xffu;
-}
-
-template <int W>
-__global__ void __launch_bounds__(RS_THREADS) k_rs_hist(const uint64_t* __restrict__ keys, uint64_t n, int shift,
-                                                        uint32_t* __restrict__ hist, int nblocks)
-{
-    __shared__ uint32_t h[256];
-    h[threadIdx.x] = 0;
-    __syncthreads();
-    uint64_t base = (uint64_t)blockIdx.x * RS_TILE;
-#pragma unroll 4
-    for (int j = 0; j < RS_ITEMS; ++j) {
-        uint64_t i = base + (uint64_t)j * RS_THREADS + threadIdx.x;
-        if (i < n) atomicAdd(&h[digit_of<W>(keys, i, shift)], 1u);
-    }
-    __syncthreads();
-    hist[(size_t)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
-}
-
-// exclusive scan, three phases over tiles of 1024 elements
-__global__ void __launch_bounds__(1024) k_scan_tiles(uint32_t* __restrict__ a, uint64_t m, uint32_t* __restrict__ sums)
-{
-    __shared__ uint32_t s[1024];
-    uint64_t i = (uint64_t)blockIdx.x * 1024 + threadIdx.x;
-    uint32_t v = i < m ? a[i] : 0;
-    s[threadIdx.x] = v;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-        uint32_t t = threadIdx.x >= (unsigned)off ? s[threadIdx.x - off] : 0;
-        __syncthreads();
-        s[threadIdx.x] += t;
-        __syncthreads();
-    }
-    if (i < m) a[i] = s[threadIdx.x] - v;
-    if (threadIdx.x == 1023) sums[blockIdx.x] = s[1023];
-}
-
-__global__ void __launch_bounds__(1024) k_scan_sums(uint32_t* __restrict__ sums, int nt)
-{
-    // single block: sequential chunks of 1024
-    __shared__ uint32_t s[1024];
-    __shared__ uint32_t carry;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (int base = 0; base < nt; base += 1024) {
-        int i = base + threadIdx.x;
-        uint32_t v = i < nt ? sums[i] : 0;
-        s[threadIdx.x] = v;
-        __syncthreads();
-        for (int off = 1; off < 1024; off <<= 1) {
-            uint32_t t = threadIdx.x >= (unsigned)off ? s[threadIdx.x - off] : 0;
-            __syncthreads();
-            s[threadIdx.x] += t;
-            __syncthreads();
-        }
-        if (i < nt) sums[i] = s[threadIdx.x] - v + carry;
-        __syncthreads();
-        if (threadIdx.x == 1023) carry += s[1023];
-        __syncthreads();
-    }
-}
-
-__global__ void __launch_bounds__(1024) k_scan_add(uint32_t* __restrict__ a, uint64_t m, const uint32_t* __restrict__ sums)
-{
-    uint64_t i = (uint64_t)blockIdx.x * 1024 + threadIdx.x;
-    if (i < m) a[i] += sums[blockIdx.x];
-}
-
-template <int W>
-__global__ void __launch_bounds__(RS_THREADS) k_rs_scatter(const uint64_t* __restrict__ keys, const uint32_t* __restrict__ pay,
-                                                           uint64_t n, int shift, const uint32_t* __restrict__ offs,
-                                                           int nblocks, uint64_t* __restrict__ keys_out,
-                                                           uint32_t* __restrict__ pay_out)
-{
-    __shared__ uint32_t running[256];
-    __shared__ uint32_t wcnt[RS_WAVES][256];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    running[t] = offs[(size_t)t * nblocks + blockIdx.x];
-    for (int w = 0; w < RS_WAVES; ++w) wcnt[w][t] = 0;
-    __syncthreads();
-    const uint64_t lt = (1ull << lane) - 1;
-    uint64_t base = (uint64_t)blockIdx.x * RS_TILE;
-    for (int j = 0; j < RS_ITEMS; ++j) {
-        uint64_t i = base + (uint64_t)j * RS_THREADS + t;
-        bool valid = i < n;
-        unsigned d = valid ? digit_of<W>(keys, i, shift) : 0;
-        uint64_t match = __ballot(valid);
-#pragma unroll
-        for (int b = 0; b < 8; ++b) {
-            uint64_t bb = __ballot(valid && ((d >> b) & 1));
-            match &= ((d >> b) & 1) ? bb : ~bb;
-        }
-        unsigned rank = (unsigned)__popcll(match & lt);
-        if (valid && rank == 0) wcnt[wave][d] = (unsigned)__popcll(match);
-        __syncthreads();
-        if (valid) {
-            uint32_t pos = running[d] + rank;
-            for (int w = 0; w < wave; ++w) pos += wcnt[w][d];
-#pragma unroll
-            for (int q = 0; q < W; ++q) keys_out[(uint64_t)pos * W + q] = keys[i * W + q];
-            pay_out[pos] = pay[i];
-        }
-        __syncthreads();
-        uint32_t tot = 0;
-        for (int w = 0; w < RS_WAVES; ++w) {
-            tot += wcnt[w][t];
-            wcnt[w][t] = 0;
-        }
-        running[t] += tot;
-        __syncthreads();
-    }
-}
-
-static int scan_exclusive(uint32_t* a, uint64_t m, DevBuf& tmp, hipStream_t s)
-{
-    uint64_t nt = (m + 1023) / 1024;
-    if (nt > (1ull << 31)) {
-        set_error("scan too large");
-        return ALTO_ERR_UNSUPPORTED;
-    }
-    if (tmp.bytes < nt * 4) ALTO_TRY(tmp.alloc(nt * 4));
-    hipLaunchKernelGGL(k_scan_tiles, dim3((unsigned)nt), dim3(1024), 0, s, a, m, tmp.as<uint32_t>());
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, s, tmp.as<uint32_t>(), (int)nt);
-    hipLaunchKernelGGL(k_scan_add, dim3((unsigned)nt), dim3(1024), 0, s, a, m, tmp.as<uint32_t>());
-    HIP_TRY(hipGetLastError());
-    return ALTO_OK;
-}
-
-// Sorts (keys, payload) by the low `bits` bits of the keys; results end in
-// the input buffers.
-template <int W>
-static int radix_sort_impl(uint64_t* keys, uint32_t* pay, uint64_t n, int bits, hipStream_t s)
-{
-    if (n <= 1 || bits <= 0) return ALTO_OK;
-    if (bits > 64 * W) {
-        set_error("radix sort: %d key bits exceed the %d-bit key", bits, 64 * W);
-        return ALTO_ERR_UNSUPPORTED;
-    }
-    if (n >= (1ull << 32)) {
-        set_error("radix sort supports fewer than 2^32 nonzeros");
-        return ALTO_ERR_UNSUPPORTED;
-    }
-    int nblocks = (int)((n + RS_TILE - 1) / RS_TILE);
-    DevBuf kb, pb, hist, tmp;
-    ALTO_TRY(kb.alloc(n * W * 8));
-    ALTO_TRY(pb.alloc(n * 4));
-    ALTO_TRY(hist.alloc((size_t)256 * nblocks * 4));
-    uint64_t* ka = keys;
-    uint64_t* kz = kb.as<uint64_t>();
-    uint32_t* pa = pay;
-    uint32_t* pz = pb.as<uint32_t>();
-    int passes = (bits + 7) / 8;
-    for (int p = 0; p < passes; ++p) {
-        int shift = p * 8;
-        hipLaunchKernelGGL(k_rs_hist<W>, dim3(nblocks), dim3(RS_THREADS), 0, s, ka, n, shift, hist.as<uint32_t>(), nblocks);
-        ALTO_TRY(scan_exclusive(hist.as<uint32_t>(), (uint64_t)256 * nblocks, tmp, s));
-        hipLaunchKernelGGL(k_rs_scatter<W>, dim3(nblocks), dim3(RS_THREADS), 0, s, ka, pa, n, shift, hist.as<uint32_t>(),
-                           nblocks, kz, pz);
-        HIP_TRY(hipGetLastError());
-        std::swap(ka, kz);
-        std::swap(pa, pz);
-    }
-    if (ka != keys) {
-        HIP_TRY(hipMemcpyAsync(keys, ka, n * W * 8, hipMemcpyDeviceToDevice, s));
-        HIP_TRY(hipMemcpyAsync(pay, pa, n * 4, hipMemcpyDeviceToDevice, s));
-    }
-    HIP_TRY(hipStreamSynchronize(s));
-    return ALTO_OK;
-}
-
-int radix_sort_pairs(uint64_t* keys, int W, uint32_t* payload, uint64_t n, int bits, hipStream_t s)
-{
-    return W == 1 ? radix_sort_impl<1>(keys, payload, n, bits, s) : radix_sort_impl<2>(keys, payload, n, bits, s);
-}
-
 // ------------------------------------------------------------------ post-sort
-__global__ void k_gather_f64(const double* __restrict__ in, const uint32_t* __restrict__ perm, uint64_t n,
-                             double* __restrict__ out)
+// values in ALTO order, cast to ValType
+__global__ void k_gather_vals(const double* __restrict__ in, const uint32_t* __restrict__ perm, uint64_t n, int val_u64,
+                              double* __restrict__ out)
+{
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
+        const double v = in[perm[i]];
+        out[i] = val_u64 ? (double)(unsigned long long)v : v;
+    }
+}
+
+// [first row, last row] before any nonzero: dims[n] and 0 (the reference's
+// empty partition)
+__global__ void k_intervals_init(DimArr dims, int nmode, uint64_t n, unsigned long long* __restrict__ iv)
 {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-        out[i] = in[perm[i]];
+        iv[i] = (i & 1) ? 0ull : (unsigned long long)dims.d[(i >> 1) % nmode];
 }
 
 // partition intervals (include/alto.hpp:874-899): per (partition, mode) the
-// [min, max] row; partition p holds [p*per, min((p+1)*per, nnz)).
+// [min, max] row; partition p holds [p*per, min((p+1)*per, nnz)).  A workgroup
+// takes slices of up to IV_SLICE nonzeros of one partition, each thread keeps
+// its minima and maxima in registers, and a slice ends in one pair of global
+// atomics per mode and wavefront: bound by reading the keys (20M nonzeros,
+// 3 modes: 1600 us with two LDS atomics per nonzero and mode before).
+constexpr uint64_t IV_SLICE = 8192;
 template <int W, int PW>
 __global__ void __launch_bounds__(256) k_intervals(const uint64_t* __restrict__ keys, LutRef g_lut,
-                                                   PackLayout L, uint64_t n, uint64_t per, unsigned long long* __restrict__ iv)
+                                                   PackLayout L, uint64_t n, uint64_t per, uint64_t slices,
+                                                   uint64_t nitems, unsigned long long* __restrict__ iv)
 {
     extern __shared__ uint64_t s_lut[];
-    __shared__ unsigned long long s_min[ALTO_MAXN], s_max[ALTO_MAXN];
     const uint64_t* lut = stage_lut<PW>(s_lut, g_lut);
-    for (uint64_t tile = blockIdx.x; tile * 256 < n; tile += gridDim.x) {
-        uint64_t base = tile * 256;
-        uint64_t p0 = base / per;
-        if (threadIdx.x < ALTO_MAXN) {
-            s_min[threadIdx.x] = ~0ull;
-            s_max[threadIdx.x] = 0;
+    for (uint64_t it = blockIdx.x; it < nitems; it += gridDim.x) {
+        const uint64_t p = it / slices;
+        const uint64_t b = p * per + (it - p * slices) * IV_SLICE;
+        uint64_t e = b + IV_SLICE < (p + 1) * per ? b + IV_SLICE : (p + 1) * per;
+        if (e > n) e = n;
+        if (b >= e) continue;
+        unsigned long long lo[ALTO_MAXN], hi[ALTO_MAXN];
+#pragma unroll
+        for (int m = 0; m < ALTO_MAXN; ++m) {
+            lo[m] = ~0ull;
+            hi[m] = 0;
         }
-        __syncthreads();
-        uint64_t i = base + threadIdx.x;
-        if (i < n) {
+        for (uint64_t i = b + threadIdx.x; i < e; i += 256) {
             uint64_t k[W], pk[PW];
 #pragma unroll
             for (int w = 0; w < W; ++w) k[w] = keys[i * W + w];
             lut_apply<W, PW>(lut, g_lut.nb, k, pk);
-            uint64_t p = i / per;
-            for (int m = 0; m < L.nmode; ++m) {
-                unsigned long long r = field<PW>(pk, L.off[m], L.bits[m]);
-                if (p == p0) {
-                    atomicMin(&s_min[m], r);
-                    atomicMax(&s_max[m], r);
-                } else {
-                    atomicMin(&iv[(p * L.nmode + m) * 2], r);
-                    atomicMax(&iv[(p * L.nmode + m) * 2 + 1], r);
+#pragma unroll
+            for (int m = 0; m < ALTO_MAXN; ++m) {
+                if (m < L.nmode) {
+                    const unsigned long long r = field<PW>(pk, L.off[m], L.bits[m]);
+                    lo[m] = r < lo[m] ? r : lo[m];
+                    hi[m] = r > hi[m] ? r : hi[m];
                 }
             }
         }
-        __syncthreads();
-        if (threadIdx.x < (unsigned)L.nmode) {
-            int m = threadIdx.x;
-            if (s_max[m] >= s_min[m] || s_min[m] != ~0ull) {
-                atomicMin(&iv[(p0 * L.nmode + m) * 2], s_min[m]);
-                atomicMax(&iv[(p0 * L.nmode + m) * 2 + 1], s_max[m]);
+#pragma unroll
+        for (int m = 0; m < ALTO_MAXN; ++m) {
+            if (m < L.nmode) {
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1) {
+                    const unsigned long long a = __shfl_xor(lo[m], o), c = __shfl_xor(hi[m], o);
+                    lo[m] = a < lo[m] ? a : lo[m];
+                    hi[m] = c > hi[m] ? c : hi[m];
+                }
+                if ((threadIdx.x & 63) == 0 && lo[m] != ~0ull) {
+                    atomicMin(&iv[(p * L.nmode + m) * 2], lo[m]);
+                    atomicMax(&iv[(p * L.nmode + m) * 2 + 1], hi[m]);
+                }
             }
         }
-        __syncthreads();
     }
 }
 
@@ -710,17 +531,10 @@ __global__ void k_fill_i32(int* __restrict__ a, uint64_t n, int v)
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) a[i] = v;
 }
 
-__global__ void k_fill_u64(unsigned long long* __restrict__ a, uint64_t n, unsigned long long v0, unsigned long long v1)
-{
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-        a[i] = (i & 1) ? v1 : v0;
-}
-
-// per-mode streams: composite key (chunk << bits_mode) | row
+// rows of one mode in ALTO order, as sort keys
 template <int W, int PW>
-__global__ void __launch_bounds__(256) k_mode_key(const uint64_t* __restrict__ keys, LutRef g_lut,
-                                                  PackLayout L, int mode, int chunk_log2, uint64_t n,
-                                                  uint64_t* __restrict__ ck, uint32_t* __restrict__ pay)
+__global__ void __launch_bounds__(256) k_mode_key(const uint64_t* __restrict__ keys, LutRef g_lut, PackLayout L, int mode,
+                                                  uint64_t n, uint64_t* __restrict__ ck)
 {
     extern __shared__ uint64_t s_lut[];
     const uint64_t* lut = stage_lut<PW>(s_lut, g_lut);
@@ -729,104 +543,158 @@ __global__ void __launch_bounds__(256) k_mode_key(const uint64_t* __restrict__ k
 #pragma unroll
         for (int w = 0; w < W; ++w) k[w] = keys[i * W + w];
         lut_apply<W, PW>(lut, g_lut.nb, k, pk);
-        uint64_t r = field<PW>(pk, L.off[mode], L.bits[mode]);
-        ck[i] = ((i >> chunk_log2) << L.bits[mode]) | r;
-        pay[i] = (uint32_t)i;
+        ck[i] = field<PW>(pk, L.off[mode], L.bits[mode]);
     }
 }
 
+// Packed coordinates and value of each nonzero side by side, in ALTO order:
+// every mode's stream is gathered from these records (one access per nonzero
+// where keys and values apart would take two, and the key's bits are permuted
+// once instead of twice per mode).
 template <int W, int PW>
-__global__ void __launch_bounds__(256) k_mode_gather(const uint64_t* __restrict__ keys, const double* __restrict__ vals,
-                                                     LutRef g_lut, const uint32_t* __restrict__ perm,
-                                                     uint64_t n, uint64_t* __restrict__ pk_out, double* __restrict__ v64,
-                                                     float* __restrict__ v32)
+__global__ void __launch_bounds__(256) k_records(const uint64_t* __restrict__ keys, const double* __restrict__ vals,
+                                                 LutRef g_lut, uint64_t n, uint64_t* __restrict__ rec)
 {
     extern __shared__ uint64_t s_lut[];
     const uint64_t* lut = stage_lut<PW>(s_lut, g_lut);
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
-        uint64_t src = perm[i];
         uint64_t k[W], pk[PW];
 #pragma unroll
-        for (int w = 0; w < W; ++w) k[w] = keys[src * W + w];
+        for (int w = 0; w < W; ++w) k[w] = keys[i * W + w];
         lut_apply<W, PW>(lut, g_lut.nb, k, pk);
 #pragma unroll
-        for (int w = 0; w < PW; ++w) pk_out[i * PW + w] = pk[w];
-        double v = vals[src];
-        if (v64) v64[i] = v;
-        if (v32) v32[i] = (float)v;
+        for (int w = 0; w < PW; ++w) rec[i * (PW + 1) + w] = pk[w];
+        rec[i * (PW + 1) + PW] = (uint64_t)__double_as_longlong(vals[i]);
     }
+}
+
+// Sort key of a mode's stream: (chunk, row of `mode`, row of `amode`) of the
+// nonzero at ALTO position idx[j] (j itself when idx is null; the positions
+// are then left to the sort), without the last field when amode < 0.
+template <typename K, int PW>
+__global__ void __launch_bounds__(256) k_stream_key(const uint64_t* __restrict__ rec, PackLayout L, int mode, int amode,
+                                                    int chunk_log2, uint64_t n, const uint32_t* __restrict__ idx,
+                                                    K* __restrict__ ck, uint32_t* __restrict__ pay)
+{
+    const int ba = amode >= 0 ? L.bits[amode] : 0, bn = L.bits[mode];
+    for (uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += (uint64_t)gridDim.x * blockDim.x) {
+        const uint64_t i = idx ? idx[j] : j;
+        uint64_t pk[PW];
+#pragma unroll
+        for (int w = 0; w < PW; ++w) pk[w] = rec[i * (PW + 1) + w];
+        uint64_t k = ((i >> chunk_log2) << bn) | field<PW>(pk, L.off[mode], bn);
+        if (amode >= 0) k = (k << ba) | field<PW>(pk, L.off[amode], ba);
+        ck[j] = (K)k;
+        if (idx) pay[j] = (uint32_t)i;
+    }
+}
+
+// where a stream's nonzeros go
+struct StreamOut {
+    uint64_t* pk;
+    double* v64;
+    float* v32;
+};
+
+template <int PW>
+__device__ inline void put_nonzero(const uint64_t* __restrict__ rec, uint64_t src, uint64_t dst, const StreamOut& o)
+{
+    uint64_t r[PW + 1];
+#pragma unroll
+    for (int w = 0; w <= PW; ++w) r[w] = rec[src * (PW + 1) + w];
+#pragma unroll
+    for (int w = 0; w < PW; ++w) o.pk[dst * PW + w] = r[w];
+    const double v = __longlong_as_double((long long)r[PW]);
+    if (o.v64) o.v64[dst] = v;
+    if (o.v32) o.v32[dst] = (float)v;
+}
+
+template <int PW>
+__global__ void __launch_bounds__(256) k_mode_gather(const uint64_t* __restrict__ rec, const uint32_t* __restrict__ perm,
+                                                     uint64_t n, StreamOut o)
+{
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
+        put_nonzero<PW>(rec, perm[i], i, o);
 }
 
 // ------------------------------------------------------------------ fiber layout
-// Sort key of a fiber-ordered stream: (chunk, row of `mode`, row of `amode`)
-// of the nonzero at ALTO position idx[j] (j itself when idx is null); the
-// chunk is that of the ALTO position.
-template <int W, int PW>
-__global__ void __launch_bounds__(256) k_fiber_key(const uint64_t* __restrict__ keys, LutRef g_lut, PackLayout L,
-                                                   int mode, int amode, int chunk_log2, uint64_t n,
-                                                   const uint32_t* __restrict__ idx, uint64_t* __restrict__ ck,
-                                                   uint32_t* __restrict__ pay)
+// Whether sorted position i lies in a run (fiber) of at least `min_len` equal
+// keys: its equal neighbours to the left and to the right, each found by
+// bisection (the keys are sorted, so equality ends once).
+template <typename K>
+__device__ inline bool fiber_long(const K* __restrict__ ck, uint64_t n, uint64_t i, uint32_t min_len, uint32_t top)
 {
-    extern __shared__ uint64_t s_lut[];
-    const uint64_t* lut = stage_lut<PW>(s_lut, g_lut);
-    const int ba = L.bits[amode], bn = L.bits[mode];
-    for (uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += (uint64_t)gridDim.x * blockDim.x) {
-        const uint64_t i = idx ? idx[j] : j;
-        uint64_t k[W], pk[PW];
+    const K k = ck[i];
+    const uint32_t want = min_len - 1;
+    uint32_t l = 0, r = 0;
+    for (uint32_t st = top; st; st >>= 1)
+        if (l + st <= want && i >= l + st && ck[i - l - st] == k) l += st;
+    for (uint32_t st = top; st; st >>= 1)
+        if (l + r + st <= want && i + r + st < n && ck[i + r + st] == k) r += st;
+    return l + r >= want;
+}
+
+// The stable split of the sorted nonzeros into those of long fibers and the
+// others: counts per tile, and (after their scan) the nonzeros put at their
+// places -- as positions in perm when it is given, else gathered into the
+// stream.  A tile is FS_ROUNDS rounds of 256 consecutive positions.
+constexpr int FS_ROUNDS = 8;
+constexpr int FS_TILE = 256 * FS_ROUNDS;
+
+template <typename K>
+__global__ void __launch_bounds__(256) k_fiber_count(const K* __restrict__ ck, uint64_t n, uint32_t min_len, uint32_t top,
+                                                     uint32_t* __restrict__ cnt)
+{
+    __shared__ uint32_t s_wave[4];
+    uint32_t c = 0;
 #pragma unroll
-        for (int w = 0; w < W; ++w) k[w] = keys[i * W + w];
-        lut_apply<W, PW>(lut, g_lut.nb, k, pk);
-        const uint64_t r = field<PW>(pk, L.off[mode], bn), a = field<PW>(pk, L.off[amode], ba);
-        ck[j] = (((i >> chunk_log2) << bn | r) << ba) | a;
-        pay[j] = (uint32_t)i;
+    for (int j = 0; j < FS_ROUNDS; ++j) {
+        const uint64_t i = (uint64_t)blockIdx.x * FS_TILE + j * 256 + threadIdx.x;
+        c += (uint32_t)__popcll(__ballot(i < n && fiber_long(ck, n, i, min_len, top)));
     }
+    if ((threadIdx.x & 63) == 0) s_wave[threadIdx.x >> 6] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) cnt[blockIdx.x] = s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
 }
 
-// h[i] = 1 where a fiber starts in the sorted keys
-__global__ void k_fiber_heads(const uint64_t* __restrict__ ck, uint64_t n, uint32_t* __restrict__ h)
+template <typename K, int PW>
+__global__ void __launch_bounds__(256) k_fiber_place(const K* __restrict__ ck, const uint32_t* __restrict__ pay, uint64_t n,
+                                                     uint32_t min_len, uint32_t top, const uint32_t* __restrict__ cnt,
+                                                     const uint32_t* __restrict__ nlong, uint32_t* __restrict__ perm,
+                                                     const uint64_t* __restrict__ rec, StreamOut o)
 {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-        h[i] = (i == 0 || ck[i] != ck[i - 1]) ? 1u : 0u;
-}
-
-// id: in, the exclusive scan of the heads; out, the fiber of each nonzero.
-// fstart[f] = first position of fiber f, fstart[nfibers] = n.
-__global__ void k_fiber_starts(const uint64_t* __restrict__ ck, uint64_t n, uint32_t* __restrict__ id,
-                               uint32_t* __restrict__ fstart)
-{
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
-        const uint32_t head = (i == 0 || ck[i] != ck[i - 1]) ? 1u : 0u;
-        const uint32_t f = id[i] + head - 1;
-        id[i] = f;
-        if (head) fstart[f] = (uint32_t)i;
-        if (i == n - 1) fstart[f + 1] = (uint32_t)n;
+    __shared__ uint32_t s_cnt[FS_ROUNDS * 4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t in = 0;  // bit j: round j's position is in a long fiber
+    uint32_t below[FS_ROUNDS];
+#pragma unroll
+    for (int j = 0; j < FS_ROUNDS; ++j) {
+        const uint64_t i = (uint64_t)blockIdx.x * FS_TILE + j * 256 + threadIdx.x;
+        const bool lg = i < n && fiber_long(ck, n, i, min_len, top);
+        const uint64_t b = __ballot(lg);
+        below[j] = (uint32_t)__popcll(b & ((1ull << lane) - 1));
+        if (lg) in |= 1u << j;
+        if (lane == 0) s_cnt[j * 4 + wave] = (uint32_t)__popcll(b);
     }
-}
-
-__device__ inline uint32_t fiber_long(const uint32_t* id, const uint32_t* fstart, uint64_t i, uint32_t min_len)
-{
-    const uint32_t f = id[i];
-    return fstart[f + 1] - fstart[f] >= min_len ? 1u : 0u;
-}
-
-__global__ void k_fiber_class(const uint32_t* __restrict__ id, const uint32_t* __restrict__ fstart, uint64_t n,
-                              uint32_t min_len, uint32_t* __restrict__ cls)
-{
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-        cls[i] = fiber_long(id, fstart, i, min_len);
-}
-
-// stable split: long-fiber nonzeros to [0, nlong), the rest after them;
-// pos = exclusive scan of the long flags
-__global__ void k_fiber_scatter(const uint32_t* __restrict__ id, const uint32_t* __restrict__ fstart,
-                                const uint32_t* __restrict__ pos, const uint32_t* __restrict__ pay, uint64_t n,
-                                uint32_t min_len, uint32_t* __restrict__ perm, uint64_t* __restrict__ nlong_out)
-{
-    const uint64_t nlong = (uint64_t)pos[n - 1] + fiber_long(id, fstart, n - 1, min_len);
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
-        const uint64_t p = fiber_long(id, fstart, i, min_len) ? pos[i] : nlong + (i - pos[i]);
-        perm[p] = pay[i];
-        if (i == 0) *nlong_out = nlong;
+    __syncthreads();
+    uint32_t run = cnt[blockIdx.x];
+    const uint64_t nl = nlong[0];
+#pragma unroll
+    for (int j = 0; j < FS_ROUNDS; ++j) {
+        uint32_t before = 0, sum = 0;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            if (w < wave) before += s_cnt[j * 4 + w];
+            sum += s_cnt[j * 4 + w];
+        }
+        const uint64_t i = (uint64_t)blockIdx.x * FS_TILE + j * 256 + threadIdx.x;
+        if (i < n) {
+            const uint64_t p = run + before + below[j];  // long nonzeros ahead of i
+            const uint64_t dst = (in >> j) & 1 ? p : nl + (i - p);
+            if (perm) perm[dst] = pay[i];
+            else put_nonzero<PW>(rec, pay[i], dst, o);
+        }
+        run += sum;
     }
 }
 
@@ -875,13 +743,10 @@ __global__ void __launch_bounds__(256) k_row_counts(const uint64_t* __restrict__
     }
 }
 
-__global__ void k_rank_keys(const uint32_t* __restrict__ cnt, uint64_t d, int bits, uint64_t* __restrict__ keys,
-                            uint32_t* __restrict__ pay)
+__global__ void k_rank_keys(const uint32_t* __restrict__ cnt, uint64_t d, int bits, uint64_t* __restrict__ keys)
 {
-    for (uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; r < d; r += (uint64_t)gridDim.x * blockDim.x) {
+    for (uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; r < d; r += (uint64_t)gridDim.x * blockDim.x)
         keys[r] = ((uint64_t)(0xffffffffu - cnt[r]) << bits) | r;
-        pay[r] = (uint32_t)r;
-    }
 }
 
 __global__ void k_rank_scatter(const uint32_t* __restrict__ pay, uint64_t d, uint32_t* __restrict__ rank_row,
@@ -925,6 +790,7 @@ static int rank_streams(alto_tensor* t, hipStream_t s)
         if (t->rank_row[m].p) continue;
         const uint64_t d = t->dims[m];
         DevBuf cnt, keys, pay;
+        SortSpace sp;
         ALTO_TRY(cnt.alloc(d * 4));
         ALTO_TRY(keys.alloc(d * 8));
         ALTO_TRY(pay.alloc(d * 4));
@@ -936,9 +802,9 @@ static int rank_streams(alto_tensor* t, hipStream_t s)
                                t->pack.off[m], t->pack.bits[m], t->ms[m].chunk_log2, cnt.as<uint32_t>());
         });
         hipLaunchKernelGGL(k_rank_keys, dim3(grid_for(d)), dim3(256), 0, s, cnt.as<uint32_t>(), d, t->pack.bits[m],
-                           keys.as<uint64_t>(), pay.as<uint32_t>());
+                           keys.as<uint64_t>());
         HIP_TRY(hipGetLastError());
-        ALTO_TRY(radix_sort_pairs(keys.as<uint64_t>(), 1, pay.as<uint32_t>(), d, 32 + t->pack.bits[m], s));
+        ALTO_TRY(sort_pairs<uint64_t>(keys, pay, true, d, 32 + t->pack.bits[m], sp, s));
         hipLaunchKernelGGL(k_rank_scatter, dim3(grid_for(d)), dim3(256), 0, s, pay.as<uint32_t>(), d,
                            t->rank_row[m].as<uint32_t>(), t->row_rank[m].as<uint32_t>());
         HIP_TRY(hipGetLastError());
@@ -990,7 +856,7 @@ struct HotK {
 template <int PW>
 __global__ void __launch_bounds__(256) k_split_key(const uint64_t* __restrict__ pk, uint64_t n, PackLayout L, int mode,
                                                    HotK hk, int chunk_log2, int cbits, uint64_t* __restrict__ ck,
-                                                   uint32_t* __restrict__ pay, unsigned int* __restrict__ pat_count)
+                                                   unsigned int* __restrict__ pat_count)
 {
     __shared__ unsigned int s_cnt[16];
     if (threadIdx.x < 16) s_cnt[threadIdx.x] = 0;
@@ -1008,7 +874,6 @@ __global__ void __launch_bounds__(256) k_split_key(const uint64_t* __restrict__ 
         }
         const uint64_t r = field<PW>(k, L.off[mode], L.bits[mode]);
         ck[i] = (((pat << cbits) | (i >> chunk_log2)) << L.bits[mode]) | r;
-        pay[i] = (uint32_t)i;
         atomicAdd(&s_cnt[pat], 1u);
     }
     __syncthreads();
@@ -1053,6 +918,7 @@ int split_stream(alto_tensor* t, int mode, const int* hot_k, hipStream_t s)
     HotK hk;
     for (int o = 0; o < ALTO_MAXN - 1; ++o) hk.k[o] = o < no ? hot_k[o] : 0;
     DevBuf ck, pay, cnt, pk2, v64, v32;
+    SortSpace sp;
     ALTO_TRY(ck.alloc(n * 8));
     ALTO_TRY(pay.alloc(n * 4));
     ALTO_TRY(cnt.alloc(64 * 4));
@@ -1062,10 +928,10 @@ int split_stream(alto_tensor* t, int mode, const int* hot_k, hipStream_t s)
     if (M.val32.p) ALTO_TRY(v32.alloc(n * 4));
     RANK_DISPATCH_PW(t->pack.pw, {
         hipLaunchKernelGGL((k_split_key<PW>), dim3(grid_for(n)), dim3(256), 0, s, M.pk.as<uint64_t>(), n, t->pack, mode,
-                           hk, M.chunk_log2, cbits, ck.as<uint64_t>(), pay.as<uint32_t>(), cnt.as<unsigned int>());
+                           hk, M.chunk_log2, cbits, ck.as<uint64_t>(), cnt.as<unsigned int>());
     });
     HIP_TRY(hipGetLastError());
-    ALTO_TRY(radix_sort_pairs(ck.as<uint64_t>(), 1, pay.as<uint32_t>(), n, bits, s));
+    ALTO_TRY(sort_pairs<uint64_t>(ck, pay, true, n, bits, sp, s));
     RANK_DISPATCH_PW(t->pack.pw, {
         hipLaunchKernelGGL((k_split_gather<PW>), dim3(grid_for(n)), dim3(256), 0, s, M.pk.as<uint64_t>(),
                            M.val64.as<double>(), M.val32.as<float>(), pay.as<uint32_t>(), n, pk2.as<uint64_t>(),
@@ -1134,69 +1000,111 @@ static StreamLayout wanted_layout(const alto_tensor* t, int m, int ranked)
     return L;
 }
 
+// waits for a stream at the end of a scope: declared behind buffers that are
+// released there
+struct Drain {
+    hipStream_t s;
+    ~Drain() { (void)hipStreamSynchronize(s); }
+};
+
+static int chunk_bits(uint64_t n, int chunk_log2)
+{
+    const uint64_t nch = chunk_log2 >= 63 ? 1 : (n + (1ull << chunk_log2) - 1) >> chunk_log2;
+    int cb = 0;
+    while ((1ull << cb) < nch) ++cb;
+    return cb;
+}
+
+// Buffers shared by the orderings of a tensor's modes (all sized for nnz)
+struct OrderSpace {
+    DevBuf rec, ck, pay, cnt, nl, perm;
+    SortSpace sort;
+};
+
 // One fiber split: the nonzeros at ALTO positions idx[0, n) (0..n-1 when
 // idx is null) ordered by (chunk, row_m, row_a) and split stably into the
-// nonzeros of fibers of at least `min_len` and the others; the ALTO
-// positions in that order go to perm[0, n), the length of the first part
-// to *nl_dev.
-static int fiber_split(alto_tensor* t, int m, int amode, int chunk_log2, int cb, uint32_t min_len,
-                       const uint32_t* idx, uint64_t n, uint64_t* ck, uint32_t* pay, uint32_t* id, uint32_t* fstart,
-                       uint32_t* cls, uint32_t* perm, DevBuf& tmp, uint64_t* nl_dev, hipStream_t s)
+// nonzeros of fibers of at least `min_len` and the others; their ALTO
+// positions in that order go to perm[0, n), or without perm the nonzeros
+// themselves to `o`.  The length of the first part goes to *nl_dev.
+// Keys of up to 32 bits are sorted as such: two thirds of the bytes per pass.
+template <typename K>
+static int fiber_split(alto_tensor* t, int m, int amode, int chunk_log2, int bits, uint32_t min_len, const uint32_t* idx,
+                       uint64_t n, OrderSpace& w, uint32_t* nl_dev, uint32_t* perm, const StreamOut& o, hipStream_t s)
 {
-    DISPATCH_WPW(t->W, t->pack.pw, {
-        hipLaunchKernelGGL((k_fiber_key<W, PW>), dim3(grid_for(n)), dim3(256), lut_smem(t->delin), s,
-                           t->key.as<uint64_t>(), lutref(t->delin), t->pack, m, amode, chunk_log2, n, idx, ck, pay);
+    const uint64_t* rec = w.rec.as<uint64_t>();
+    RANK_DISPATCH_PW(t->pack.pw, {
+        hipLaunchKernelGGL((k_stream_key<K, PW>), dim3(grid_for(n)), dim3(256), 0, s, rec, t->pack, m, amode, chunk_log2,
+                           n, idx, w.ck.as<K>(), w.pay.as<uint32_t>());
     });
     HIP_TRY(hipGetLastError());
-    ALTO_TRY(radix_sort_pairs(ck, 1, pay, n, cb + t->pack.bits[m] + t->pack.bits[amode], s));
-    hipLaunchKernelGGL(k_fiber_heads, dim3(grid_for(n)), dim3(256), 0, s, ck, n, id);
-    ALTO_TRY(scan_exclusive(id, n, tmp, s));
-    hipLaunchKernelGGL(k_fiber_starts, dim3(grid_for(n)), dim3(256), 0, s, ck, n, id, fstart);
-    hipLaunchKernelGGL(k_fiber_class, dim3(grid_for(n)), dim3(256), 0, s, id, fstart, n, min_len, cls);
-    ALTO_TRY(scan_exclusive(cls, n, tmp, s));
-    hipLaunchKernelGGL(k_fiber_scatter, dim3(grid_for(n)), dim3(256), 0, s, id, fstart, cls, pay, n, min_len, perm,
-                       nl_dev);
+    ALTO_TRY(sort_pairs<K>(w.ck, w.pay, idx == nullptr, n, bits, w.sort, s));
+    uint32_t top = 1;
+    while (top * 2 <= min_len - 1) top *= 2;
+    const uint64_t nt = (n + FS_TILE - 1) / FS_TILE;
+    hipLaunchKernelGGL(k_fiber_count<K>, dim3((unsigned)nt), dim3(256), 0, s, w.ck.as<K>(), n, min_len, top,
+                       w.cnt.as<uint32_t>());
+    HIP_TRY(hipGetLastError());
+    ALTO_TRY(scan_rows(w.cnt.as<uint32_t>(), 1, nt, nl_dev, s));
+    RANK_DISPATCH_PW(t->pack.pw, {
+        hipLaunchKernelGGL((k_fiber_place<K, PW>), dim3((unsigned)nt), dim3(256), 0, s, w.ck.as<K>(),
+                           w.pay.as<uint32_t>(), n, min_len, top, w.cnt.as<uint32_t>(), nl_dev, perm, rec, o);
+    });
     HIP_TRY(hipGetLastError());
     return ALTO_OK;
 }
 
-// Orders the nonzeros of stream m by (chunk, row_m, row_a) and splits them
-// into long- and short-fiber parts; with a second fiber mode b the short
-// part is ordered by (chunk, row_m, row_b) and split again.  The
-// permutation ends in `pay`, the lengths of the fiber parts in *nlong and
-// *nlong2.  Synchronous on `s`.
-static int fiber_order(alto_tensor* t, int m, const StreamLayout& L, DevBuf& ck, DevBuf& pay, hipStream_t s,
-                       uint64_t* nlong, uint64_t* nlong2)
+static int fiber_split_any(alto_tensor* t, int m, int amode, int chunk_log2, uint32_t min_len, const uint32_t* idx,
+                           uint64_t n, OrderSpace& w, uint32_t* nl_dev, uint32_t* perm, const StreamOut& o,
+                           hipStream_t s)
+{
+    const int bits = chunk_bits(t->nnz, chunk_log2) + t->pack.bits[m] + t->pack.bits[amode];
+    return bits <= 32 ? fiber_split<uint32_t>(t, m, amode, chunk_log2, bits, min_len, idx, n, w, nl_dev, perm, o, s)
+                      : fiber_split<uint64_t>(t, m, amode, chunk_log2, bits, min_len, idx, n, w, nl_dev, perm, o, s);
+}
+
+// Orders the nonzeros of stream m by (chunk, row_m, row_a), long fibers first
+// and the others after them, and writes the stream; with a second fiber mode
+// b the others are ordered by (chunk, row_m, row_b) and split again.  The
+// lengths of the fiber parts go to nl_dev[0] and nl_dev[1] (the latter is
+// left alone without a second fiber part).
+static int fiber_order(alto_tensor* t, int m, const StreamLayout& L, OrderSpace& w, uint32_t* nl_dev, const StreamOut& o,
+                       hipStream_t s)
 {
     const uint64_t n = t->nnz;
-    const uint64_t nch = (n + (1ull << L.chunk_log2) - 1) >> L.chunk_log2;
-    int cb = 0;
-    while ((1ull << cb) < nch) ++cb;
-    DevBuf id, fstart, cls, perm, tmp, nl;
-    ALTO_TRY(id.alloc(n * 4));
-    ALTO_TRY(fstart.alloc((n + 1) * 4));
-    ALTO_TRY(cls.alloc(n * 4));
-    ALTO_TRY(perm.alloc(n * 4));
-    ALTO_TRY(nl.alloc(16));
-    uint64_t* ckp = ck.as<uint64_t>();
-    uint32_t *payp = pay.as<uint32_t>(), *permp = perm.as<uint32_t>();
-    ALTO_TRY(fiber_split(t, m, L.fib_mode, L.chunk_log2, cb, (uint32_t)L.fib_min, nullptr, n, ckp, payp,
-                         id.as<uint32_t>(), fstart.as<uint32_t>(), cls.as<uint32_t>(), permp, tmp, nl.as<uint64_t>(),
-                         s));
-    HIP_TRY(hipMemcpyAsync(nlong, nl.p, 8, hipMemcpyDeviceToHost, s));
+    if (L.fib_mode2 < 0)
+        return fiber_split_any(t, m, L.fib_mode, L.chunk_log2, (uint32_t)L.fib_min, nullptr, n, w, nl_dev, nullptr, o, s);
+    if (!w.perm.p) ALTO_TRY(w.perm.alloc(n * 4));
+    uint32_t* perm = w.perm.as<uint32_t>();
+    ALTO_TRY(fiber_split_any(t, m, L.fib_mode, L.chunk_log2, (uint32_t)L.fib_min, nullptr, n, w, nl_dev, perm, o, s));
+    uint32_t nlong = 0;
+    HIP_TRY(hipMemcpyAsync(&nlong, nl_dev, 4, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
-    *nlong2 = 0;
-    const uint64_t rest = n - *nlong;
-    if (L.fib_mode2 >= 0 && rest > 0) {
-        // the short part [nlong, n) of perm holds the ALTO positions it orders
-        const uint64_t o = *nlong;
-        ALTO_TRY(fiber_split(t, m, L.fib_mode2, L.chunk_log2, cb, (uint32_t)L.fib_min, permp + o, rest, ckp + o,
-                             payp + o, id.as<uint32_t>(), fstart.as<uint32_t>(), cls.as<uint32_t>(), permp + o, tmp,
-                             nl.as<uint64_t>() + 1, s));
-        HIP_TRY(hipMemcpyAsync(nlong2, nl.as<uint64_t>() + 1, 8, hipMemcpyDeviceToHost, s));
-    }
-    HIP_TRY(hipMemcpyAsync(pay.p, perm.p, n * 4, hipMemcpyDeviceToDevice, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    if (nlong < n)  // the short part [nlong, n) of perm holds the ALTO positions it orders
+        ALTO_TRY(fiber_split_any(t, m, L.fib_mode2, L.chunk_log2, (uint32_t)L.fib_min, perm + nlong, n - nlong, w,
+                                 nl_dev + 1, perm + nlong, o, s));
+    RANK_DISPATCH_PW(t->pack.pw, {
+        hipLaunchKernelGGL((k_mode_gather<PW>), dim3(grid_for(n)), dim3(256), 0, s, w.rec.as<uint64_t>(), perm, n, o);
+    });
+    HIP_TRY(hipGetLastError());
+    return ALTO_OK;
+}
+
+// The stream of mode m ordered by (chunk, row) into `o`
+template <typename K>
+static int row_order(alto_tensor* t, int m, int chunk_log2, int bits, OrderSpace& w, const StreamOut& o, hipStream_t s)
+{
+    const uint64_t n = t->nnz;
+    RANK_DISPATCH_PW(t->pack.pw, {
+        hipLaunchKernelGGL((k_stream_key<K, PW>), dim3(grid_for(n)), dim3(256), 0, s, w.rec.as<uint64_t>(), t->pack, m,
+                           -1, chunk_log2, n, nullptr, w.ck.as<K>(), nullptr);
+    });
+    HIP_TRY(hipGetLastError());
+    ALTO_TRY(sort_pairs<K>(w.ck, w.pay, true, n, bits, w.sort, s));
+    RANK_DISPATCH_PW(t->pack.pw, {
+        hipLaunchKernelGGL((k_mode_gather<PW>), dim3(grid_for(n)), dim3(256), 0, s, w.rec.as<uint64_t>(),
+                           w.pay.as<uint32_t>(), n, o);
+    });
+    HIP_TRY(hipGetLastError());
     return ALTO_OK;
 }
 
@@ -1206,6 +1114,7 @@ int prepare_mode_streams(alto_tensor* t, int need64, int need32, hipStream_t s)
     const int want_chunk = tuned_chunk_log2();
     if (want_chunk > 0 && want_chunk != t->chunk_log2) t->chunk_log2 = want_chunk;
     const int ranked = det_enabled() ? 0 : (int)rank_applicable(t);
+    int fibers = 0;  // modes ordered by fibers here
     StreamLayout want[ALTO_MAXN];
     bool any = false, reorder = false;
     for (int m = 0; m < t->nmode; ++m) {
@@ -1235,13 +1144,22 @@ int prepare_mode_streams(alto_tensor* t, int need64, int need32, hipStream_t s)
             M.nlong = M.nlong2 = 0;
         }
     }
-    DevBuf ck, pay;
-    ALTO_TRY(ck.alloc(n * 8));
-    ALTO_TRY(pay.alloc(n * 4));
+    OrderSpace w;
+    const Drain drain{s};  // before w goes back to the cache, whichever way out
+    ALTO_TRY(w.rec.alloc(n * (t->pack.pw + 1) * 8));
+    ALTO_TRY(w.ck.alloc(n * 8));
+    ALTO_TRY(w.pay.alloc(n * 4));
+    ALTO_TRY(w.cnt.alloc((n + FS_TILE - 1) / FS_TILE * 4));
+    ALTO_TRY(w.nl.alloc(ALTO_MAXN * 2 * 4));
+    ALTO_TRY(fill_zero(w.nl.as<uint32_t>(), ALTO_MAXN * 2, s));
+    DISPATCH_WPW(t->W, t->pack.pw, {
+        hipLaunchKernelGGL((k_records<W, PW>), dim3(grid_for(n)), dim3(256), lut_smem(t->delin), s,
+                           t->key.as<uint64_t>(), t->vals.as<double>(), lutref(t->delin), n, w.rec.as<uint64_t>());
+    });
+    HIP_TRY(hipGetLastError());
     for (int m = 0; m < t->nmode; ++m) {
         ModeStream& M = t->ms[m];
         if (M.pk.p && (!need64 || M.val64.p) && (!need32 || M.val32.p)) continue;
-        M.chunk_log2 = want[m].chunk_log2;
         M.ranked = 0;
         M.split = 0;
         M.pat_start.clear();
@@ -1251,36 +1169,31 @@ int prepare_mode_streams(alto_tensor* t, int need64, int need32, hipStream_t s)
         if (!M.pk.p) ALTO_TRY(M.pk.alloc(n * t->pack.pw * 8));
         if (w64 && !M.val64.p) ALTO_TRY(M.val64.alloc(n * 8));
         if (w32 && !M.val32.p) ALTO_TRY(M.val32.alloc(n * 4));
-        if (want[m].fib_mode >= 0) {
-            uint64_t nlong = 0, nlong2 = 0;
-            ALTO_TRY(fiber_order(t, m, want[m], ck, pay, s, &nlong, &nlong2));
-            M.fib_mode = want[m].fib_mode;
-            M.fib_mode2 = want[m].fib_mode2;
-            M.fib_min = want[m].fib_min;
-            M.nlong = nlong;
-            M.nlong2 = nlong2;
+        const StreamOut o{M.pk.as<uint64_t>(), w64 ? M.val64.as<double>() : nullptr, w32 ? M.val32.as<float>() : nullptr};
+        const StreamLayout& L = want[m];
+        if (L.fib_mode >= 0) {
+            ALTO_TRY(fiber_order(t, m, L, w, w.nl.as<uint32_t>() + 2 * m, o, s));
+            fibers |= 1 << m;
         } else {
-            uint64_t nchunks = (n + (1ull << M.chunk_log2) - 1) >> M.chunk_log2;
-            int cbits = 0;
-            while ((1ull << cbits) < nchunks) ++cbits;
-            DISPATCH_WPW(t->W, t->pack.pw, {
-                hipLaunchKernelGGL((k_mode_key<W, PW>), dim3(grid_for(n)), dim3(256), lut_smem(t->delin), s,
-                                   t->key.as<uint64_t>(), lutref(t->delin), t->pack, m, M.chunk_log2, n,
-                                   ck.as<uint64_t>(), pay.as<uint32_t>());
-            });
-            HIP_TRY(hipGetLastError());
-            ALTO_TRY(radix_sort_pairs(ck.as<uint64_t>(), 1, pay.as<uint32_t>(), n, t->pack.bits[m] + cbits, s));
-            M.fib_mode = M.fib_mode2 = -1;
-            M.fib_min = 0;
-            M.nlong = M.nlong2 = 0;
+            const int bits = t->pack.bits[m] + chunk_bits(n, L.chunk_log2);
+            if (bits <= 32) ALTO_TRY(row_order<uint32_t>(t, m, L.chunk_log2, bits, w, o, s));
+            else ALTO_TRY(row_order<uint64_t>(t, m, L.chunk_log2, bits, w, o, s));
         }
-        DISPATCH_WPW(t->W, t->pack.pw, {
-            hipLaunchKernelGGL((k_mode_gather<W, PW>), dim3(grid_for(n)), dim3(256), lut_smem(t->delin), s,
-                               t->key.as<uint64_t>(), t->vals.as<double>(), lutref(t->delin),
-                               pay.as<uint32_t>(), n, M.pk.as<uint64_t>(), w64 ? M.val64.as<double>() : nullptr,
-                               w32 ? M.val32.as<float>() : nullptr);
-        });
-        HIP_TRY(hipGetLastError());
+        M.chunk_log2 = L.chunk_log2;
+        M.fib_mode = L.fib_mode;
+        M.fib_mode2 = L.fib_mode2;
+        M.fib_min = L.fib_min;
+        M.nlong = M.nlong2 = 0;
+    }
+    if (fibers) {
+        uint32_t nl[ALTO_MAXN * 2];
+        HIP_TRY(hipMemcpyAsync(nl, w.nl.p, sizeof nl, hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        for (int m = 0; m < t->nmode; ++m)
+            if ((fibers >> m) & 1) {
+                t->ms[m].nlong = nl[2 * m];
+                t->ms[m].nlong2 = nl[2 * m + 1];
+            }
     }
     if (rank_applicable(t)) ALTO_TRY(rank_streams(t, s));
     HIP_TRY(hipStreamSynchronize(s));
@@ -1327,7 +1240,9 @@ static int create_impl(int nmode, const uint64_t* dims, uint64_t nnz, const uint
     }
     ALTO_TRY(build_luts(t, s));
 
-    // inputs to device
+    // inputs to device (the staging buffers, like every temporary here, are
+    // released only after the stream has drained: the allocator hands freed
+    // blocks to other streams)
     DevBuf dcoord[ALTO_MAXN], dvals;
     CoordPtrs cp = {};
     const double* dv = vals;
@@ -1344,40 +1259,27 @@ static int create_impl(int nmode, const uint64_t* dims, uint64_t nnz, const uint
         for (int m = 0; m < nmode; ++m) cp.c[m] = cidx[m];
     }
 
-    {
-        DevBuf bad;
-        ALTO_TRY(bad.alloc(4));
-        ALTO_TRY(fill_zero(bad.as<int>(), 1, s));
-        DimArr da = {};
-        for (int m = 0; m < nmode; ++m) da.d[m] = dims[m];
-        hipLaunchKernelGGL(k_validate, dim3(grid_for(nnz)), dim3(256), 0, s, cp, nmode, da, nnz, bad.as<int>());
-        HIP_TRY(hipGetLastError());
-        int hbad = 0;
-        HIP_TRY(hipMemcpyAsync(&hbad, bad.p, 4, hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
-        if (hbad) {
-            set_error("alto_tensor_create: a coordinate is outside dims");
-            return ALTO_ERR_ARG;
-        }
-    }
     ALTO_TRY(t->key.alloc(nnz * t->W * 8));
     ALTO_TRY(t->vals.alloc(nnz * 8));
-    DevBuf vtmp, pay;
-    ALTO_TRY(vtmp.alloc(nnz * 8));
+    DevBuf pay, bad, iv;
+    SortSpace sp;
+    const Drain drain{s};
     ALTO_TRY(pay.alloc(nnz * 4));
+    ALTO_TRY(bad.alloc(4));
+    ALTO_TRY(fill_zero(bad.as<int>(), 1, s));
+    DimArr da = {};
+    for (int m = 0; m < nmode; ++m) da.d[m] = dims[m];
     DISPATCH_WPW(t->W, t->pack.pw, {
-        hipLaunchKernelGGL((k_linearize<PW, W>), dim3(grid_for(nnz)), dim3(256), lut_smem(t->lin), s, cp, nmode, t->pack, dv,
-                           val_kind == ALTO_VAL_U64, lutref(t->lin), nnz, t->key.as<uint64_t>(),
-                           vtmp.as<double>(), pay.as<uint32_t>());
+        hipLaunchKernelGGL((k_linearize<PW, W>), dim3(grid_for(nnz)), dim3(256), lut_smem(t->lin), s, cp, nmode, da,
+                           t->pack, lutref(t->lin), nnz, t->key.as<uint64_t>(), bad.as<int>());
     });
     HIP_TRY(hipGetLastError());
     // sort_alto: by the ALTO key (unique after duplicate merging; stable otherwise)
-    ALTO_TRY(radix_sort_pairs(t->key.as<uint64_t>(), t->W, pay.as<uint32_t>(), nnz, t->alto_bits, s));
-    hipLaunchKernelGGL(k_gather_f64, dim3(grid_for(nnz)), dim3(256), 0, s, vtmp.as<double>(), pay.as<uint32_t>(), nnz,
-                       t->vals.as<double>());
+    if (t->W == 1) ALTO_TRY(sort_pairs<uint64_t>(t->key, pay, true, nnz, t->alto_bits, sp, s));
+    else ALTO_TRY(sort_pairs<Key128>(t->key, pay, true, nnz, t->alto_bits, sp, s));
+    hipLaunchKernelGGL(k_gather_vals, dim3(grid_for(nnz)), dim3(256), 0, s, dv, pay.as<uint32_t>(), nnz,
+                       val_kind == ALTO_VAL_U64, t->vals.as<double>());
     HIP_TRY(hipGetLastError());
-    // the staging buffers are released only after the stream has drained
-    // (end of this function): the allocator hands freed blocks to other streams
 
     // oidx flag (include/alto.hpp:250-258)
     for (int m = 0; m < nmode; ++m)
@@ -1388,26 +1290,26 @@ static int create_impl(int nmode, const uint64_t* dims, uint64_t nnz, const uint
     t->prtn_ptr.assign(nprtn + 1, 0);
     for (int p = 0; p < nprtn; ++p) t->prtn_ptr[p + 1] = std::min<uint64_t>((uint64_t)(p + 1) * per, nnz);
     {
-        DevBuf iv;
-        uint64_t niv = (uint64_t)nprtn * nmode * 2;
+        const uint64_t niv = (uint64_t)nprtn * nmode * 2;
         ALTO_TRY(iv.alloc(niv * 8));
-        // start = dims[n] (empty partition convention), stop = 0: fill then fix starts
-        std::vector<unsigned long long> init(niv);
-        for (int p = 0; p < nprtn; ++p)
-            for (int m = 0; m < nmode; ++m) {
-                init[(p * nmode + m) * 2] = dims[m];
-                init[(p * nmode + m) * 2 + 1] = 0;
-            }
-        HIP_TRY(hipMemcpyAsync(iv.p, init.data(), niv * 8, hipMemcpyHostToDevice, s));
+        hipLaunchKernelGGL(k_intervals_init, dim3(grid_for(niv)), dim3(256), 0, s, da, nmode, niv,
+                           iv.as<unsigned long long>());
+        const uint64_t slices = (per + IV_SLICE - 1) / IV_SLICE, nitems = (uint64_t)nprtn * slices;
         DISPATCH_WPW(t->W, t->pack.pw, {
-            hipLaunchKernelGGL((k_intervals<W, PW>), dim3(grid_for(nnz, 256, 8192)), dim3(256), lut_smem(t->delin), s,
-                               t->key.as<uint64_t>(), lutref(t->delin), t->pack, nnz, per,
-                               iv.as<unsigned long long>());
+            hipLaunchKernelGGL((k_intervals<W, PW>), dim3((unsigned)std::min<uint64_t>(nitems, 4096)), dim3(256),
+                               lut_smem(t->delin), s, t->key.as<uint64_t>(), lutref(t->delin), t->pack, nnz, per,
+                               slices, nitems, iv.as<unsigned long long>());
         });
         HIP_TRY(hipGetLastError());
         t->intervals.assign(niv, 0);
+        int hbad = 0;
+        HIP_TRY(hipMemcpyAsync(&hbad, bad.p, 4, hipMemcpyDeviceToHost, s));
         HIP_TRY(hipMemcpyAsync(t->intervals.data(), iv.p, niv * 8, hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));
+        if (hbad) {  // nothing so far used a row as an index
+            set_error("alto_tensor_create: a coordinate is outside dims");
+            return ALTO_ERR_ARG;
+        }
     }
 
     // CR bits (include/alto.hpp:930-1027)
@@ -1438,7 +1340,6 @@ static int create_impl(int nmode, const uint64_t* dims, uint64_t nnz, const uint
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipStreamSynchronize(s));
     }
-    HIP_TRY(hipStreamSynchronize(s));
     *out = guard.release();
     return ALTO_OK;
 }
@@ -1526,15 +1427,16 @@ int alto_tensor_export_oidx(const alto_tensor_t* t, int mode, uint64_t* oidx)
     }
     uint64_t n = t->nnz;
     DevBuf ck, pay;
+    SortSpace sp;
     ALTO_TRY(ck.alloc(n * 8));
     ALTO_TRY(pay.alloc(n * 4));
-    // rows with chunk_log2 = 63 -> chunk id 0 for every nonzero: a plain stable sort by row
+    // a plain stable sort by row
     DISPATCH_WPW(t->W, t->pack.pw, {
         hipLaunchKernelGGL((k_mode_key<W, PW>), dim3(grid_for(n)), dim3(256), lut_smem(t->delin), 0, t->key.as<uint64_t>(),
-                           lutref(t->delin), t->pack, mode, 63, n, ck.as<uint64_t>(), pay.as<uint32_t>());
+                           lutref(t->delin), t->pack, mode, n, ck.as<uint64_t>());
     });
     HIP_TRY(hipGetLastError());
-    ALTO_TRY(radix_sort_pairs(ck.as<uint64_t>(), 1, pay.as<uint32_t>(), n, t->pack.bits[mode], 0));
+    ALTO_TRY(sort_pairs<uint64_t>(ck, pay, true, n, t->pack.bits[mode], sp, 0));
     std::vector<uint32_t> h(n);
     HIP_TRY(hipMemcpy(h.data(), pay.p, n * 4, hipMemcpyDeviceToHost));
     for (uint64_t i = 0; i < n; ++i) oidx[i] = h[i];

@@ -19,13 +19,13 @@
 
 namespace alto {
 
-// Nonzeros walked by one lane group: ALTO_TUNE_SEG when set, else a power
-// of two in [512, 4096] (from 256 below 4M nonzeros) sized so that a launch
-// has about 2^21 threads (G lanes per group), doubled for FP32 accumulation.  Long segments cut the
-// flushes -- and with them the atomic traffic on heavily used output rows
-// -- while enough groups remain to fill the chip (measured on MI355X: 512
-// for the 77M-nonzero 3-mode tensor in FP64, 1024 in FP32; 1024-4096 for the
-// 200M-nonzero 5-mode one; 512 for 14M-nonzero rank-8 tensors).
+// Nonzeros walked by one lane group of the kernels that flush every group's
+// rows by itself (Phi, the strided MTTKRP lanes, hot-row streams):
+// ALTO_TUNE_SEG when set, else a power of two in [512, 4096] sized so that a
+// launch has about 2^21 threads (G lanes per group), doubled for FP32
+// accumulation.  Long segments cut the flushes -- and with them the atomic
+// traffic on heavily used output rows -- while enough groups remain to fill
+// the chip.
 static int g_seg = 0;
 int tuned_seg(uint64_t nnz, int G, int acc_bytes)
 {
@@ -47,6 +47,35 @@ int tuned_seg(uint64_t nnz, int G, int acc_bytes)
     while (seg < 4096 && (uint64_t)seg * 3 / 2 < want) seg <<= 1;
     return seg;
 }
+
+// Nonzeros walked by one lane group of the vector-lane MTTKRP kernels (G
+// lanes, E columns per lane), whose workgroups combine their groups' last
+// rows before they flush (flush_last_rows), so that a segment need not be
+// long for the heavy rows' sake.  A group walks its segment in steps that
+// each wait for their gathers; the shorter it is, the more wavefronts hide
+// that.  About 4096 wavefronts (four per SIMD) are enough, more only add
+// flushes: nnz G / 2^18 nonzeros as a power of two, between
+//  - 8, or G / 2 (a workgroup of few wide groups combines little: rank 64,
+//    60K nonzeros: 17 us at 8, 13.4 at 16 and 32) and
+//  - 32 (G <= 4), 64, or 128 (four columns per lane, G >= 32): a workgroup
+//    then covers one to four thousand nonzeros, and the heavy rows' atomics
+//    no longer show.
+// All-mode averages in FP64 at 8, 16, 32, 64, 128, 256 (before, with the rule
+// above and no combining): rank 16, 200K nonzeros 11.2, 12.3, 14.4, 21, 34, 56
+// us (24.6); 1000^3, 1M, rank 16 23, 21, 19, 19, 25, 41 us (24.7); 4 modes,
+// 3M, rank 32 179, 104, 81, 82, 86, 93 us (142); at 32 .. 1024: 20M, rank 32
+// 458, 445, 462, 494, 578, 791 us (664); 76.9M, rank 32 1308, 1230, 1259,
+// 1280, 1349, 1416 us (1471).
+int lane_seg(uint64_t nnz, int G, int E)
+{
+    if (g_seg > 0) return g_seg;
+    const int lo = G / 2 > 8 ? G / 2 : 8;
+    const int hi = E >= 4 || G >= 32 ? 128 : G <= 4 ? 32 : 64;
+    const uint64_t want = nnz * (uint64_t)G >> 18;
+    int seg = lo;
+    while (seg < hi && (uint64_t)seg * 3 / 2 < want) seg <<= 1;
+    return seg;
+}
 static int g_chunk = 0;
 static int g_nt = 0;
 // lane mapping of the MTTKRP kernel; -1 = per element type
@@ -55,7 +84,7 @@ static int g_graphs = 0;
 static int g_hot = 0;
 static int g_hot_block = 512;
 static int g_hot_lds = 32768;
-static int g_narrow_max = 32;
+static int g_narrow_max = -1;  // -1: per element type (lane_cols)
 static int g_narrow_small = 1;
 // Phi kernel: 0 = runtime batch loop with LDS permutes, 1 = compile-time
 // batch with DPP broadcasts (5% faster on the 120M-count CP-APR workload)
@@ -380,7 +409,7 @@ int alto_mttkrp_autotune(alto_tensor_t* t, uint64_t rank, int precision, const v
         best_ms = def_ms;
         // segment lengths within 4x of the size rule's choice (the others
         // measured slower on every tensor tried, up to 10x on large ones)
-        const int h = tuned_seg(t->nnz, group_lanes(R), precision == ALTO_PREC_F64 ? 8 : 4);
+        const int h = lane_seg(t->nnz, group_lanes(R), precision == ALTO_PREC_F64 ? 2 : 4);
         for (int v : variants)
             for (int sg : segs) {
                 if (sg * 4 < h || sg > h * 4) continue;

@@ -21,8 +21,8 @@ struct MttkrpTune {
     int nt = 0;             // non-temporal stream loads
     int hot_block = 512;    // threads per workgroup of the ranked-stream kernel
     int hot_lds = 49152;    // LDS bytes per workgroup for hot rows
-    int narrow_max = 32;    // FP32 / BF16 ranks that use two columns per lane
-    int narrow_small = 1;   // ... and every rank below 4M nonzeros
+    int narrow_max = -1;    // FP32 / BF16 ranks that use two columns per lane, -1 = per element type
+    int narrow_small = 1;   // ... and every rank below 1M nonzeros
 };
 
 // Column mapping of a lane group: strided (lane gl holds c = gl + q*G, so
@@ -40,7 +40,13 @@ typedef float v4f32 __attribute__((ext_vector_type(4)));
 typedef float v2f32 __attribute__((ext_vector_type(2)));
 typedef uint32_t v2u32 __attribute__((ext_vector_type(2)));
 
-template <typename V, typename T> __device__ inline const V* vcast(const T* p) { return reinterpret_cast<const V*>(p); }
+// (global loads of up to 16 bytes need 4-byte alignment only, so rows of any
+// rank can be read in vectors)
+template <typename V, typename T> __device__ inline auto vcast(const T* p)
+{
+    typedef V unaligned __attribute__((aligned(alignof(T) < 4 ? 4 : alignof(T))));
+    return reinterpret_cast<const unaligned*>(p);
+}
 template <typename V, typename T> __device__ inline lds_ptr<V> vcast(lds_ptr<T> p)
 {
     return reinterpret_cast<lds_ptr<V>>(p);
@@ -313,19 +319,80 @@ template <int G, int L> __device__ __forceinline__ float bcast_val(float v)
     return __uint_as_float(bcast32<G, L>(__float_as_uint(v)));
 }
 
-// E = 16 / sizeof(FT) consecutive columns per lane in one 16-byte load; the
-// host guarantees 16-byte aligned rows (R * sizeof(FT) % 16 == 0), so a lane
-// either loads a whole vector or lies beyond the rank
-template <typename FT, typename AT, int E, typename P>
-__device__ __forceinline__ void load16(P row, int gl, int R, AT (&x)[E])
+// First column of the E consecutive ones that lane gl of a group holds (R >= E).
+// Where E does not divide the rank the last lane moves back to the row's last
+// E columns: it shares some with its neighbour, which alone flushes them, and
+// every load is one whole vector inside the row.  Lanes beyond the rank read
+// the same columns and flush none.
+template <int E>
+__device__ __forceinline__ int first_col(int gl, int R) { return min(gl * E, R - E); }
+
+template <typename AT, typename OT, int E>
+__device__ __forceinline__ void flush_cols(OT* out, uint32_t row, int R, int gl, int cb, const AT (&acc)[E])
 {
-    // branch-free: lanes beyond the rank read the row's first vector and
-    // drop it
-    const int c0 = gl * E;
-    const bool in = c0 < R;
-    VecLoad<FT, E>::load(row + (in ? c0 : 0), x);
+    OT* o = out + (uint64_t)row * R + cb;
 #pragma unroll
-    for (int q = 0; q < E; ++q) x[q] = in ? x[q] : (AT)0;
+    for (int q = 0; q < E; ++q)
+        if (cb + q >= gl * E) atomic_add_hw(&o[q], (OT)acc[q]);
+}
+
+// The last row of every lane group of a workgroup, combined before it is
+// flushed.  The workgroup's groups walk consecutive segments, so a heavy row
+// that covers several of them would cost one atomic per group and column on
+// the same addresses; here the first group of each run of equal last rows
+// adds up the run's partial sums (in OT) and flushes once.  That is what lets
+// a launch take short segments, i.e. enough wavefronts to hide the gather
+// latency (lane_seg).  Inside a wavefront the runs are summed by a segmented
+// shuffle reduction, and a run that reaches the wavefront's end goes on into
+// the next ones through LDS (one barrier; a loop over up to 64 groups in LDS
+// instead made a 10K-nonzero launch 3 us longer).  Every thread of the
+// workgroup calls it; cur = 0xffffffff: the group had no nonzeros.
+template <typename AT, typename OT, int G, int E>
+__device__ __forceinline__ void flush_last_rows(OT* out, uint32_t cur, int R, int gl, int cb, const AT (&acc)[E])
+{
+    constexpr int GPW = 64 / G, NW = 4;  // groups per wavefront, wavefronts
+    __shared__ uint32_t s_first[NW], s_last[NW];  // rows of a wavefront's first and last group
+    __shared__ int s_whole[NW];                   // all of its groups hold that row
+    __shared__ __align__(16) OT s_sum[NW][64 / GPW * E];  // the first run's sums
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane / G;
+    OT sum[E];
+#pragma unroll
+    for (int q = 0; q < E; ++q) sum[q] = (OT)acc[q];
+    bool head = true;
+    int end = GPW;  // the group after this group's run
+    if constexpr (GPW > 1) {
+        const uint32_t before = (uint32_t)__shfl_up((int)cur, G);  // by every lane
+        head = g == 0 || before != cur;
+        const uint64_t later = __ballot(head && gl == 0) & ~((2ull << (lane - gl)) - 1);
+        if (later) end = __builtin_ctzll(later) / G;
+#pragma unroll
+        for (int d = 1; d < GPW; d <<= 1) {
+#pragma unroll
+            for (int q = 0; q < E; ++q) {
+                const OT y = __shfl_down(sum[q], d * G);
+                if (g + d < end) sum[q] += y;
+            }
+        }
+    }
+    if (g == 0) {
+        if (gl == 0) {
+            s_first[wave] = cur;
+            s_whole[wave] = end == GPW;
+        }
+#pragma unroll
+        for (int q = 0; q < E; ++q) s_sum[wave][gl * E + q] = sum[q];
+    }
+    if (lane == 63) s_last[wave] = cur;
+    __syncthreads();
+    if (!head || cur == 0xffffffffu || (g == 0 && wave > 0 && s_last[wave - 1] == cur)) return;
+    if (end == GPW) {
+        for (int w = wave + 1; w < NW && s_first[w] == cur; ++w) {
+#pragma unroll
+            for (int q = 0; q < E; ++q) sum[q] += s_sum[w][gl * E + q];
+            if (!s_whole[w]) break;
+        }
+    }
+    flush_cols<OT, OT, E>(out, cur, R, gl, cb, sum);
 }
 
 // The MTTKRP stream kernel with 16-byte lanes: per batch of G nonzeros each
@@ -349,14 +416,15 @@ __device__ __forceinline__ void mttkrp16_body(const StreamArgs<FT, VT, OT>& a, u
     // flight per group at a time
     constexpr int NS = G < 4 ? 4 / G : 1;
     constexpr int B = G * NS;
-    constexpr int J = 4;
+    constexpr int J = E == 8 ? 2 : 4;
     const int lane = threadIdx.x & 63;
     const int gl = lane & (G - 1);
     const uint64_t group = (block * 256 + threadIdx.x) / G;
-    const uint64_t s = group * a.seg;
-    if (s >= a.nnz) return;
+    const uint64_t s0 = group * a.seg;
+    const uint64_t s = s0 < a.nnz ? s0 : a.nnz;
     const uint64_t e = s + a.seg < a.nnz ? s + a.seg : a.nnz;
     const int R = a.rank;
+    const int cb = first_col<E>(gl, R);
 
     AT acc[E];
 #pragma unroll
@@ -416,8 +484,8 @@ __device__ __forceinline__ void mttkrp16_body(const StreamArgs<FT, VT, OT>& a, u
                     constexpr int slot = (j0 + jj) / G, src = (j0 + jj) % G;
                     const uint32_t off = bcast32<G, src>(offs[slot][o]);
                     AT x[E];
-                    if constexpr ((HM >> o) & 1) load16<FT, AT, E>(H + off, gl, R, x);
-                    else load16<FT, AT, E>(U + off, gl, R, x);
+                    if constexpr ((HM >> o) & 1) VecLoad<FT, E>::load(H + off + cb, x);
+                    else VecLoad<FT, E>::load(U + off + cb, x);
 #pragma unroll
                     for (int q = 0; q < E; ++q) prod[jj][q] *= x[q];
                 });
@@ -441,7 +509,7 @@ __device__ __forceinline__ void mttkrp16_body(const StreamArgs<FT, VT, OT>& a, u
             for (int jj = 0; jj < J; ++jj) {
                 if (j0 + jj < cnt) {
                     if (rj[jj] != cur) {
-                        if (cur != 0xffffffffu) flush_row<AT, OT, G, E, true>(a.out, cur, R, gl, acc);
+                        if (cur != 0xffffffffu) flush_cols<AT, OT, E>(a.out, cur, R, gl, cb, acc);
                         cur = rj[jj];
 #pragma unroll
                         for (int q = 0; q < E; ++q) acc[q] = 0;
@@ -452,7 +520,9 @@ __device__ __forceinline__ void mttkrp16_body(const StreamArgs<FT, VT, OT>& a, u
             }
         });
     }
-    if (cur != 0xffffffffu) flush_row<AT, OT, G, E, true>(a.out, cur, R, gl, acc);
+    // (the split streams' kernels keep all of their LDS for staged rows)
+    if constexpr (HM == 0) flush_last_rows<AT, OT, G, E>(a.out, cur, R, gl, cb, acc);
+    else if (cur != 0xffffffffu) flush_cols<AT, OT, E>(a.out, cur, R, gl, cb, acc);
 }
 
 template <typename FT, typename VT, typename AT, typename OT, int G, int E, int PW, int NO, int HM>
@@ -484,16 +554,17 @@ __global__ void __launch_bounds__(256) k_mttkrp_fib(StreamArgs<FT, VT, OT> a, co
 {
     constexpr int NS = G < 4 ? 4 / G : 1;
     constexpr int B = G * NS;
-    constexpr int J = 4;
+    constexpr int J = E == 8 ? 2 : 4;
     const uint64_t block = xcd_block(a.nblocks_real);
     if (block == ~0ull) return;
     const int lane = threadIdx.x & 63;
     const int gl = lane & (G - 1);
     const uint64_t group = (block * 256 + threadIdx.x) / G;
-    const uint64_t s = group * a.seg;
-    if (s >= a.nnz) return;
+    const uint64_t s0 = group * a.seg;
+    const uint64_t s = s0 < a.nnz ? s0 : a.nnz;
     const uint64_t e = s + a.seg < a.nnz ? s + a.seg : a.nnz;
     const int R = a.rank;
+    const int cb = first_col<E>(gl, R);
 
     AT acc[E], ua_last[E];
 #pragma unroll
@@ -556,21 +627,18 @@ __global__ void __launch_bounds__(256) k_mttkrp_fib(StreamArgs<FT, VT, OT> a, co
                     constexpr int slot = (j0 + jj) / G, src = (j0 + jj) % G;
                     const uint32_t off = bcast32<G, src>(offs[slot][o]);
                     AT x[E];
-                    load16<FT, AT, E>(U + off, gl, R, x);
+                    VecLoad<FT, E>::load(U + off + cb, x);
 #pragma unroll
                     for (int q = 0; q < E; ++q) prod[jj][q] *= x[q];
                 });
             });
-            // lanes beyond the rank load the row's first vector and keep it:
-            // they never flush, so no select follows the load
             AT ra[J][E];
             uint32_t ldm = 0;  // positions loaded (uniform)
-            const int c0 = gl * E < R ? gl * E : 0;
 #pragma unroll
             for (int jj = 0; jj < J; ++jj) {
                 const bool head = jj == 0 ? (!have_a || aj[0] != prev_a) : aj[jj] != aj[jj - 1];
                 if (__any(head)) {
-                    VecLoad<FT, E>::load(Ua + aj[jj] + c0, ra[jj]);
+                    VecLoad<FT, E>::load(Ua + aj[jj] + cb, ra[jj]);
                     ldm |= 1u << jj;
                 }
             }
@@ -610,7 +678,7 @@ __global__ void __launch_bounds__(256) k_mttkrp_fib(StreamArgs<FT, VT, OT> a, co
             for (int jj = 0; jj < J; ++jj) {
                 if (j0 + jj < cnt) {
                     if (rj[jj] != cur) {
-                        if (cur != 0xffffffffu) flush_row<AT, OT, G, E, true>(a.out, cur, R, gl, acc);
+                        if (cur != 0xffffffffu) flush_cols<AT, OT, E>(a.out, cur, R, gl, cb, acc);
                         cur = rj[jj];
 #pragma unroll
                         for (int q = 0; q < E; ++q) acc[q] = 0;
@@ -621,7 +689,7 @@ __global__ void __launch_bounds__(256) k_mttkrp_fib(StreamArgs<FT, VT, OT> a, co
             }
         });
     }
-    if (cur != 0xffffffffu) flush_row<AT, OT, G, E, true>(a.out, cur, R, gl, acc);
+    flush_last_rows<AT, OT, G, E>(a.out, cur, R, gl, cb, acc);
 }
 
 // Many MTTKRPs (different tensors, modes, sizes; one rank and lane shape) in
@@ -647,7 +715,38 @@ __global__ void __launch_bounds__(256) k_mttkrp16_batch(BatchTable<FT, VT, OT> t
     mttkrp16_body<FT, VT, AT, OT, G, E, PW, ALTO_MAXN - 1, 0, true>(tab.a[j], block - tab.start[j], hot_smem);
 }
 
-// the vector-lane kernel needs factor rows aligned to the lane's load width
+// Columns per lane of the vector-lane kernels for a tensor of nnz nonzeros;
+// 0: the strided kernel (rank 1, bf16 rows that are not whole dwords).  A
+// wave-wide load costs the vector-memory path the same ~20 cycles for 8- and
+// for 16-byte lanes, so wide lanes halve the gathers' cost; what speaks
+// against them is that a wavefront then holds twice the lane groups, each of
+// which flushes rows and starts fibers at its own positions.
+//   FP64: two columns, 16 bytes.
+//   FP32: four columns from rank 17 on (rank 32: 20M nonzeros, 4 modes, 254 us
+//     per MTTKRP against 328 with two; 76.9M, 3 modes, 755 against 927; rank
+//     16: 205 against 174).
+//   BF16: four from rank 33 on (rank 32: 3M nonzeros 63 us against 50; rank
+//     64: 2M nonzeros 66 against 84).
+// Below 1M nonzeros a launch is bound by latency and flushes and every rank
+// takes two columns (200K nonzeros, 5 modes, rank 32: 17 us against 19).
+template <typename FT, typename VT, typename OT>
+inline int lane_cols(const StreamArgs<FT, VT, OT>& a, uint64_t nnz, int R, const MttkrpTune& k)
+{
+    constexpr bool F64 = std::is_same<FT, double>::value, BF16 = std::is_same<FT, bf16_t>::value;
+    if (BF16) {
+        if (R & 1) return 0;
+        for (int o = 0; o < a.nother; ++o)
+            if ((uintptr_t)a.Uo[o] % 4 != 0) return 0;
+    }
+    int E = 2;
+    if (!F64) {
+        const int narrow = k.narrow_max >= 0 ? k.narrow_max : BF16 ? 32 : 16;
+        if (R > narrow && !(k.narrow_small && nnz < (1ull << 20) && R <= 128)) E = 4;
+    }
+    return R >= E ? E : R >= 2 ? 2 : 0;
+}
+
+// LDS rows of the hot-row kernels are read in aligned vectors
 template <typename FT, typename VT, typename OT>
 inline bool rows_aligned(const StreamArgs<FT, VT, OT>& a, int R, int bytes)
 {
@@ -655,6 +754,14 @@ inline bool rows_aligned(const StreamArgs<FT, VT, OT>& a, int R, int bytes)
     for (int o = 0; o < a.nother; ++o)
         if ((uintptr_t)a.Uo[o] % bytes != 0) return false;
     return true;
+}
+
+// lanes per nonzero with E columns per lane (R <= 128: at most 128 / E)
+inline int lanes_for(int R, int E)
+{
+    int G = 1;
+    while (G * E < R) G <<= 1;
+    return G;
 }
 
 // The fiber parts of a fiber-ordered stream through k_mttkrp_fib (G lanes
@@ -694,12 +801,13 @@ int launch_fiber_tier(const alto_tensor* t, int mode, int fmode, uint64_t first,
         else if (o == 2) KF_(GG, PWW, 2);      \
         else KF_(GG, PWW, 3);                  \
     } while (0)
-#define KFG_(GG)                               \
-    do {                                       \
-        if (G == GG) {                         \
-            if (t->pack.pw == 1) KFN_(GG, 1);  \
-            else KFN_(GG, 2);                  \
-        }                                      \
+#define KFG_(GG)                                   \
+    do {                                           \
+        if constexpr (GG * E <= 128)               \
+            if (G == GG) {                         \
+                if (t->pack.pw == 1) KFN_(GG, 1);  \
+                else KFN_(GG, 2);                  \
+            }                                      \
     } while (0)
     KFG_(1);
     KFG_(2);
@@ -747,12 +855,123 @@ inline void skip_long_part(const alto_tensor* t, uint64_t nlong, StreamArgs<FT, 
     a.nnz -= nlong;
 }
 
+// The vector-lane kernels over the whole of a mode's stream, its fiber parts
+// first
+template <typename FT, typename VT, typename AT, typename OT, int E>
+int launch_lanes(const alto_tensor* t, int mode, int R, const FT* const* U, StreamArgs<FT, VT, OT>& a, int seg,
+                 hipStream_t s)
+{
+    const ModeStream& M = t->ms[mode];
+    const int G = lanes_for(R, E);
+    if (seg <= 0) seg = lane_seg(t->nnz, G, E);
+    a.seg = (uint64_t)seg;
+    const uint64_t nfib = M.nlong + M.nlong2;
+    if (M.fib_mode >= 0 && nfib > 0 && a.nother >= 2) {
+        ALTO_TRY(fiber_part(t, mode, R, U, a, G, E, seg, s));
+        skip_long_part(t, nfib, a);
+        if (a.nnz == 0) return ALTO_OK;
+    }
+    const dim3 grid = stream_grid(a.nnz, seg, G, a);
+#define KN_(GG, PWW)                                                                                            \
+    do {                                                                                                        \
+        switch (a.nother) {                                                                                     \
+        case 1: hipLaunchKernelGGL((k_mttkrp16<FT, VT, AT, OT, GG, E, PWW, 1, 0>), grid, dim3(256), 0, s, a); break; \
+        case 2: hipLaunchKernelGGL((k_mttkrp16<FT, VT, AT, OT, GG, E, PWW, 2, 0>), grid, dim3(256), 0, s, a); break; \
+        case 3: hipLaunchKernelGGL((k_mttkrp16<FT, VT, AT, OT, GG, E, PWW, 3, 0>), grid, dim3(256), 0, s, a); break; \
+        default: hipLaunchKernelGGL((k_mttkrp16<FT, VT, AT, OT, GG, E, PWW, 4, 0>), grid, dim3(256), 0, s, a); break; \
+        }                                                                                                       \
+    } while (0)
+#define KNG_(GG)                                     \
+    do {                                             \
+        if constexpr (GG * E <= 128)                 \
+            if (G == GG) {                           \
+                if (t->pack.pw == 1) KN_(GG, 1);     \
+                else KN_(GG, 2);                     \
+            }                                        \
+    } while (0)
+    KNG_(1);
+    KNG_(2);
+    KNG_(4);
+    KNG_(8);
+    KNG_(16);
+    KNG_(32);
+    KNG_(64);
+#undef KNG_
+#undef KN_
+    HIP_TRY(hipGetLastError());
+    return ALTO_OK;
+}
+
+// The vector-lane kernel over the hot-pattern groups of a split stream (one
+// or two other modes), one launch per pattern
+template <typename FT, typename VT, typename AT, typename OT, int E>
+int launch_split(const alto_tensor* t, int mode, int R, const StreamArgs<FT, VT, OT>& a, int seg, hipStream_t s)
+{
+    const ModeStream& M = t->ms[mode];
+    const int G = lanes_for(R, E);
+    if (seg <= 0) seg = tuned_seg(t->nnz, G, (int)sizeof(AT));
+    const int npat = 1 << a.nother;
+    for (int p = 0; p < npat; ++p) {
+        StreamArgs<FT, VT, OT> b = a;
+        b.seg = (uint64_t)seg;
+        uint32_t lds = 0;
+        const uint64_t s0 = M.pat_start[p], cnt = M.pat_start[p + 1] - s0;
+        if (cnt == 0) continue;
+        b.pk = a.pk + s0 * t->pack.pw;
+        b.val = a.val + s0;
+        b.nnz = cnt;
+        for (int o = 0; o < a.nother; ++o) {
+            b.hot_n[o] = (p >> o) & 1 ? (uint32_t)(M.hot_k[o] * R) : 0u;
+            b.hot_base[o] = lds;
+            lds += (uint32_t)((b.hot_n[o] * sizeof(FT) + 15) / 16 * 16);
+        }
+        if (lds > 160u * 1024u) {
+            set_error("mttkrp: %u bytes of staged rows exceed the 160 KiB of LDS (rank %d)", lds, R);
+            return ALTO_ERR_UNSUPPORTED;
+        }
+        const dim3 grid = stream_grid(b.nnz, seg, G, b);
+#define K16L_(GG, PWW, NOO, HMM) \
+    hipLaunchKernelGGL((k_mttkrp16<FT, VT, AT, OT, GG, E, PWW, NOO, HMM>), grid, dim3(256), lds, s, b)
+#define K16N_(GG, PWW)                           \
+    do {                                         \
+        switch (b.nother * 4 + p) {              \
+        case 4: K16L_(GG, PWW, 1, 0); break;     \
+        case 5: K16L_(GG, PWW, 1, 1); break;     \
+        case 8: K16L_(GG, PWW, 2, 0); break;     \
+        case 9: K16L_(GG, PWW, 2, 1); break;     \
+        case 10: K16L_(GG, PWW, 2, 2); break;    \
+        default: K16L_(GG, PWW, 2, 3); break;    \
+        }                                        \
+    } while (0)
+#define K16_(GG)                                     \
+    do {                                             \
+        if constexpr (GG * E <= 128)                 \
+            if (G == GG) {                           \
+                if (t->pack.pw == 1) K16N_(GG, 1);   \
+                else K16N_(GG, 2);                   \
+            }                                        \
+    } while (0)
+        K16_(1);
+        K16_(2);
+        K16_(4);
+        K16_(8);
+        K16_(16);
+        K16_(32);
+        K16_(64);
+#undef K16_
+#undef K16N_
+#undef K16L_
+        HIP_TRY(hipGetLastError());
+    }
+    return ALTO_OK;
+}
+
 // Lane mappings: 0 = 2 strided columns per lane (each gather instruction
 // reads G consecutive elements of a row); 1 = 4 contiguous columns per lane;
-// 2 = contiguous columns per lane in one vector load (16 bytes; 8 for BF16),
-// broadcasts through DPP / readlane.  -1 = 2 (measured fastest on MI355X for
-// every element type).  Ranked streams without the hot-pattern split use
-// mapping 0 or 1.
+// 2 = contiguous columns per lane in one vector load (lane_cols), broadcasts
+// through DPP / readlane.  -1 = 2 (measured fastest on MI355X for every
+// element type).  Ranked streams without the hot-pattern split use mapping 0
+// or 1.
 template <typename FT, typename VT, typename AT, typename OT>
 int launch_mttkrp(const alto_tensor* t, int mode, int R, const FT* const* U, const VT* val, OT* out, int seg,
                   const MttkrpTune& k, hipStream_t s)
@@ -764,132 +983,19 @@ int launch_mttkrp(const alto_tensor* t, int mode, int R, const FT* const* U, con
     a.out = out;
     int v = k.variant >= 0 ? k.variant : 2;
     const bool hot = t->ms[mode].ranked != 0 && a.nother > 0;
-    // elements per lane of the vector-lane mapping: one 16-byte load (FP64,
-    // FP32), one 8-byte load for BF16 (four columns: eight would need ~110
-    // VGPRs and halve the occupancy)
+    // one 16-byte load per lane (FP64, FP32), one 8-byte load for BF16
     constexpr int E16 = std::is_same<FT, bf16_t>::value ? 4 : 16 / sizeof(FT);
-    const ModeStream& M = t->ms[mode];
-    const bool split = M.split && hot && a.nother <= 2;
-    if (v == 2 && ((hot && !split) || !rows_aligned(a, R, E16 * (int)sizeof(FT)) || R > 64 * E16 || a.nother < 1)) v = 0;
-    // FP32 / BF16 rows of rank <= 16: two columns per lane, so that a wave
-    // holds at most 16 groups (with 4 columns per lane it would hold up to
-    // 32, and each row change of any group costs the wave a round of
-    // atomics); measured 1.3x faster at ranks 8 and 16
-    // Below 4M nonzeros (flushes dominate, launches are latency-bound) every
-    // rank takes two columns per lane, as FP64 does with its 16-byte lanes:
-    // 4 groups per wave at rank 64 instead of 2 made FP32 ~40% slower than
-    // FP64 there.
-    constexpr bool NARROW_OK = !std::is_same<FT, double>::value;
-    const bool narrow_rank = R <= k.narrow_max || (k.narrow_small && t->nnz < (4ull << 20) && R <= 128);
-    const uint64_t nfib = M.nlong + M.nlong2;
-    const bool fib = M.fib_mode >= 0 && nfib > 0 && !hot && a.nother >= 2;
-    if (v == 2 && NARROW_OK && narrow_rank && !split && a.nother >= 1 && rows_aligned(a, R, 2 * (int)sizeof(FT))) {
-        int G = 1;
-        while (G * 2 < R) G <<= 1;
-        if (seg <= 0) seg = tuned_seg(t->nnz, G, (int)sizeof(AT));
-        a.seg = (uint64_t)seg;
-        if (fib) {
-            ALTO_TRY(fiber_part(t, mode, R, U, a, G, 2, seg, s));
-            skip_long_part(t, nfib, a);
-            if (a.nnz == 0) return ALTO_OK;
-        }
-        dim3 grid = stream_grid(a.nnz, seg, G, a);
-#define KN_(GG, PWW)                                                                                            \
-    do {                                                                                                        \
-        switch (a.nother) {                                                                                     \
-        case 1: hipLaunchKernelGGL((k_mttkrp16<FT, VT, AT, OT, GG, 2, PWW, 1, 0>), grid, dim3(256), 0, s, a); break; \
-        case 2: hipLaunchKernelGGL((k_mttkrp16<FT, VT, AT, OT, GG, 2, PWW, 2, 0>), grid, dim3(256), 0, s, a); break; \
-        case 3: hipLaunchKernelGGL((k_mttkrp16<FT, VT, AT, OT, GG, 2, PWW, 3, 0>), grid, dim3(256), 0, s, a); break; \
-        default: hipLaunchKernelGGL((k_mttkrp16<FT, VT, AT, OT, GG, 2, PWW, 4, 0>), grid, dim3(256), 0, s, a); break; \
-        }                                                                                                       \
-    } while (0)
-#define KNG_(GG)                                 \
-    do {                                         \
-        if (G == GG) {                           \
-            if (t->pack.pw == 1) KN_(GG, 1);     \
-            else KN_(GG, 2);                     \
-        }                                        \
-    } while (0)
-        KNG_(1);
-        KNG_(2);
-        KNG_(4);
-        KNG_(8);
-        KNG_(16);
-        KNG_(32);
-        KNG_(64);
-#undef KNG_
-#undef KN_
-        HIP_TRY(hipGetLastError());
-        return ALTO_OK;
+    if (v == 2 && hot) {
+        if (t->ms[mode].split && a.nother <= 2 && rows_aligned(a, R, E16 * (int)sizeof(FT)))
+            return launch_split<FT, VT, AT, OT, E16>(t, mode, R, a, seg, s);
+        v = 0;
     }
     if (v == 2) {
-        int G = 1;
-        while (G * E16 < R) G <<= 1;
-        if (seg <= 0) seg = tuned_seg(t->nnz, G, (int)sizeof(AT));
-        a.seg = (uint64_t)seg;
-        if (fib && !split) {
-            ALTO_TRY(fiber_part(t, mode, R, U, a, G, E16, seg, s));
-            skip_long_part(t, nfib, a);
-            if (a.nnz == 0) return ALTO_OK;
-        }
-        // one launch per hot-pattern group (one launch over the whole stream
-        // when it is not split)
-        const int npat = split ? 1 << a.nother : 1;
-        for (int p = 0; p < npat; ++p) {
-            StreamArgs<FT, VT, OT> b = a;
-            uint32_t lds = 0;
-            if (split) {
-                const uint64_t s0 = M.pat_start[p], cnt = M.pat_start[p + 1] - s0;
-                if (cnt == 0) continue;
-                b.pk = a.pk + s0 * t->pack.pw;
-                b.val = a.val + s0;
-                b.nnz = cnt;
-                for (int o = 0; o < a.nother; ++o) {
-                    b.hot_n[o] = (p >> o) & 1 ? (uint32_t)(M.hot_k[o] * R) : 0u;
-                    b.hot_base[o] = lds;
-                    lds += (uint32_t)((b.hot_n[o] * sizeof(FT) + 15) / 16 * 16);
-                }
-            }
-            if (lds > 160u * 1024u) {
-                set_error("mttkrp: %u bytes of staged rows exceed the 160 KiB of LDS (rank %d)", lds, R);
-                return ALTO_ERR_UNSUPPORTED;
-            }
-            dim3 grid = stream_grid(b.nnz, seg, G, b);
-#define K16L_(GG, PWW, NOO, HMM) \
-    hipLaunchKernelGGL((k_mttkrp16<FT, VT, AT, OT, GG, E16, PWW, NOO, HMM>), grid, dim3(256), lds, s, b)
-#define K16N_(GG, PWW)                                     \
-    do {                                                   \
-        switch (b.nother * 16 + p) {                       \
-        case 16: K16L_(GG, PWW, 1, 0); break;              \
-        case 17: K16L_(GG, PWW, 1, 1); break;              \
-        case 32: K16L_(GG, PWW, 2, 0); break;              \
-        case 33: K16L_(GG, PWW, 2, 1); break;              \
-        case 34: K16L_(GG, PWW, 2, 2); break;              \
-        case 35: K16L_(GG, PWW, 2, 3); break;              \
-        case 48: K16L_(GG, PWW, 3, 0); break;              \
-        default: K16L_(GG, PWW, 4, 0); break;              \
-        }                                                  \
-    } while (0)
-#define K16_(GG)                                 \
-    do {                                         \
-        if (G == GG) {                           \
-            if (t->pack.pw == 1) K16N_(GG, 1);   \
-            else K16N_(GG, 2);                   \
-        }                                        \
-    } while (0)
-            K16_(1);
-            K16_(2);
-            K16_(4);
-            K16_(8);
-            K16_(16);
-            K16_(32);
-            K16_(64);
-#undef K16_
-#undef K16N_
-#undef K16L_
-            HIP_TRY(hipGetLastError());
-        }
-        return ALTO_OK;
+        const int E = a.nother < 1 ? 0 : lane_cols(a, t->nnz, R, k);
+        if (E == 2) return launch_lanes<FT, VT, AT, OT, 2>(t, mode, R, U, a, seg, s);
+        if constexpr (E16 == 4)
+            if (E == 4) return launch_lanes<FT, VT, AT, OT, 4>(t, mode, R, U, a, seg, s);
+        v = 0;
     }
     const int E = v == 1 ? 4 : 2;
     int G = 4;
@@ -935,21 +1041,15 @@ int launch_mttkrp(const alto_tensor* t, int mode, int R, const FT* const* U, con
 
 // lanes per nonzero (G) and elements per lane (E) of the vector-lane kernel
 // for this tensor and mode, as launch_mttkrp picks them; false when the
-// launch would take another kernel (ranked streams, unaligned rows, other
-// mappings)
+// launch would take another kernel (ranked streams, other mappings)
 template <typename FT, typename VT, typename OT>
 inline bool vector_lane_shape(const alto_tensor* t, int mode, int R, const StreamArgs<FT, VT, OT>& a,
                               const MttkrpTune& k, int& G, int& E)
 {
-    constexpr int E16 = std::is_same<FT, bf16_t>::value ? 4 : 16 / sizeof(FT);
-    constexpr bool NARROW_OK = !std::is_same<FT, double>::value;
     if (!(k.variant < 0 || k.variant == 2) || a.nother < 1 || t->ms[mode].ranked != 0) return false;
-    const bool narrow_rank = R <= k.narrow_max || (k.narrow_small && t->nnz < (4ull << 20) && R <= 128);
-    if (NARROW_OK && narrow_rank && rows_aligned(a, R, 2 * (int)sizeof(FT))) E = 2;
-    else if (rows_aligned(a, R, E16 * (int)sizeof(FT)) && R <= 64 * E16) E = E16;
-    else return false;
-    G = 1;
-    while (G * E < R) G <<= 1;
+    E = lane_cols(a, t->nnz, R, k);
+    if (E == 0) return false;
+    G = lanes_for(R, E);
     return true;
 }
 
@@ -958,8 +1058,10 @@ inline void launch_batch_table(const BatchTable<FT, VT, OT>& tab, int G, int pw,
 {
 #define KB_(GG)                                                                                              \
     do {                                                                                                     \
-        if (pw == 1) hipLaunchKernelGGL((k_mttkrp16_batch<FT, VT, AT, OT, GG, E, 1>), grid, dim3(256), 0, s, tab); \
-        else hipLaunchKernelGGL((k_mttkrp16_batch<FT, VT, AT, OT, GG, E, 2>), grid, dim3(256), 0, s, tab);        \
+        if constexpr (GG * E <= 128) {                                                                       \
+            if (pw == 1) hipLaunchKernelGGL((k_mttkrp16_batch<FT, VT, AT, OT, GG, E, 1>), grid, dim3(256), 0, s, tab); \
+            else hipLaunchKernelGGL((k_mttkrp16_batch<FT, VT, AT, OT, GG, E, 2>), grid, dim3(256), 0, s, tab);    \
+        }                                                                                                    \
     } while (0)
     switch (G) {
     case 2: KB_(2); break;
@@ -1004,7 +1106,7 @@ int launch_mttkrp_batch(int n, alto_tensor* const* ts, const int* modes, int R, 
             ALTO_TRY((launch_mttkrp<FT, VT, AT, OT>(t, modes[i], R, U[i], vals[i], outs[i], seg, k, s)));
             continue;
         }
-        a.seg = (uint64_t)(seg > 0 ? seg : tuned_seg(t->nnz, G, (int)sizeof(AT)));
+        a.seg = (uint64_t)(seg > 0 ? seg : lane_seg(t->nnz, G, E));
         (void)stream_grid(t->nnz, (int)a.seg, G, a);
         Group* g = nullptr;
         for (auto& x : groups)

@@ -143,8 +143,8 @@ int alto_coo_mttkrp(int nmodes, const uint64_t* dims, uint64_t nnz, const uint64
  * ALTO_TUNE_NONTEMPORAL: 1 = stream the nonzeros with non-temporal loads.
  * ALTO_TUNE_MTTKRP_VARIANT: lane mapping of the MTTKRP kernel: 0 = 2 strided
  * columns per lane, 1 = 4 contiguous columns per lane, 2 = one vector load
- * per lane and row, 16 bytes (8 for BF16) (needs rows aligned to that width,
- * else 0 is used); -1 (default) = 2.
+ * per lane and row, up to 16 bytes (rank 1 and BF16 rows that are not whole
+ * 4-byte words use 0); -1 (default) = 2.
  * ALTO_TUNE_GRAPHS: 1 = CP-ALS sessions capture one iteration as a HIP graph
  * and replay it (non-verbose iterate calls; phase timers are then not kept).
  * ALTO_TUNE_HOT_ROWS: 1 = the streams address the other modes' factor rows
@@ -158,14 +158,15 @@ int alto_coo_mttkrp(int nmodes, const uint64_t* dims, uint64_t nnz, const uint64
  * (256/512/1024).
  * ALTO_TUNE_HOT_LDS: LDS bytes per workgroup for the staged rows (default
  * 32768).
- * ALTO_TUNE_NARROW_RANK: FP32 / BF16 ranks up to this value (0..128,
- * default 32) use two columns per lane in the vector-lane mapping (fewer
- * lane groups per wave, so fewer rounds of FP64 row flushes).
+ * ALTO_TUNE_NARROW_RANK: FP32 / BF16 ranks up to this value (0..128) use
+ * two columns per lane in the vector-lane mapping (fewer lane groups per
+ * wave, so fewer rounds of FP64 row flushes), above it four; by default 16
+ * for FP32 and 32 for BF16.
  * ALTO_TUNE_PHI_VARIANT: CP-APR Phi kernel, 0 = runtime batch loop with LDS
  * permutes, 1 = compile-time batch with DPP broadcasts (default), 2 = 16-byte
  * lanes with the model row reloaded only where the row changes (even ranks
  * and 16-byte aligned factors; others take 1).
- * ALTO_TUNE_NARROW_SMALL: 1 (default) = below 4M nonzeros every FP32 / BF16
+ * ALTO_TUNE_NARROW_SMALL: 1 (default) = below 1M nonzeros every FP32 / BF16
  * rank uses two columns per lane.
  * ALTO_TUNE_FIBERS: 1 (default) = mode streams of tensors with at least
  * ALTO_TUNE_FIBER_MIN_NNZ nonzeros (default 4M) and 3+ modes are ordered by

@@ -339,11 +339,12 @@ int cp_apr_impl(alto_tensor* t, int R, int max_iters, int max_inner, double epsi
     // products are stored per nonzero by the first Phi of the mode and read
     // back by the others, when nnz x R doubles fit in half the free memory
     // (at most 64 GiB)
+    const int variant = phi_variant();  // one for the run: the cache has its layout
     bool cache = apr_pi_cache_enabled() && !det_enabled() && max_inner > 1;
     if (cache) {
         size_t fr = 0, tot = 0;
         HIP_TRY(hipMemGetInfo(&fr, &tot));
-        const uint64_t want = t->nnz * (uint64_t)R * sizeof(double);
+        const uint64_t want = phi_cache_doubles(t->nnz, R, variant) * sizeof(double);
         cache = want <= fr / 2 && want <= (64ull << 30) && c.pic.alloc(want) == ALTO_OK;
     }
     int iter;
@@ -370,7 +371,7 @@ int cp_apr_impl(alto_tensor* t, int R, int max_iters, int max_inner, double epsi
                 inner_per_mode[n]++;
                 HIP_TRY(hipEventRecord(ev0[inner], s));
                 ALTO_TRY(phi_device_cached(t, n, R, Uptr, Ph, eps_div_zero, s, 0, c.pic.as<double>(),
-                                           cache ? (inner == 0 ? 1 : 2) : 0));
+                                           cache ? (inner == 0 ? 1 : 2) : 0, variant));
                 HIP_TRY(hipEventRecord(ev1[inner], s));
                 timed = inner + 1;
                 const unsigned nb = ew_blocks(ne);

@@ -3,6 +3,7 @@
 // Reference semantics: CalculatePhi_alto_par (include/apr.hpp:295-303,
 // :383-501).
 #include "mttkrp_kernels.hpp"
+#include "phi_cols.hpp"
 
 namespace alto {
 
@@ -420,16 +421,22 @@ __global__ void __launch_bounds__(256)
 }
 
 // ------------------------------------------------------------------ host side
+// doubles of a product cache that fits whichever kernel `variant` picks
+uint64_t phi_cache_doubles(uint64_t nnz, int R, int variant)
+{
+    return variant == 1 && phi_cols_rank(R, 1) ? phi_cols_cache(nnz, R) : nnz * (uint64_t)R;
+}
+
 int phi_device(alto_tensor* t, int mode, int R, const double* const* U, double* phi, double eps, hipStream_t s, int seg)
 {
-    return phi_device_cached(t, mode, R, U, phi, eps, s, seg, nullptr, 0);
+    return phi_device_cached(t, mode, R, U, phi, eps, s, seg, nullptr, 0, phi_variant());
 }
 
 // pim: 0 = no cache; 1 = store the products of the other modes' rows per
-// nonzero into pc (nnz x R doubles, stream order); 2 = read them from pc
-// (stored by a pim 1 call for the same mode and factors)
+// nonzero into pc (phi_cache_doubles of them); 2 = read them from pc (stored
+// by a pim 1 call for the same mode, factors and variant)
 int phi_device_cached(alto_tensor* t, int mode, int R, const double* const* U, double* phi, double eps, hipStream_t s,
-                      int seg, double* pc, int pim)
+                      int seg, double* pc, int pim, int variant)
 {
     if (mode < 0 || mode >= t->nmode || R < 1 || R > 128) {
         set_error("phi: mode %d / rank %d out of range (rank 1..128)", mode, R);
@@ -446,10 +453,11 @@ int phi_device_cached(alto_tensor* t, int mode, int R, const double* const* U, d
     ALTO_TRY(set_factors(t, mode, U, a, s));
     a.val = t->ms[mode].val64.as<double>();
     a.out = phi;
+    if (variant == 1 && phi_cols_rank(R, pim)) return launch_phi_cols(a, t->pack.pw, U[mode], eps, pc, pim, s);
     dim3 grid = stream_grid(t->nnz, seg, group_lanes(R), a);
     bool al16 = R % 2 == 0 && ((uintptr_t)U[mode] & 15) == 0;
     for (int o = 0; o < a.nother; ++o) al16 = al16 && ((uintptr_t)a.Uo[o] & 15) == 0;
-    if (phi_variant() == 2 && al16 && (!pim || ((uintptr_t)pc & 15) == 0)) {
+    if (variant == 2 && al16 && (!pim || ((uintptr_t)pc & 15) == 0)) {
         const int no = t->nmode - 1;
 #define PHI16_P_(N_, P_) hipLaunchKernelGGL((k_phi16<G, PW, N_, P_>), grid, dim3(256), 0, s, a, U[mode], eps, pc)
 #define PHI16_NO_(N_)                      \
@@ -466,7 +474,7 @@ int phi_device_cached(alto_tensor* t, int mode, int R, const double* const* U, d
         });
 #undef PHI16_NO_
 #undef PHI16_P_
-    } else if (phi_variant() >= 1 || pim) {
+    } else if (variant >= 1 || pim) {
         const int no = t->nmode - 1;
 #define PHI_NO_(N_)                                                                                              \
     do {                                                                                                         \

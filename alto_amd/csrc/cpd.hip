@@ -97,8 +97,8 @@ struct CpdState {
     // product is taken from the stored values in the last mode's Gram pass
     // (pin_gram), so that the fit is that of the model the MTTKRPs see
     static constexpr bool rounds = !std::is_same<UT, ST>::value;
-    UT* u(int m) { return U[m].as<UT>(); }
-    ST* st(int m) { return std::is_same<UT, ST>::value ? reinterpret_cast<ST*>(U[m].p) : S[m].as<ST>(); }
+    UT* u(int m) const { return U[m].as<UT>(); }
+    ST* st(int m) const { return std::is_same<UT, ST>::value ? reinterpret_cast<ST*>(U[m].p) : S[m].as<ST>(); }
 };
 
 template <typename UT, typename ST, typename MT>
@@ -217,12 +217,86 @@ static int cpd_mode_step(alto_tensor* t, CpdState<UT, ST, MT>& c, int j, int it,
     return cpd_mode_rest(t, c, j, it, pt, s);
 }
 
+// partials of the fit's inner product that the last mode's update leaves
+template <typename UT, typename ST, typename MT>
+static int cpd_inner_parts(const alto_tensor* t, const CpdState<UT, ST, MT>& c)
+{
+    const uint64_t rows = t->dims[c.N - 1];
+    return c.rounds ? gram_blocks(rows) : c.R <= 64 ? solve_blocks(rows, c.R) : c.nb_solve;
+}
+
+// whether mode j's update leaves its Gram in partials (in gpart) for the next
+// one (storage that rounds: the last mode's Gram pass still reads the M that
+// its launch would clear)
+template <typename UT, typename ST, typename MT>
+static bool cpd_defers(const alto_tensor* t, const CpdState<UT, ST, MT>& c, int j)
+{
+    return gram_can_stay_partial(t->dims[j], c.R, t->dims[(j + 1) % c.N]) && !(c.rounds && j == c.N - 1);
+}
+template <typename UT, typename ST, typename MT>
+static PendingGram cpd_pending(const alto_tensor* t, const CpdState<UT, ST, MT>& c, int j)
+{
+    PendingGram p;
+    if (cpd_defers(t, c, j)) {
+        p.part = c.gpart.template as<double>();
+        p.mode = j;
+        p.n = gram_blocks(t->dims[j]);
+    }
+    return p;
+}
+
+// the arguments of mode j's update (rank <= 64)
+template <typename UT, typename ST, typename MT>
+static void cpd_mode_job(const alto_tensor* t, const CpdState<UT, ST, MT>& c, int j, int it, DenseModeJob* x)
+{
+    static_assert(std::is_same<MT, double>::value, "the row solves read an FP64 M");
+    const int N = c.N, R = c.R;
+    const bool last = j == N - 1;
+    x->grams = c.grams.template as<double>();
+    x->nmode = N;
+    x->mode = j;
+    // (set-up leaves all Grams complete)
+    x->pend = it == 0 && j == 0 ? PendingGram{} : cpd_pending(t, c, (j + N - 1) % N);
+    x->defer = cpd_defers(t, c, j);
+    x->P = c.P.template as<double>();
+    x->wsA = c.wsA.template as<double>();
+    x->wsQ = c.wsQ.template as<double>();
+    x->status = c.status.template as<int>();
+    x->M = c.M.template as<double>();
+    x->I = t->dims[j];
+    x->U = c.u(j);
+    x->psum = c.psum.template as<double>();
+    x->pmax = c.pmax.template as<double>();
+    x->pin = last && !c.rounds ? c.pin.template as<double>() : nullptr;
+    x->Mgram = last && c.rounds ? c.M.template as<double>() : nullptr;
+    x->pin_gram = last && c.rounds ? c.pin_gram.template as<double>() : nullptr;
+    x->nb = solve_blocks(x->I, R);
+    x->which = it == 0 ? 0 : 1;
+    x->lambda = c.lambda.template as<double>();
+    x->S = std::is_same<UT, ST>::value ? nullptr : (void*)c.st(j);
+    x->G = c.grams.template as<double>() + (size_t)j * R * R;
+    x->gpart = c.gpart.template as<double>();
+    x->zero = c.M.p;
+    x->zero_bytes = t->dims[(j + 1) % N] * R * sizeof(MT);
+}
+
 // the mode update after its MTTKRP (M holds M_j): R x R solve, row solves,
 // λ, Gram + scaling (which also clears M for the next mode)
 template <typename UT, typename ST, typename MT>
 static int cpd_mode_rest(alto_tensor* t, CpdState<UT, ST, MT>& c, int j, int it, PhaseTimer& pt, hipStream_t s)
 {
     const int R = c.R, N = c.N;
+    if (R <= 64) {
+        DenseModeJob job;
+        cpd_mode_job(t, c, j, it, &job);
+        const bool f64 = gram_f64(c.prec);
+        ALTO_TRY((dense_mode_one<UT, ST>(job, R, f64, s, 0)));
+        ALTO_TRY(pt.mark(PH_PINV));
+        ALTO_TRY((dense_mode_one<UT, ST>(job, R, f64, s, 1)));
+        ALTO_TRY(pt.mark(PH_NORM));
+        ALTO_TRY((dense_mode_one<UT, ST>(job, R, f64, s, 2)));
+        return pt.mark(PH_UPDATE);
+    }
     ALTO_TRY(chol_device(c.grams.template as<double>(), N, j, R, c.L.template as<double>(), c.P.template as<double>(),
                          c.wsA.template as<double>(), c.wsQ.template as<double>(), c.status.template as<int>(), s));
     // the last mode's solve also leaves the fit's inner-product partials
@@ -244,7 +318,7 @@ static int cpd_mode_rest(alto_tensor* t, CpdState<UT, ST, MT>& c, int j, int it,
         c.u(j), t->dims[j], R, c.lambda.template as<double>(), std::is_same<UT, ST>::value ? nullptr : c.st(j),
         c.grams.template as<double>() + (size_t)j * R * R, c.gpart.template as<double>(), s, gram_f64(c.prec), c.M.p,
         next_rows * R * sizeof(MT), inner ? c.M.template as<double>() : nullptr,
-        inner ? (R <= 64 ? c.pin_gram.template as<double>() : c.ipart.template as<double>()) : nullptr)));
+        inner ? c.ipart.template as<double>() : nullptr)));
     ALTO_TRY(pt.mark(PH_UPDATE));
     return ALTO_OK;
 }
@@ -258,11 +332,11 @@ static int cpd_fit_step(alto_tensor* t, CpdState<UT, ST, MT>& c, double normX, h
         return fit_device(c.grams.template as<double>(), c.N, c.R, c.lambda.template as<double>(),
                           c.ipart.template as<double>(), normX, c.fitbuf.template as<double>(), s);
     if (c.rounds)
-        return fit_scalar_device(c.grams.template as<double>(), c.N, c.R, c.lambda.template as<double>(),
-                                 c.pin_gram.template as<double>(), gram_blocks(t->dims[c.N - 1]), normX,
+        return fit_scalar_device(c.grams.template as<double>(), cpd_pending(t, c, c.N - 1), c.N, c.R, c.lambda.template as<double>(),
+                                 c.pin_gram.template as<double>(), cpd_inner_parts(t, c), normX,
                                  c.fitbuf.template as<double>(), s);
-    return fit_scalar_device(c.grams.template as<double>(), c.N, c.R, c.lambda.template as<double>(),
-                             c.pin.template as<double>(), c.nb_solve, normX, c.fitbuf.template as<double>(), s);
+    return fit_scalar_device(c.grams.template as<double>(), cpd_pending(t, c, c.N - 1), c.N, c.R, c.lambda.template as<double>(),
+                             c.pin.template as<double>(), cpd_inner_parts(t, c), normX, c.fitbuf.template as<double>(), s);
 }
 
 // A CP-ALS model resident on the device (factors, Grams, workspaces) that
@@ -407,37 +481,10 @@ struct CpdSession : CpdSessionBase {
         return fence(st);
     }
     // the arguments cpd_mode_rest and cpd_fit_step pass to their launches
-    void mode_job(int j, DenseModeJob* x) override
-    {
-        static_assert(std::is_same<MT, double>::value, "the row solves read an FP64 M");
-        const int N = c.N;
-        x->grams = c.grams.template as<double>();
-        x->nmode = N;
-        x->mode = j;
-        x->P = c.P.template as<double>();
-        x->wsA = c.wsA.template as<double>();
-        x->wsQ = c.wsQ.template as<double>();
-        x->status = c.status.template as<int>();
-        x->M = c.M.template as<double>();
-        x->I = t->dims[j];
-        x->U = c.u(j);
-        x->psum = c.psum.template as<double>();
-        x->pmax = c.pmax.template as<double>();
-        const bool last = j == N - 1;
-        x->pin = last && !c.rounds ? c.pin.template as<double>() : nullptr;
-        x->Mgram = last && c.rounds ? c.M.template as<double>() : nullptr;
-        x->pin_gram = last && c.rounds ? c.pin_gram.template as<double>() : nullptr;
-        x->nb = c.nb_solve;
-        x->which = it == 0 ? 0 : 1;
-        x->lambda = c.lambda.template as<double>();
-        x->S = std::is_same<UT, ST>::value ? nullptr : (void*)c.st(j);
-        x->G = c.grams.template as<double>() + (size_t)j * R * R;
-        x->gpart = c.gpart.template as<double>();
-        x->zero = c.M.p;
-        x->zero_bytes = t->dims[(j + 1) % N] * R * sizeof(MT);
-    }
+    void mode_job(int j, DenseModeJob* x) override { cpd_mode_job(t, c, j, it, x); }
     void fit_job(double* gather, DenseFitJob* f) override
     {
+        f->pend = cpd_pending(t, c, c.N - 1);
         f->grams = c.grams.template as<double>();
         f->lambda = c.lambda.template as<double>();
         f->pin = c.rounds ? c.pin_gram.template as<double>() : c.pin.template as<double>();
@@ -445,7 +492,7 @@ struct CpdSession : CpdSessionBase {
         f->gather = gather;
         f->normX = normX;
         f->nmode = c.N;
-        f->nb = c.rounds ? gram_blocks(t->dims[c.N - 1]) : c.nb_solve;
+        f->nb = cpd_inner_parts(t, c);
     }
     int iterate(int max_iters, double eps, double* fit_trace, int* ran, int verbose) override
     {

@@ -226,32 +226,27 @@ __global__ void __launch_bounds__(256) k_gram_rows(T* __restrict__ U, uint64_t I
     gram_rows_body<T, ST, F64, T16, SCALE, INNER>(U, I, R, rows_per_block, part, lambda, S, Mi, pin, blockIdx.x);
 }
 
-__global__ void k_sum_partials(const double* __restrict__ part, int nparts, int n, double* __restrict__ out)
-{
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
-        double s = 0;
-        for (int p = 0; p < nparts; ++p) s += part[(size_t)p * n + k];
-        out[k] = s;
-    }
-}
-
 // out[k] = sum_p part[p n + k]: a block covers 32 consecutive k, its 8
 // wave halves stride over the partials, and the 8 sums are added in a fixed
 // order (deterministic).  Blocks from nsum on clear `zero` (nz bytes, a
 // multiple of 4): a buffer the caller needs zeroed next, for free in this
 // launch.
+__device__ __forceinline__ void clear_body(void* __restrict__ zero, uint64_t nz, uint32_t bid, uint32_t nblk)
+{
+    const uint64_t t = (uint64_t)bid * blockDim.x + threadIdx.x, stride = (uint64_t)nblk * blockDim.x;
+    uint4* z16 = reinterpret_cast<uint4*>(zero);
+    const uint64_t n16 = nz / 16;
+    for (uint64_t i = t; i < n16; i += stride) z16[i] = make_uint4(0, 0, 0, 0);
+    uint32_t* z4 = reinterpret_cast<uint32_t*>(zero);
+    for (uint64_t i = n16 * 4 + t; i < nz / 4; i += stride) z4[i] = 0;
+}
+
 __device__ __forceinline__ void sum_cols_body(const double* __restrict__ part, int nparts, int n,
                                               double* __restrict__ out, int nsum, void* __restrict__ zero, uint64_t nz,
                                               uint32_t bid, uint32_t nblk)
 {
     if ((int)bid >= nsum) {
-        const uint64_t t = (uint64_t)(bid - nsum) * blockDim.x + threadIdx.x;
-        const uint64_t stride = (uint64_t)(nblk - nsum) * blockDim.x;
-        uint4* z16 = reinterpret_cast<uint4*>(zero);
-        const uint64_t n16 = nz / 16;
-        for (uint64_t i = t; i < n16; i += stride) z16[i] = make_uint4(0, 0, 0, 0);
-        uint32_t* z4 = reinterpret_cast<uint32_t*>(zero);
-        for (uint64_t i = n16 * 4 + t; i < nz / 4; i += stride) z4[i] = 0;
+        clear_body(zero, nz, bid - nsum, nblk - nsum);
         return;
     }
     __shared__ double s[8][33];
@@ -341,39 +336,11 @@ int gram_scale_device(UT* U, uint64_t I, int R, const double* lambda, ST* S, dou
                       bool f64, void* zero, uint64_t zero_bytes, const double* Mi, double* pin)
 {
     constexpr bool same = std::is_same<UT, ST>::value;
-    if (R > 64) {
-        ALTO_TRY((scale_device<UT, ST>(U, I, R, lambda, same ? nullptr : S, s)));
-        ALTO_TRY(gram_device<ST>(same ? reinterpret_cast<const ST*>(U) : S, I, R, G, part, s, f64));
-        if (Mi) ALTO_TRY((inner_partial_device<ST, double>(same ? reinterpret_cast<const ST*>(U) : S, Mi, I, R, pin, s)));
-        if (zero_bytes) ALTO_TRY(sum_cols_device(nullptr, 0, 0, nullptr, zero, zero_bytes, s));
-        return ALTO_OK;
-    }
-    const int nb = gram_blocks(I);
-    const uint64_t rpb = ((I + nb - 1) / nb + 15) / 16 * 16;
-    const size_t lds = (size_t)R * R * 8;
-#define GSI_(TT, F, IN)                                                                                        \
-    hipLaunchKernelGGL((k_gram_rows<UT, ST, F, TT, true, IN>), dim3(nb), dim3(256), lds, s, U, I, R, rpb, part, \
-                       lambda, S, Mi, pin)
-#define GS_(TT)                           \
-    do {                                  \
-        if (Mi) {                         \
-            if (f64) GSI_(TT, true, true); \
-            else GSI_(TT, false, true);    \
-        } else if (f64) {                 \
-            GSI_(TT, true, false);        \
-        } else {                          \
-            GSI_(TT, false, false);       \
-        }                                 \
-    } while (0)
-    switch ((R + 15) / 16) {
-    case 1: GS_(1); break;
-    case 2: GS_(2); break;
-    case 3: GS_(3); break;
-    default: GS_(4); break;
-    }
-#undef GS_
-#undef GSI_
-    return sum_cols_device(part, nb, R * R, G, zero, zero_bytes, s);
+    ALTO_TRY((scale_device<UT, ST>(U, I, R, lambda, same ? nullptr : S, s)));
+    ALTO_TRY(gram_device<ST>(same ? reinterpret_cast<const ST*>(U) : S, I, R, G, part, s, f64));
+    if (Mi) ALTO_TRY((inner_partial_device<ST, double>(same ? reinterpret_cast<const ST*>(U) : S, Mi, I, R, pin, s)));
+    if (zero_bytes) ALTO_TRY(sum_cols_device(nullptr, 0, 0, nullptr, zero, zero_bytes, s));
+    return ALTO_OK;
 }
 template int gram_scale_device<double, double>(double*, uint64_t, int, const double*, double*, double*, double*,
                                                hipStream_t, bool, void*, uint64_t, const double*, double*);
@@ -445,125 +412,213 @@ int gram_noalloc(const void* U, uint64_t dim, int R, int precision, double* gram
 // reference's dpotrf test; then status = 1 and the same workgroup computes
 // the pseudo-inverse (pinv_body).  status 0: W = V^-1.
 //
-// Thread t keeps the entries (r0 + rstep n, jc) of the matrix in registers,
-// rstep = BT / R, r0 = t / R, jc = t % R (BT threads: 1024 from R = 17 on,
-// so that a thread holds at most 16 entries and the waves of all four SIMDs
-// share each step).  Step k reads column k (the elimination factors, pivot
-// included) and row k from LDS buffer k & 1 and updates every register; the
-// owners of column and row k + 1 write their new values into the other
-// buffer as they compute them, so one barrier per step orders everything
-// (buffer (k + 1) & 1 is written after the barrier of step k, which every
-// reader of step k - 1, the buffer's previous use, has passed).
-__device__ __attribute__((noinline)) void pinv_body(const double* __restrict__ grams, int nmode, int mode, int R,
-                                                    double* __restrict__ A, double* __restrict__ Q,
-                                                    double* __restrict__ Pout);
+// A chain of R dependent steps in one workgroup: latency is all that counts.
+// The arithmetic per entry is that of the textbook loop (the inverse does not
+// depend on how it is spread); a pivot that fails is only noted, and the steps
+// behind it run on without effect.
+//
+// Above rank 16 wavefront w keeps rows w RPW .. of the matrix in registers,
+// lane l their columns l (and l + 64): the elimination factors of its own rows
+// are then one v_readlane away, and all that a step takes from the others is
+// the pivot row, which comes divided by its pivot.  The owner of row k + 1
+// updates that row first, at raised priority, divides it and leaves it in the
+// LDS buffer that step k does not read, so that one barrier per step orders
+// everything (the buffer's previous readers have passed the barrier of step k)
+// and the division is done by one wavefront, not by all.  Rank 64: 54 -> 31 us
+// (0.48 us a step).
+__device__ __attribute__((noinline)) void pinv_body(int R, double* A, double* Q, double* Pout);
 
-template <int BT, int NPT>
+__device__ __forceinline__ double lane_value(double v, int l)
+{
+    const uint64_t u = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)u, l), hi = __builtin_amdgcn_readlane((uint32_t)(u >> 32), l);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+// the product of the other modes' Grams at (i, c)
+__device__ __forceinline__ double gram_product(const double* __restrict__ grams, int nmode, int mode, int R, int i, int c)
+{
+    double v = 1.0;
+#pragma unroll
+    for (int m = 0; m < ALTO_MAXN; ++m)
+        if (m < nmode && m != mode) v *= grams[(size_t)m * R * R + i * R + c];
+    return v;
+}
+
+// load(i, c): the entries of V; store(i, c, value) for every entry of the
+// inverse; false: a pivot failed (the entries are then meaningless).  RPW rows
+// per wavefront, CPL columns per lane; every thread of the workgroup takes part.
+template <int RPW, int CPL, typename L, typename F>
+__device__ __forceinline__ bool spd_inverse_rows(int R, L&& load, F&& store)
+{
+    __shared__ double s_row[2][64 * CPL];  // the pivot row over its pivot
+    __shared__ int s_bad;
+    const int lane = threadIdx.x & 63;
+    const int row0 = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * RPW;
+    if (threadIdx.x == 0) s_bad = 0;
+    double a[RPW][CPL];
+    // entries outside the matrix repeat its last row and column, and are
+    // neither published nor stored
+#pragma unroll
+    for (int n = 0; n < RPW; ++n)
+#pragma unroll
+        for (int h = 0; h < CPL; ++h)
+            a[n][h] = load(min(row0 + n, R - 1), min(lane + 64 * h, R - 1));
+    __syncthreads();
+    // leaves row k (held as x) over its pivot in buffer k & 1
+    auto publish = [&](const double (&x)[CPL], int k) {
+        const double piv = lane_value(CPL == 2 && k >= 64 ? x[CPL - 1] : x[0], k & 63);
+#pragma unroll
+        for (int h = 0; h < CPL; ++h) s_row[k & 1][lane + 64 * h] = (lane + 64 * h == k ? 1.0 : x[h]) / piv;
+        if (!(piv > 0.0)) s_bad = 1;
+    };
+    if (row0 == 0) publish(a[0], 0);
+    for (int k = 0; k < R; ++k) {
+        __syncthreads();
+        // row k becomes the pivot row, its diagonal slot holding 1 / pivot;
+        // the others lose their factor times it (column k: -factor / pivot)
+        double rk[CPL];
+#pragma unroll
+        for (int h = 0; h < CPL; ++h) rk[h] = s_row[k & 1][lane + 64 * h];
+        auto update = [&](int n) {
+            const double c = lane_value(CPL == 2 && k >= 64 ? a[n][CPL - 1] : a[n][0], k & 63);
+#pragma unroll
+            for (int h = 0; h < CPL; ++h) {
+                const double x = lane + 64 * h == k ? 0.0 : a[n][h];
+                a[n][h] = fma(-c, rk[h], x);
+            }
+        };
+        const int next = k + 1 - row0, own = k - row0;  // uniform
+        if (next >= 0 && next < RPW && k + 1 < R) {
+            __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+            for (int n = 0; n < RPW; ++n)
+                if (n == next) {
+                    update(n);
+                    publish(a[n], k + 1);
+                }
+            __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+            for (int n = 0; n < RPW; ++n)
+                if (n != next) update(n);
+        } else {
+#pragma unroll
+            for (int n = 0; n < RPW; ++n) update(n);
+        }
+        if (own >= 0 && own < RPW) {
+#pragma unroll
+            for (int n = 0; n < RPW; ++n)
+                if (n == own) {
+#pragma unroll
+                    for (int h = 0; h < CPL; ++h) a[n][h] = rk[h];
+                }
+        }
+    }
+    __syncthreads();
+    if (s_bad) return false;
+#pragma unroll
+    for (int n = 0; n < RPW; ++n)
+#pragma unroll
+        for (int h = 0; h < CPL; ++h)
+            if (row0 + n < R && lane + 64 * h < R) store(row0 + n, lane + 64 * h, a[n][h]);
+    return true;
+}
+
+// The same for R <= 16 by one wavefront (called by all of its lanes): lane
+// 16 q + c holds column c of rows 4 q .. 4 q + 3, and pivot row and factors
+// come through lane permutes: no barrier at all.  A loop, not unrolled: code
+// that runs once is fetched from memory at ~250 cycles per 64 bytes, which
+// made an unrolled form (DPP broadcasts of constant lanes) twice as slow.
+template <typename L, typename F>
+__device__ __forceinline__ bool spd_inverse16(int R, L&& load, F&& store)
+{
+    const int lane = threadIdx.x & 63, q = lane >> 4, c = lane & 15;
+    double a[4];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) a[n] = load(min(4 * q + n, R - 1), min(c, R - 1));
+    bool ok = true;
+#pragma unroll 1
+    for (int k = 0; k < R; ++k) {
+        const int kn = k & 3;  // uniform
+        const double mine = kn == 0 ? a[0] : kn == 1 ? a[1] : kn == 2 ? a[2] : a[3];
+        const double row = __shfl(mine, (k >> 2) * 16 + c);
+        double f[4];
+#pragma unroll
+        for (int n = 0; n < 4; ++n) f[n] = __shfl(a[n], (lane & 48) | k);
+        const double piv = lane_value(row, k);
+        ok = ok && piv > 0.0;
+        const double rk = (c == k ? 1.0 : row) / piv;
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            const double x = c == k ? 0.0 : a[n];
+            a[n] = 4 * q + n == k ? rk : fma(-f[n], rk, x);
+        }
+    }
+    if (!ok) return false;  // the pivots are uniform
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+        if (4 * q + n < R && c < R) store(4 * q + n, c, a[n]);
+    return true;
+}
+
+// V^-1 through put(i, c, value), or false; RPW = 0: rank <= 16, by the first
+// wavefront
+template <int RPW, int CPL, typename L, typename F>
+__device__ __forceinline__ bool spd_inverse(int R, L&& load, F&& put)
+{
+    if constexpr (RPW == 0) {
+        __shared__ int s_ok;
+        if (threadIdx.x < 64) {
+            const bool ok = spd_inverse16(R, load, put);
+            if (threadIdx.x == 0) s_ok = ok;
+        }
+        __syncthreads();
+        return s_ok;
+    } else {
+        return spd_inverse_rows<RPW, CPL>(R, load, put);
+    }
+}
+
+// V^-1, or V^+ where a pivot fails, into W (global memory)
+template <int RPW, int CPL>
 __device__ __forceinline__ void spd_inverse_body(const double* __restrict__ grams, int nmode, int mode, int R,
                                                  double* __restrict__ W, int* __restrict__ status,
                                                  double* __restrict__ wsA, double* __restrict__ wsQ)
 {
-    __shared__ double s_col[2][128], s_row[2][128];
-    const int tid = threadIdx.x;
-    const int rstep = BT / R, r0 = tid / R, jc = tid % R;
-    const bool active = tid < rstep * R;
-    // rows of this thread are clamped into the matrix so that every load and
-    // LDS read below is unconditional (entries of rows >= R are never stored)
-    auto rc = [&](int n) { return min(r0 + rstep * n, R - 1); };
-    double a[NPT];
-#pragma unroll
-    for (int n = 0; n < NPT; ++n) a[n] = 1.0;
-#pragma unroll
-    for (int m = 0; m < ALTO_MAXN; ++m) {
-        if (m < nmode && m != mode) {
-            const double* g = grams + (size_t)m * R * R + (active ? jc : 0);
-#pragma unroll
-            for (int n = 0; n < NPT; ++n) a[n] *= g[rc(n) * R];
-        }
-    }
-    // column 0 and row 0 for the first step; every later step's column and
-    // row are written by their owners as they update them
-    if (active) {
-#pragma unroll
-        for (int n = 0; n < NPT; ++n) {
-            const int i = r0 + rstep * n;
-            if (i < R && jc == 0) s_col[0][i] = a[n];
-        }
-        if (r0 == 0) s_row[0][jc] = a[0];
-    }
-    int ok = 1;
-    for (int k = 0; k < R; ++k) {
-        const int b = k & 1, nb = b ^ 1;
+    const bool ok = spd_inverse<RPW, CPL>(
+        R, [&](int i, int c) { return gram_product(grams, nmode, mode, R, i, c); },
+        [&](int i, int c, double v) { W[i * R + c] = v; });
+    if (threadIdx.x == 0) *status = ok ? 0 : 1;
+    if (!ok) {
         __syncthreads();
-        const double piv = s_col[b][k];
-        if (!(piv > 0.0)) {  // uniform: every thread read the same pivot
-            ok = 0;
-            break;
+        for (int k = threadIdx.x; k < R * R; k += blockDim.x) {  // symmetric, from the lower triangle
+            const int i = k / R, c = k % R;
+            wsA[k] = gram_product(grams, nmode, mode, R, max(i, c), min(i, c));
         }
-        // row k scaled by 1 / pivot, its diagonal slot holding 1 / pivot;
-        // the other rows lose s_col[i] times it (column k becomes -s_col / piv)
-        const double rk = (jc == k ? 1.0 : s_row[b][jc]) / piv;
-        constexpr int CH = NPT < 16 ? NPT : 16;  // LDS reads in flight per batch
-#pragma unroll
-        for (int n0 = 0; n0 < NPT; n0 += CH) {
-            double cv[CH];
-#pragma unroll
-            for (int n = 0; n < CH; ++n) cv[n] = s_col[b][rc(n0 + n)];
-#pragma unroll
-            for (int n = 0; n < CH; ++n) {
-                const int i = r0 + rstep * (n0 + n);
-                const double v = i == k ? rk : (jc == k ? 0.0 : a[n0 + n]) - cv[n] * rk;
-                a[n0 + n] = v;
-                if (active && i < R) {
-                    if (jc == k + 1) s_col[nb][i] = v;
-                    if (i == k + 1) s_row[nb][jc] = v;
-                }
-            }
-        }
+        pinv_body(R, wsA, wsQ, W);
     }
-    if (ok) {
-        if (active) {
-#pragma unroll
-            for (int n = 0; n < NPT; ++n)
-                if (r0 + rstep * n < R) W[(r0 + rstep * n) * R + jc] = a[n];
-        }
-        if (tid == 0) *status = 0;
-        return;
-    }
-    if (tid == 0) *status = 1;
-    __syncthreads();
-    pinv_body(grams, nmode, mode, R, wsA, wsQ, W);
 }
 
-template <int BT, int NPT>
+template <int BT, int RPW, int CPL>
 __global__ void __launch_bounds__(BT) k_spd_inverse(const double* __restrict__ grams, int nmode, int mode, int R,
                                                     double* __restrict__ W, int* __restrict__ status,
                                                     double* __restrict__ wsA, double* __restrict__ wsQ)
 {
-    spd_inverse_body<BT, NPT>(grams, nmode, mode, R, W, status, wsA, wsQ);
+    spd_inverse_body<RPW, CPL>(grams, nmode, mode, R, W, status, wsA, wsQ);
 }
 
 // Minimum-norm pseudo-inverse V^+ = Q diag(1/e) Q^T over |e| > R*eps*max|e|
-// (parallel cyclic Jacobi; runs only after a failed Cholesky).  A and Q live in the
-// workspace (global memory), shared through work-group barriers.
-__device__ __attribute__((noinline)) void pinv_body(const double* __restrict__ grams, int nmode, int mode, int R,
-                                                    double* __restrict__ A, double* __restrict__ Q,
-                                                    double* __restrict__ Pout)
+// (parallel cyclic Jacobi; runs only after a failed Cholesky).  A holds V and
+// is overwritten; A, Q and Pout (R x R, global memory or LDS) are shared
+// through work-group barriers.
+__device__ __attribute__((noinline)) void pinv_body(int R, double* A, double* Q, double* Pout)
 {
     const int tid = threadIdx.x;
     __shared__ double s_red[1024];
     __shared__ double s_c[64], s_s[64];
     __shared__ int s_p[64], s_q[64];
     __shared__ int s_stop;
-    for (int k = tid; k < R * R; k += blockDim.x) {
-        const int i = k / R, c = k % R;
-        const int lo = i >= c ? k : c * R + i;  // symmetric from the lower triangle
-        double v = 1.0;
-        for (int m = 0; m < nmode; ++m)
-            if (m != mode) v *= grams[(size_t)m * R * R + lo];
-        A[k] = v;
-        Q[k] = i == c ? 1.0 : 0.0;
-    }
+    for (int k = tid; k < R * R; k += blockDim.x) Q[k] = k / R == k % R ? 1.0 : 0.0;
     __syncthreads();
     // a non-finite V has no pseudo-inverse: return NaN at once
     __shared__ int s_bad;
@@ -680,9 +735,11 @@ __device__ __attribute__((noinline)) void pinv_body(const double* __restrict__ g
 // U[i,c] M[i,c] over the block's rows (the fit's inner product: with
 // U = lambda * U_normalised it equals sum_c lambda_c <U_normalised[:,c], M[:,c]>).
 // The 16 x R block of M is loaded into registers before the products, so
-// its loads are in flight together.  T16: 16-column tiles (R <= 16 T16).
-template <typename MT, typename UT, int T16, bool LOWP>
-__device__ __forceinline__ void apply_body(const MT* __restrict__ M, uint64_t I, int R, const double* __restrict__ Wg,
+// its loads are in flight together; the first block's before W is there:
+// prepare(sW, stride) leaves W in LDS (ending in a barrier).  T16: 16-column
+// tiles (R <= 16 T16).
+template <typename MT, typename UT, int T16, bool LOWP, typename F>
+__device__ __forceinline__ void apply_body(const MT* __restrict__ M, uint64_t I, int R, F&& prepare,
                                            UT* __restrict__ U, double* __restrict__ psum, double* __restrict__ pmax,
                                            double* __restrict__ pin, uint32_t bid, uint32_t nblk)
 {
@@ -696,8 +753,6 @@ __device__ __forceinline__ void apply_body(const MT* __restrict__ M, uint64_t I,
     extern __shared__ double sWd[];  // W, row stride WS
     mma_t* sW = reinterpret_cast<mma_t*>(sWd);
     const int WS = R + 2;
-    for (int k = threadIdx.x; k < R * R; k += blockDim.x) sW[(k / R) * WS + k % R] = (mma_t)Wg[k];
-    __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r16 = lane & 15, kq = lane >> 4;
     double ss[T16], mx[T16];
@@ -707,14 +762,20 @@ __device__ __forceinline__ void apply_body(const MT* __restrict__ M, uint64_t I,
         mx[t] = -INFINITY;
     }
     double in = 0;
-    for (uint64_t row0 = ((uint64_t)bid * 4 + wave) * 16; row0 < I; row0 += (uint64_t)nblk * 64) {
+    mma_t av[KS];
+    auto load = [&](uint64_t row0) {
         const uint64_t ra = row0 + r16;
-        mma_t av[KS];
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             const int k = ks * 4 + kq;
             av[ks] = (ra < I && k < R) ? (mma_t)M[ra * R + k] : (mma_t)0;
         }
+    };
+    const uint64_t first = ((uint64_t)bid * 4 + wave) * 16;
+    load(first);
+    prepare(sW, WS);
+    for (uint64_t row0 = first; row0 < I; row0 += (uint64_t)nblk * 64) {
+        if (row0 != first) load(row0);
         acc_t acc[T16];
 #pragma unroll
         for (int t = 0; t < T16; ++t) acc[t] = acc_t{0, 0, 0, 0};
@@ -787,12 +848,29 @@ __device__ __forceinline__ void apply_body(const MT* __restrict__ M, uint64_t I,
     }
 }
 
+// W from global memory (by rows: no divisions by the rank)
+struct WFrom {
+    const double* W;
+    int R;
+    template <typename T> __device__ __forceinline__ void operator()(T* sW, int WS) const
+    {
+        for (int i = threadIdx.x >> 6; i < R; i += 4)
+            for (int c = threadIdx.x & 63; c < R; c += 64) sW[i * WS + c] = (T)W[i * R + c];
+        __syncthreads();
+    }
+};
+
 template <typename MT, typename UT, int T16, bool LOWP>
 __global__ void __launch_bounds__(256) k_apply(const MT* __restrict__ M, uint64_t I, int R, const double* __restrict__ Wg,
                                                UT* __restrict__ U, double* __restrict__ psum, double* __restrict__ pmax,
                                                double* __restrict__ pin)
 {
-    apply_body<MT, UT, T16, LOWP>(M, I, R, Wg, U, psum, pmax, pin, blockIdx.x, gridDim.x);
+    apply_body<MT, UT, T16, LOWP>(M, I, R, WFrom{Wg, R}, U, psum, pmax, pin, blockIdx.x, gridDim.x);
+}
+
+__device__ inline double lambda_of(int which, double ss, double mx)
+{
+    return which == 0 ? sqrt(ss) : fmax(1.0, fmax(mx, 0.0));
 }
 
 // lambda: iteration 0 -> 2-norm of each column; later -> max(1, max_i U[i,r]).
@@ -816,7 +894,7 @@ __device__ __forceinline__ void lambda_body(const double* __restrict__ psum, con
         }
         __syncthreads();
     }
-    if (threadIdx.x == 0) lambda[c] = which == 0 ? sqrt(sa[0]) : fmax(1.0, fmax(sb[0], 0.0));
+    if (threadIdx.x == 0) lambda[c] = lambda_of(which, sa[0], sb[0]);
 }
 
 __global__ void __launch_bounds__(256) k_lambda(const double* __restrict__ psum, const double* __restrict__ pmax, int nb,
@@ -864,7 +942,7 @@ __global__ void k_inner_partial(const UT* __restrict__ U, const MT* __restrict__
 // when res > 0, as in the reference)
 // inner from per-column partials (nb x R, weighted by lambda) or, with
 // scalar set, from nb per-block totals already carrying lambda
-__device__ __forceinline__ void fit_body(const double* __restrict__ grams, int nmode, int R,
+__device__ __forceinline__ void fit_body(const double* __restrict__ grams, PendingGram pend, int nmode, int R,
                                          const double* __restrict__ lambda, const double* __restrict__ ipart, int nb,
                                          int scalar, double normX, double* __restrict__ out)
 {
@@ -883,7 +961,7 @@ __device__ __forceinline__ void fit_body(const double* __restrict__ grams, int n
         const int i = k / R, j = k % R;
         if (j > i) continue;
         double t = lambda[i] * lambda[j];
-        for (int m = 0; m < nmode; ++m) t *= grams[(size_t)m * R * R + k];
+        for (int m = 0; m < nmode; ++m) t *= m == pend.mode ? pend.sum(k, R) : grams[(size_t)m * R * R + k];
         nu += i == j ? t : 2.0 * t;
     }
     s_in[threadIdx.x] = inner;
@@ -906,11 +984,11 @@ __device__ __forceinline__ void fit_body(const double* __restrict__ grams, int n
     }
 }
 
-__global__ void __launch_bounds__(256) k_fit(const double* __restrict__ grams, int nmode, int R,
+__global__ void __launch_bounds__(256) k_fit(const double* __restrict__ grams, PendingGram pend, int nmode, int R,
                                              const double* __restrict__ lambda, const double* __restrict__ ipart,
                                              int nb, int scalar, double normX, double* __restrict__ out)
 {
-    fit_body(grams, nmode, R, lambda, ipart, nb, scalar, normX, out);
+    fit_body(grams, pend, nmode, R, lambda, ipart, nb, scalar, normX, out);
 }
 
 __global__ void k_sumsq_partial(const double* __restrict__ v, uint64_t n, double* __restrict__ part)
@@ -967,13 +1045,13 @@ int chol_device(const double* grams, int nmode, int mode, int R, double* L, doub
         return ALTO_ERR_UNSUPPORTED;
     }
     (void)L;
-    // registers per thread: ceil(R / (BT / R)) matrix entries
-#define SPD_(BT, NPT) \
-    hipLaunchKernelGGL((k_spd_inverse<BT, NPT>), dim3(1), dim3(BT), 0, s, grams, nmode, mode, R, P, status, wsA, wsQ)
-    if (R <= 16) SPD_(256, 1);
-    else if (R <= 32) SPD_(1024, 1);
-    else if (R <= 64) SPD_(1024, 4);
-    else SPD_(1024, 16);
+    // rows per wavefront and columns per lane
+#define SPD_(BT, RPW, CPL) \
+    hipLaunchKernelGGL((k_spd_inverse<BT, RPW, CPL>), dim3(1), dim3(BT), 0, s, grams, nmode, mode, R, P, status, wsA, wsQ)
+    if (R <= 16) SPD_(256, 0, 1);
+    else if (R <= 32) SPD_(1024, 2, 1);
+    else if (R <= 64) SPD_(1024, 4, 1);
+    else SPD_(1024, 8, 2);
 #undef SPD_
     HIP_TRY(hipGetLastError());
     return ALTO_OK;
@@ -1054,15 +1132,16 @@ template int inner_partial_device<float, double>(const float*, const double*, ui
 int fit_device(const double* grams, int nmode, int R, const double* lambda, const double* ipart, double normX,
                double* out, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_fit, dim3(1), dim3(256), 0, s, grams, nmode, R, lambda, ipart, INNER_BLOCKS, 0, normX, out);
+    hipLaunchKernelGGL(k_fit, dim3(1), dim3(256), 0, s, grams, PendingGram{}, nmode, R, lambda, ipart,
+                       INNER_BLOCKS, 0, normX, out);
     HIP_TRY(hipGetLastError());
     return ALTO_OK;
 }
 
-int fit_scalar_device(const double* grams, int nmode, int R, const double* lambda, const double* pin, int nb,
-                      double normX, double* out, hipStream_t s)
+int fit_scalar_device(const double* grams, const PendingGram& pend, int nmode, int R, const double* lambda,
+                      const double* pin, int nb, double normX, double* out, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_fit, dim3(1), dim3(256), 0, s, grams, nmode, R, lambda, pin, nb, 1, normX, out);
+    hipLaunchKernelGGL(k_fit, dim3(1), dim3(256), 0, s, grams, pend, nmode, R, lambda, pin, nb, 1, normX, out);
     HIP_TRY(hipGetLastError());
     return ALTO_OK;
 }
@@ -1071,26 +1150,52 @@ int normsq_device(const double* v, uint64_t n, double* part, double* out, hipStr
 {
     const int nb = 256;
     hipLaunchKernelGGL(k_sumsq_partial, dim3(nb), dim3(256), 0, s, v, n, part);
-    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(1), 0, s, part, nb, 1, out);
     HIP_TRY(hipGetLastError());
-    return ALTO_OK;
+    return sum_cols_device(part, nb, 1, out, nullptr, 0, s);
 }
 
-// ------------------------------------------------------------------ batched mode updates
-// The mode-j update of several CP-ALS models (lockstep sessions of one rank
-// and precision) in one launch per kernel: each kernel's table (up to
-// DENSE_BATCH_MAX jobs, in the kernel arguments) gives job k the logical
-// blocks [start[k], start[k + 1]) -- its own launch's grid -- and each block
-// finds its job by a uniform scan.  The bodies are the single-model
-// kernels', so every job computes what its own launches would.
-template <typename J>
+// ------------------------------------------------------------------ mode updates
+// The update of one mode after its MTTKRP, of one CP-ALS model or of several
+// (lockstep sessions of one rank and precision): each kernel's table (N jobs,
+// in the kernel arguments) gives job k the logical blocks [start[k],
+// start[k + 1]) and each block finds its job by a uniform scan, so a model's
+// values do not depend on which others share the launch.
+//
+// In general five launches: inverse, row solves, lambda, scaling + Gram,
+// partial sums + clearing of the next M.  Small modes are bound by the launches
+// themselves (2 to 8 us each and a gap behind it), so there
+//   - up to rank 32 every row-solve block inverts V for itself while its rows
+//     of M are on their way (fuse_inverse),
+//   - every Gram block takes lambda from the row solves' partials itself
+//     (fuse_lambda: at most 2048 of each, 16 KB per block),
+//   - the Gram stays in partials, which the blocks of the next mode's row
+//     solves (and the fit) add up for themselves, in the same order, and the
+//     Gram launch clears the next M in blocks of its own,
+// which leaves two launches.  Measured: 16 models of 10K-200K nonzeros, rank
+// 16: the dense kernels of a mode step 31 -> 23 us in 2 launches instead of 5;
+// 1000 rows, rank 16, one model: 23 -> 16.5 us.  (A single workgroup doing the
+// whole update took 18.6 us for those 1000 rows, bound by what one CU can load
+// and store.)  Where the lines lie, whole mode updates of three equal modes
+// just below and above each: inverse in the row solves, rank 16, 32768 rows 59
+// against 63 us, rank 32, 16384 rows 80.5 and 32768 rows 90 against 82 us;
+// lambda in the Gram launch, rank 16, 8192 rows 52.3 against 52.1 us, rank 64,
+// 2048 rows 112 against 111 us (so it ends there); Gram in partials, rank 16,
+// 2048 rows 48 us, 4096 rows 51.5 against 50.4 us.
+static bool fuse_inverse(uint64_t I, int R) { return R <= 32 && solve_blocks(I, R) <= (R <= 16 ? 512 : 256); }
+static bool fuse_lambda(uint64_t I, int R) { return solve_blocks(I, R) * R <= 2048; }
+bool gram_can_stay_partial(uint64_t I, int R, uint64_t next_I)
+{
+    return fuse_inverse(next_I, R) && (uint64_t)gram_blocks(I) * R * R <= 2048;
+}
+
+template <typename J, int N>
 struct BatchTab {
-    J a[DENSE_BATCH_MAX];
-    uint32_t start[DENSE_BATCH_MAX + 1];
+    J a[N];
+    uint32_t start[N + 1];
     int n;
 };
-template <typename J>
-__device__ inline int batch_job(const BatchTab<J>& t, uint32_t b)
+template <typename J, int N>
+__device__ inline int batch_job(const BatchTab<J, N>& t, uint32_t b)
 {
     int k = 0;
     while (k + 1 < t.n && b >= t.start[k + 1]) ++k;
@@ -1110,6 +1215,13 @@ struct ApplyJob {
     double *psum, *pmax, *pin;
     uint64_t I;
 };
+struct SolveJob {
+    PendingGram pend;
+    ApplyJob x;
+    double* grams;
+    int* status;
+    int nmode, mode;
+};
 struct LambdaJob {
     const double *psum, *pmax;
     double* lambda;
@@ -1118,11 +1230,18 @@ struct LambdaJob {
 struct GramJob {
     void* U;
     void* S;
-    const double* lambda;
+    double* lambda;
     double* part;
     const double* Mi;
     double* pin;
     uint64_t I, rpb;
+    // lambda from the row solves' nb partials (psum null: it is there)
+    const double *psum, *pmax;
+    int nb, which;
+    // blocks from ngram on clear `zero`
+    uint32_t ngram;
+    void* zero;
+    uint64_t nz;
 };
 struct SumJob {
     const double* part;
@@ -1132,6 +1251,7 @@ struct SumJob {
     int nparts, nsum;
 };
 struct FitJob {
+    PendingGram pend;
     const double *grams, *lambda, *pin;
     double* out;
     double* gather;
@@ -1139,38 +1259,120 @@ struct FitJob {
     int nmode, nb;
 };
 
-template <int BT, int NPT>
-__global__ void __launch_bounds__(BT) k_spd_inverse_batch(BatchTab<SpdJob> t, int R)
+template <int BT, int RPW, int N>
+__global__ void __launch_bounds__(BT) k_spd_inverse_batch(BatchTab<SpdJob, N> t, int R)
 {
     const SpdJob& j = t.a[blockIdx.x];
-    spd_inverse_body<BT, NPT>(j.grams, j.nmode, j.mode, R, j.P, j.status, j.wsA, j.wsQ);
+    spd_inverse_body<RPW, 1>(j.grams, j.nmode, j.mode, R, j.P, j.status, j.wsA, j.wsQ);
 }
 
-template <typename MT, typename UT, int T16, bool LOWP>
-__global__ void __launch_bounds__(256) k_apply_batch(BatchTab<ApplyJob> t, int R)
+template <typename MT, typename UT, int T16, bool LOWP, int N>
+__global__ void __launch_bounds__(256) k_apply_batch(BatchTab<ApplyJob, N> t, int R)
 {
     const int k = batch_job(t, blockIdx.x);
     const ApplyJob& j = t.a[k];
-    apply_body<MT, UT, T16, LOWP>(j.M, j.I, R, j.P, (UT*)j.U, j.psum, j.pmax, j.pin, blockIdx.x - t.start[k],
+    apply_body<MT, UT, T16, LOWP>(j.M, j.I, R, WFrom{j.P, R}, (UT*)j.U, j.psum, j.pmax, j.pin, blockIdx.x - t.start[k],
                                   t.start[k + 1] - t.start[k]);
 }
 
-__global__ void __launch_bounds__(256) k_lambda_batch(BatchTab<LambdaJob> t, int R)
+// Row solves that invert V themselves (R <= 32).  V is put together in LDS by
+// all threads; the model's first block leaves a pending Gram's sum in its place.
+// The pseudo-inverse of a failed pivot is every block's own too, in LDS.
+template <typename UT, int T16, bool LOWP, int N>
+__global__ void __launch_bounds__(256) k_solve_batch(BatchTab<SolveJob, N> t, int R)
+{
+    constexpr int C = 16 * T16;
+    __shared__ double s_v[C * C], s_p[C * C], s_q[C * C];
+    const int k = batch_job(t, blockIdx.x);
+    const SolveJob& j = t.a[k];
+    const uint32_t bid = blockIdx.x - t.start[k];
+    auto prepare = [&](auto* sW, int WS) {
+        using T = typename std::remove_pointer<decltype(sW)>::type;
+        for (int e = threadIdx.x; e < C * C; e += 256) {
+            const int i = e / C, c = e % C;
+            if (i < R && c < R) {
+                double v = 1.0;
+#pragma unroll
+                for (int m = 0; m < ALTO_MAXN; ++m)
+                    if (m < j.nmode && m != j.mode && m != j.pend.mode) v *= j.grams[(size_t)m * R * R + i * R + c];
+                if (j.pend.mode >= 0) {
+                    const double g = j.pend.sum(i * R + c, R);
+                    if (bid == 0) j.grams[(size_t)j.pend.mode * R * R + i * R + c] = g;
+                    if (j.pend.mode != j.mode) v *= g;
+                }
+                s_v[i * R + c] = v;
+            }
+        }
+        __syncthreads();
+        const bool ok = spd_inverse<T16 == 1 ? 0 : 4 * T16, 1>(
+            R, [&](int i, int c) { return s_v[i * R + c]; }, [&](int i, int c, double v) { sW[i * WS + c] = (T)v; });
+        if (threadIdx.x == 0 && bid == 0) *j.status = ok ? 0 : 1;
+        if (!ok) {  // uniform
+            for (int e = threadIdx.x; e < R * R; e += 256) {  // symmetric, from the lower triangle
+                const int i = e / R, c = e % R;
+                s_p[e] = s_v[max(i, c) * R + min(i, c)];
+            }
+            __syncthreads();
+            pinv_body(R, s_p, s_q, s_v);
+            __syncthreads();
+            for (int e = threadIdx.x; e < R * R; e += 256) sW[(e / R) * WS + e % R] = (T)s_v[e];
+        }
+        __syncthreads();
+    };
+    apply_body<double, UT, T16, LOWP>(j.x.M, j.x.I, R, prepare, (UT*)j.x.U, j.x.psum, j.x.pmax, j.x.pin, bid,
+                                      t.start[k + 1] - t.start[k]);
+}
+
+template <int N>
+__global__ void __launch_bounds__(256) k_lambda_batch(BatchTab<LambdaJob, N> t, int R)
 {
     const LambdaJob& j = t.a[blockIdx.x / R];
     lambda_body(j.psum, j.pmax, j.nb, R, j.which, j.lambda, blockIdx.x % R);
 }
 
-template <typename T, typename ST, bool F64, int T16, bool INNER>
-__global__ void __launch_bounds__(256) k_gram_rows_batch(BatchTab<GramJob> t, int R)
+template <typename T, typename ST, bool F64, int T16, bool INNER, int N>
+__global__ void __launch_bounds__(256) k_gram_rows_batch(BatchTab<GramJob, N> t, int R)
 {
     const int k = batch_job(t, blockIdx.x);
     const GramJob& j = t.a[k];
-    gram_rows_body<T, ST, F64, T16, true, INNER>((T*)j.U, j.I, R, j.rpb, j.part, j.lambda, (ST*)j.S, j.Mi, j.pin,
-                                                 blockIdx.x - t.start[k]);
+    const uint32_t bid = blockIdx.x - t.start[k];
+    if (bid >= j.ngram) {
+        clear_body(j.zero, j.nz, bid - j.ngram, t.start[k + 1] - t.start[k] - j.ngram);
+        return;
+    }
+    const double* lambda = j.lambda;
+    __shared__ double s_lambda[16 * T16];
+    if (j.psum) {  // uniform
+        // thread (g, c) takes every G-th partial of column c, the G sums are
+        // added in order: the same in every block
+        constexpr int CW = T16 == 1 ? 16 : T16 == 2 ? 32 : 64, G = 256 / CW;
+        __shared__ double s_a[256], s_b[256];
+        const int c = threadIdx.x % CW, g = threadIdx.x / CW;
+        double a = 0, b = -INFINITY;
+        if (c < R)
+            for (int p = g; p < j.nb; p += G) {
+                a += j.psum[(size_t)p * R + c];
+                b = fmax(b, j.pmax[(size_t)p * R + c]);
+            }
+        s_a[threadIdx.x] = a;
+        s_b[threadIdx.x] = b;
+        __syncthreads();
+        if ((int)threadIdx.x < R) {
+            for (int q = 1; q < G; ++q) {
+                a += s_a[q * CW + c];
+                b = fmax(b, s_b[q * CW + c]);
+            }
+            s_lambda[c] = lambda_of(j.which, a, b);
+            if (bid == 0) j.lambda[c] = s_lambda[c];
+        }
+        __syncthreads();
+        lambda = s_lambda;
+    }
+    gram_rows_body<T, ST, F64, T16, true, INNER>((T*)j.U, j.I, R, j.rpb, j.part, lambda, (ST*)j.S, j.Mi, j.pin, bid);
 }
 
-__global__ void __launch_bounds__(256) k_sum_cols_batch(BatchTab<SumJob> t, int n)
+template <int N>
+__global__ void __launch_bounds__(256) k_sum_cols_batch(BatchTab<SumJob, N> t, int n)
 {
     const int k = batch_job(t, blockIdx.x);
     const SumJob& j = t.a[k];
@@ -1178,11 +1380,145 @@ __global__ void __launch_bounds__(256) k_sum_cols_batch(BatchTab<SumJob> t, int 
                   t.start[k + 1] - t.start[k]);
 }
 
-__global__ void __launch_bounds__(256) k_fit_batch(BatchTab<FitJob> t, int R)
+__global__ void __launch_bounds__(256) k_fit_batch(BatchTab<FitJob, DENSE_BATCH_MAX> t, int R)
 {
     const FitJob& j = t.a[blockIdx.x];
-    fit_body(j.grams, j.nmode, R, j.lambda, j.pin, j.nb, 1, j.normX, j.out);
+    fit_body(j.grams, j.pend, j.nmode, R, j.lambda, j.pin, j.nb, 1, j.normX, j.out);
     if (threadIdx.x == 0) j.gather[0] = j.out[0];
+}
+
+// blocks that clear nz bytes
+static uint32_t clear_blocks(uint64_t nz)
+{
+    uint64_t b = (nz / 16 + 255) / 256;
+    if (b > 1024) b = 1024;
+    return (uint32_t)(nz && b == 0 ? 1 : b);
+}
+
+template <typename UT, typename ST, int N>
+static int mode_solve(int n, const DenseModeJob* m, int R, hipStream_t s)
+{
+    BatchTab<SpdJob, N> sp{};
+    BatchTab<ApplyJob, N> ap{};
+    BatchTab<SolveJob, N> so{};
+    for (int k = 0; k < n; ++k) {
+        const DenseModeJob& x = m[k];
+        const ApplyJob a{x.M, x.P, x.U, x.psum, x.pmax, x.pin, x.I};
+        if (fuse_inverse(x.I, R)) {
+            so.a[so.n] = SolveJob{x.pend, a, x.grams, x.status, x.nmode, x.mode};
+            so.start[so.n + 1] = so.start[so.n] + (uint32_t)x.nb;
+            ++so.n;
+            continue;
+        }
+        if (x.pend.mode >= 0) {
+            set_error("mode update: a Gram in partials before a mode of %llu rows", (unsigned long long)x.I);
+            return ALTO_ERR_UNSUPPORTED;
+        }
+        sp.a[sp.n++] = SpdJob{x.grams, x.P, x.wsA, x.wsQ, x.status, x.nmode, x.mode};
+        ap.a[ap.n] = a;
+        ap.start[ap.n + 1] = ap.start[ap.n] + (uint32_t)x.nb;
+        ++ap.n;
+    }
+    const size_t lds = (size_t)R * (R + 2) * 8;
+    const bool lowp = std::is_same<UT, float>::value && !dense_f64_enabled();
+    if (so.n) {
+#define SO_(TT, L) hipLaunchKernelGGL((k_solve_batch<UT, TT, L, N>), dim3(so.start[so.n]), dim3(256), lds, s, so, R)
+#define SOT_(TT)                                         \
+    do {                                                 \
+        if constexpr (std::is_same<UT, float>::value) {  \
+            if (lowp) SO_(TT, true);                     \
+            else SO_(TT, false);                         \
+        } else {                                         \
+            SO_(TT, false);                              \
+        }                                                \
+    } while (0)
+        if (R <= 16) SOT_(1);
+        else SOT_(2);
+#undef SOT_
+#undef SO_
+    }
+    if (ap.n) {
+#define SPD_(BT, RPW) hipLaunchKernelGGL((k_spd_inverse_batch<BT, RPW, N>), dim3(sp.n), dim3(BT), 0, s, sp, R)
+        if (R <= 16) SPD_(256, 0);
+        else if (R <= 32) SPD_(1024, 2);
+        else SPD_(1024, 4);
+#undef SPD_
+#define AP_(TT)                                                                                                       \
+    do {                                                                                                              \
+        if (lowp)                                                                                                     \
+            hipLaunchKernelGGL((k_apply_batch<double, UT, TT, true, N>), dim3(ap.start[ap.n]), dim3(256), lds, s, ap, R); \
+        else                                                                                                          \
+            hipLaunchKernelGGL((k_apply_batch<double, UT, TT, false, N>), dim3(ap.start[ap.n]), dim3(256), lds, s, ap, \
+                               R);                                                                                    \
+    } while (0)
+        switch ((R + 15) / 16) {
+        case 1: AP_(1); break;
+        case 2: AP_(2); break;
+        case 3: AP_(3); break;
+        default: AP_(4); break;
+        }
+#undef AP_
+    }
+    HIP_TRY(hipGetLastError());
+    return ALTO_OK;
+}
+
+template <typename UT, typename ST, int N>
+static int mode_lambda(int n, const DenseModeJob* m, int R, hipStream_t s)
+{
+    BatchTab<LambdaJob, N> la{};
+    for (int k = 0; k < n; ++k)
+        if (!fuse_lambda(m[k].I, R))
+            la.a[la.n++] = LambdaJob{m[k].psum, m[k].pmax, m[k].lambda, m[k].nb, m[k].which};
+    if (!la.n) return ALTO_OK;
+    hipLaunchKernelGGL((k_lambda_batch<N>), dim3(la.n * R), dim3(256), 0, s, la, R);
+    HIP_TRY(hipGetLastError());
+    return ALTO_OK;
+}
+
+template <typename UT, typename ST, int N>
+static int mode_gram(int n, const DenseModeJob* m, int R, bool f64, hipStream_t s)
+{
+    constexpr bool same = std::is_same<UT, ST>::value;
+    BatchTab<GramJob, N> gr{};
+    BatchTab<SumJob, N> su{};
+    gr.n = n;
+    for (int k = 0; k < n; ++k) {
+        const DenseModeJob& x = m[k];
+        const int gb = gram_blocks(x.I);
+        const uint64_t rpb = ((x.I + gb - 1) / gb + 15) / 16 * 16;
+        const bool fl = fuse_lambda(x.I, R);
+        gr.a[k] = GramJob{x.U, same ? nullptr : x.S, x.lambda, x.gpart, x.Mgram, x.pin_gram, x.I, rpb,
+                          fl ? x.psum : nullptr, x.pmax, x.nb, x.which, (uint32_t)gb, x.zero, x.defer ? x.zero_bytes : 0};
+        gr.start[k + 1] = gr.start[k] + (uint32_t)gb + (x.defer ? clear_blocks(x.zero_bytes) : 0);
+        if (x.defer) continue;
+        const int nsum = (R * R + 31) / 32;
+        su.a[su.n] = SumJob{x.gpart, x.G, x.zero, x.zero_bytes, gb, nsum};
+        su.start[su.n + 1] = su.start[su.n] + (uint32_t)nsum + clear_blocks(x.zero_bytes);
+        ++su.n;
+    }
+    const size_t lds = (size_t)R * R * 8;
+    // storage that rounds (BF16): the last modes' fit inner products from
+    // the stored values, in the same launch
+#define GS_(TT)                                                                                                        \
+    do {                                                                                                               \
+        if (f64)                                                                                                       \
+            hipLaunchKernelGGL((k_gram_rows_batch<UT, ST, true, TT, !same, N>), dim3(gr.start[n]), dim3(256), lds, s, gr, \
+                               R);                                                                                     \
+        else                                                                                                           \
+            hipLaunchKernelGGL((k_gram_rows_batch<UT, ST, false, TT, !same, N>), dim3(gr.start[n]), dim3(256), lds, s, \
+                               gr, R);                                                                                 \
+    } while (0)
+    switch ((R + 15) / 16) {
+    case 1: GS_(1); break;
+    case 2: GS_(2); break;
+    case 3: GS_(3); break;
+    default: GS_(4); break;
+    }
+#undef GS_
+    if (su.n) hipLaunchKernelGGL((k_sum_cols_batch<N>), dim3(su.start[su.n]), dim3(256), 0, s, su, R * R);
+    HIP_TRY(hipGetLastError());
+    return ALTO_OK;
 }
 
 template <typename UT, typename ST>
@@ -1192,81 +1528,24 @@ int dense_mode_batch(int n, const DenseModeJob* m, int R, bool f64, hipStream_t 
         set_error("dense_mode_batch: %d jobs of rank %d (1..%d jobs, rank 1..64)", n, R, DENSE_BATCH_MAX);
         return ALTO_ERR_ARG;
     }
-    constexpr bool same = std::is_same<UT, ST>::value;
-    BatchTab<SpdJob> sp{};
-    BatchTab<ApplyJob> ap{};
-    BatchTab<LambdaJob> la{};
-    BatchTab<GramJob> gr{};
-    BatchTab<SumJob> su{};
-    sp.n = ap.n = la.n = gr.n = su.n = n;
-    ap.start[0] = gr.start[0] = su.start[0] = 0;
-    for (int k = 0; k < n; ++k) {
-        const DenseModeJob& x = m[k];
-        sp.a[k] = SpdJob{x.grams, x.P, x.wsA, x.wsQ, x.status, x.nmode, x.mode};
-        ap.a[k] = ApplyJob{x.M, x.P, x.U, x.psum, x.pmax, x.pin, x.I};
-        ap.start[k + 1] = ap.start[k] + (uint32_t)x.nb;
-        la.a[k] = LambdaJob{x.psum, x.pmax, x.lambda, x.nb, x.which};
-        const int gb = gram_blocks(x.I);
-        const uint64_t rpb = ((x.I + gb - 1) / gb + 15) / 16 * 16;
-        gr.a[k] = GramJob{x.U, same ? nullptr : x.S, x.lambda, x.gpart, x.Mgram, x.pin_gram, x.I, rpb};
-        gr.start[k + 1] = gr.start[k] + (uint32_t)gb;
-        // the sums and the clearing of the next mode's M, as sum_cols_device
-        const int nsum = (R * R + 31) / 32;
-        uint64_t nzb = (x.zero_bytes / 16 + 255) / 256;
-        if (nzb > 1024) nzb = 1024;
-        if (x.zero_bytes && nzb == 0) nzb = 1;
-        su.a[k] = SumJob{x.gpart, x.G, x.zero, x.zero_bytes, gb, nsum};
-        su.start[k + 1] = su.start[k] + (uint32_t)(nsum + nzb);
-    }
-#define SPD_(BT, NPT) hipLaunchKernelGGL((k_spd_inverse_batch<BT, NPT>), dim3(n), dim3(BT), 0, s, sp, R)
-    if (R <= 16) SPD_(256, 1);
-    else if (R <= 32) SPD_(1024, 1);
-    else SPD_(1024, 4);
-#undef SPD_
-    const size_t lds_ap = (size_t)R * (R + 2) * 8;
-    const bool lowp = std::is_same<UT, float>::value && !dense_f64_enabled();
-#define AP_(TT)                                                                                                  \
-    do {                                                                                                         \
-        if (lowp)                                                                                                \
-            hipLaunchKernelGGL((k_apply_batch<double, UT, TT, true>), dim3(ap.start[n]), dim3(256), lds_ap, s, ap, R); \
-        else                                                                                                     \
-            hipLaunchKernelGGL((k_apply_batch<double, UT, TT, false>), dim3(ap.start[n]), dim3(256), lds_ap, s, ap, \
-                               R);                                                                               \
-    } while (0)
-    switch ((R + 15) / 16) {
-    case 1: AP_(1); break;
-    case 2: AP_(2); break;
-    case 3: AP_(3); break;
-    default: AP_(4); break;
-    }
-#undef AP_
-    hipLaunchKernelGGL(k_lambda_batch, dim3(n * R), dim3(256), 0, s, la, R);
-    const size_t lds_gr = (size_t)R * R * 8;
-    // storage that rounds (BF16): the last modes' fit inner products from
-    // the stored values, in the same launch
-#define GS_(TT)                                                                                                     \
-    do {                                                                                                            \
-        if (f64)                                                                                                    \
-            hipLaunchKernelGGL((k_gram_rows_batch<UT, ST, true, TT, !same>), dim3(gr.start[n]), dim3(256), lds_gr, s, \
-                               gr, R);                                                                              \
-        else                                                                                                        \
-            hipLaunchKernelGGL((k_gram_rows_batch<UT, ST, false, TT, !same>), dim3(gr.start[n]), dim3(256), lds_gr, \
-                               s, gr, R);                                                                           \
-    } while (0)
-    switch ((R + 15) / 16) {
-    case 1: GS_(1); break;
-    case 2: GS_(2); break;
-    case 3: GS_(3); break;
-    default: GS_(4); break;
-    }
-#undef GS_
-    hipLaunchKernelGGL(k_sum_cols_batch, dim3(su.start[n]), dim3(256), 0, s, su, R * R);
-    HIP_TRY(hipGetLastError());
-    return ALTO_OK;
+    ALTO_TRY((mode_solve<UT, ST, DENSE_BATCH_MAX>(n, m, R, s)));
+    ALTO_TRY((mode_lambda<UT, ST, DENSE_BATCH_MAX>(n, m, R, s)));
+    return mode_gram<UT, ST, DENSE_BATCH_MAX>(n, m, R, f64, s);
 }
 template int dense_mode_batch<double, double>(int, const DenseModeJob*, int, bool, hipStream_t);
 template int dense_mode_batch<float, float>(int, const DenseModeJob*, int, bool, hipStream_t);
 template int dense_mode_batch<float, bf16_t>(int, const DenseModeJob*, int, bool, hipStream_t);
+
+template <typename UT, typename ST>
+int dense_mode_one(const DenseModeJob& m, int R, bool f64, hipStream_t s, int step)
+{
+    if (step == 0) return mode_solve<UT, ST, 1>(1, &m, R, s);
+    if (step == 1) return mode_lambda<UT, ST, 1>(1, &m, R, s);
+    return mode_gram<UT, ST, 1>(1, &m, R, f64, s);
+}
+template int dense_mode_one<double, double>(const DenseModeJob&, int, bool, hipStream_t, int);
+template int dense_mode_one<float, float>(const DenseModeJob&, int, bool, hipStream_t, int);
+template int dense_mode_one<float, bf16_t>(const DenseModeJob&, int, bool, hipStream_t, int);
 
 int fit_batch(int n, const DenseFitJob* f, int R, hipStream_t s)
 {
@@ -1274,10 +1553,10 @@ int fit_batch(int n, const DenseFitJob* f, int R, hipStream_t s)
         set_error("fit_batch: %d jobs (1..%d)", n, DENSE_BATCH_MAX);
         return ALTO_ERR_ARG;
     }
-    BatchTab<FitJob> t{};
+    BatchTab<FitJob, DENSE_BATCH_MAX> t{};
     t.n = n;
     for (int k = 0; k < n; ++k)
-        t.a[k] = FitJob{f[k].grams, f[k].lambda, f[k].pin, f[k].out, f[k].gather, f[k].normX, f[k].nmode, f[k].nb};
+        t.a[k] = FitJob{f[k].pend, f[k].grams, f[k].lambda, f[k].pin, f[k].out, f[k].gather, f[k].normX, f[k].nmode, f[k].nb};
     hipLaunchKernelGGL(k_fit_batch, dim3(n), dim3(256), 0, s, t, R);
     HIP_TRY(hipGetLastError());
     return ALTO_OK;

@@ -35,12 +35,26 @@ template <typename UT, typename MT>
 int inner_partial_device(const UT* U, const MT* Mm, uint64_t I, int R, double* part, hipStream_t s);
 int fit_device(const double* grams, int nmode, int R, const double* lambda, const double* ipart, double normX,
                double* out, hipStream_t s);
-int fit_scalar_device(const double* grams, int nmode, int R, const double* lambda, const double* pin, int nb,
-                      double normX, double* out, hipStream_t s);
 int random_factor_device(double* U, uint64_t n, uint64_t seed, int mode, hipStream_t s);
 int normsq_device(const double* v, uint64_t n, double* part, double* out, hipStream_t s);
 // alto_update_gram_noalloc (partials in a per-device scratch array)
 int gram_noalloc(const void* U, uint64_t dim, int R, int precision, double* gram, hipStream_t s);
+
+// The Gram of mode `mode` (-1: none) as n partials of R x R, not yet added up
+// into the array of Grams
+struct PendingGram {
+    const double* part = nullptr;
+    int mode = -1, n = 0;
+    __device__ double sum(int k, int R) const
+    {
+        double t = 0;
+        for (int p = 0; p < n; ++p) t += part[(size_t)p * R * R + k];
+        return t;
+    }
+};
+
+int fit_scalar_device(const double* grams, const PendingGram& pend, int nmode, int R, const double* lambda,
+                      const double* pin, int nb, double normX, double* out, hipStream_t s);
 
 // One CP-ALS model's mode update after its MTTKRP (M = M_mode): V^-1 from
 // the other modes' Grams, U = M V^-1 with the column statistics (and the
@@ -49,8 +63,10 @@ int gram_noalloc(const void* U, uint64_t dim, int R, int precision, double* gram
 // and the clearing of zero_bytes of `zero` -- the launches of chol_device,
 // solve_device, lambda_device and gram_scale_device for R <= 64
 struct DenseModeJob {
-    const double* grams;
+    double* grams;
     int nmode, mode;
+    PendingGram pend;  // a Gram that the update before this one left in partials
+    int defer;         // leave this one's in partials (gram_can_stay_partial)
     double *P, *wsA, *wsQ;
     int* status;
     const double* M;
@@ -69,14 +85,23 @@ struct DenseModeJob {
     const double* Mgram;
     double* pin_gram;
 };
+// whether a mode of I rows may leave its Gram in partials (DenseModeJob::defer)
+// when the next mode to be updated has next_I rows
+bool gram_can_stay_partial(uint64_t I, int R, uint64_t next_I);
+
 constexpr int DENSE_BATCH_MAX = 16;
 // the mode updates of n <= DENSE_BATCH_MAX models of one rank (<= 64) and
-// factor / storage types in 5 launches (one per kernel, all models each)
+// factor / storage types, all models in each launch
 template <typename UT, typename ST>
 int dense_mode_batch(int n, const DenseModeJob* jobs, int R, bool f64, hipStream_t s);
+// one model's update in its steps: 0 = row solves, 1 = lambda, 2 = scaling,
+// Gram and clearing
+template <typename UT, typename ST>
+int dense_mode_one(const DenseModeJob& job, int R, bool f64, hipStream_t s, int step);
 // the fits of n <= DENSE_BATCH_MAX models (fit_scalar_device each), one
 // launch; each fit is also copied to gather[0]
 struct DenseFitJob {
+    PendingGram pend;
     const double *grams, *lambda, *pin;
     double* out;
     double* gather;

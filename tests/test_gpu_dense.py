@@ -1,0 +1,105 @@
+"""GPU parity of the CP-ALS mode updates at the sizes where their launches
+change: the inverse per rank class, row solves that invert V themselves (up to
+rank 16 and 32768 rows, rank 32 and 16384), lambda taken in the Gram launch (64
+rows x rank up to 2048 x 64) and Grams left in partials (256-row blocks x rank^2
+up to 2048)."""
+import numpy as np
+import pytest
+import scipy.linalg
+
+import oracle
+from tests._tensors import uniform_tensor
+
+pytestmark = pytest.mark.gpu
+EPS = np.finfo(np.float64).eps
+
+
+def _A():
+    import alto_amd
+    return alto_amd
+
+
+def _run(dims, R, iters, dup=False, prec=0):
+    """(factors, lambda, fits) of the library and of the oracle."""
+    cidx, vals = uniform_tensor(dims, 6000, 17)
+    U, _ = oracle.random_init(dims, R, 3)
+    if dup:  # equal columns: V is singular and its elimination meets a zero pivot
+        for u in U:
+            u[:, R - 1] = u[:, 0]
+    g = _A().AltoTensor(dims, cidx, vals, nprtn=8)
+    s = _A().CpdSession(g, U, precision=prec)
+    fits, _ = s.iterate(iters)
+    return s.get(), fits, (dims, cidx, vals, U)
+
+
+def _als(dims, cidx, vals, U, iters):
+    """CP-ALS in numpy with the largest condition number of a V on the way."""
+    U = [u.copy() for u in U]
+    N, R, cond = len(dims), U[0].shape[1], 1.0
+    grams = [u.T @ u for u in U]
+    fits = []
+    for it in range(iters):
+        for j in range(N):
+            rows = np.prod([U[m][cidx[m].astype(np.int64)] for m in range(N) if m != j], axis=0) * vals[:, None]
+            M = np.zeros((dims[j], R))
+            np.add.at(M, cidx[j].astype(np.int64), rows)
+            V = np.prod([grams[m] for m in range(N) if m != j], axis=0)
+            cond = max(cond, np.linalg.cond(V))
+            u = scipy.linalg.solve(V, M.T, assume_a="pos").T
+            lam = np.sqrt((u * u).sum(0)) if it == 0 else np.maximum(u.max(0), 1.0)
+            U[j] = u / lam
+            grams[j] = U[j].T @ U[j]
+        normX = (vals * vals).sum()
+        inner = (M * U[-1] * lam).sum()
+        normU = lam @ np.prod(grams, axis=0) @ lam
+        fits.append(1 - np.sqrt(normX + normU - 2 * inner) / np.sqrt(normX))
+    return U, lam, fits, cond
+
+
+EDGES = [(1, 300), (15, 2048), (16, 2048), (16, 2049), (16, 8192), (16, 8193), (16, 32768), (16, 32769), (17, 512),
+         (31, 3800), (32, 512), (32, 513), (32, 16384), (32, 16385), (33, 2048), (48, 2730), (63, 2049), (64, 2048),
+         (64, 2049), (65, 500), (128, 300)]
+
+
+@pytest.mark.parametrize("R,rows", EDGES)
+def test_mode_updates_match_numpy(R, rows):
+    """Three iterations.  Every solve may lose cond(V) rounding errors per
+    term of its sums, and each update starts from the one before it."""
+    dims = [rows, 2 * R + 7, 3 * R + 5]
+    (U, lam, _, _), fits, args = _run(dims, R, 3)
+    Uo, lo, fo, cond = _als(*args, 3)
+    tol = 9 * 8 * R * EPS * cond
+    np.testing.assert_allclose(fits, fo, rtol=0, atol=tol)
+    np.testing.assert_allclose(lam, lo, rtol=tol)
+    for a, b in zip(U, Uo):
+        np.testing.assert_allclose(a, b, rtol=0, atol=tol * np.abs(b).max())
+
+
+@pytest.mark.parametrize("R", [2, 15, 16, 17, 32, 33, 64])
+def test_singular_v_takes_the_pseudo_inverse(R):
+    """The first update of a model with two equal columns against LAPACK's
+    minimum-norm solution (later updates see factors that differ from equal
+    columns by rounding)."""
+    dims = [70, 2 * R + 7, 3 * R + 5]
+    (U, _, _, _), _, (_, cidx, vals, U0) = _run(dims, R, 1, dup=True)
+    rows = U0[1][cidx[1].astype(np.int64)] * U0[2][cidx[2].astype(np.int64)] * vals[:, None]
+    M = np.zeros((dims[0], R))
+    np.add.at(M, cidx[0].astype(np.int64), rows)
+    V = (U0[1].T @ U0[1]) * (U0[2].T @ U0[2])
+    e = np.linalg.eigvalsh(V)
+    want = M @ np.linalg.pinv(V, rcond=1e-12, hermitian=True)
+    want /= np.sqrt((want * want).sum(0))
+    np.testing.assert_allclose(U[0], want, rtol=0, atol=64 * R * EPS * e[-1] / e[1] * np.abs(want).max())
+
+
+@pytest.mark.parametrize("prec,tol", [(1, 1e-4), (2, 1e-3)])
+@pytest.mark.parametrize("R,rows", [(16, 2048), (16, 8193), (32, 513), (64, 2049)])
+def test_mode_updates_reduced_precision(prec, tol, R, rows):
+    """FP32 / BF16 models: the fit within the bounds the CP-ALS runs of these
+    precisions keep elsewhere."""
+    dims = [rows, 2 * R + 7, 3 * R + 5]
+    _, fits, (_, cidx, vals, U) = _run(dims, R, 4, prec=prec)
+    o = oracle.OracleAlto(dims, cidx, vals, nprtn=8)
+    Uo, lo = oracle.random_init(dims, R, 3)
+    _, fo = o.cpd_als(Uo, lo, 4, 0.0)
+    assert abs(fits[-1] - fo[-1]) <= tol * max(1.0, abs(fo[-1]))

@@ -48,32 +48,31 @@ int tuned_seg(uint64_t nnz, int G, int acc_bytes)
     return seg;
 }
 
-// Nonzeros walked by one lane group of the vector-lane MTTKRP kernels (G
-// lanes, E columns per lane), whose workgroups combine their groups' last
-// rows before they flush (flush_last_rows), so that a segment need not be
-// long for the heavy rows' sake.  A group walks its segment in steps that
-// each wait for their gathers; the shorter it is, the more wavefronts hide
-// that.  About 4096 wavefronts (four per SIMD) are enough, more only add
-// flushes: nnz G / 2^18 nonzeros as a power of two, between
+// Nonzeros walked by one lane group (G lanes) of the vector-lane MTTKRP kernels,
+// whose workgroups combine their groups' last rows before they flush
+// (flush_last_rows), so that a segment need not be long for the heavy rows'
+// sake.  A group walks its segment in steps that each wait for their gathers;
+// the shorter it is, the more wavefronts hide that.  About 4096 wavefronts
+// (four per SIMD) are enough, more only add flushes: nnz G / 2^18 nonzeros,
+// the largest power of two below two thirds of that, between
 //  - 8, or G / 2 (a workgroup of few wide groups combines little: rank 64,
 //    60K nonzeros: 17 us at 8, 13.4 at 16 and 32) and
-//  - 32 (G <= 4), 64, or 128 (four columns per lane, G >= 32): a workgroup
-//    then covers one to four thousand nonzeros, and the heavy rows' atomics
-//    no longer show.
-// All-mode averages in FP64 at 8, 16, 32, 64, 128, 256 (before, with the rule
-// above and no combining): rank 16, 200K nonzeros 11.2, 12.3, 14.4, 21, 34, 56
-// us (24.6); 1000^3, 1M, rank 16 23, 21, 19, 19, 25, 41 us (24.7); 4 modes,
-// 3M, rank 32 179, 104, 81, 82, 86, 93 us (142); at 32 .. 1024: 20M, rank 32
-// 458, 445, 462, 494, 578, 791 us (664); 76.9M, rank 32 1308, 1230, 1259,
-// 1280, 1349, 1416 us (1471).
-int lane_seg(uint64_t nnz, int G, int E)
+//  - 32 (G <= 4), 64, or 128 (G >= 32): a workgroup then covers one to four
+//    thousand nonzeros, and the heavy rows' atomics no longer show.
+// All-mode averages at 16, 32, 64, 128, 256: FP64 rank 16, 200K nonzeros 11.3,
+// 12.6, 17.6, 26.5, 44 us; 1000^3, 1M, rank 16 17.3, 17.6, 18.1, 22.6, 36 us; 4
+// modes, 3M, rank 16 50, 50, 54, 59, 83; 20M, rank 32 448, 427, 435, 454, 482;
+// rank 64 840, 689, 652, 643, 650; 76.9M, rank 32 1267, 1223, 1195, 1250, 1269;
+// FP32 4 modes, 3M, rank 32 57, 56, 60, 70, 98; BF16 rank 64, 8M 167 (32), 173,
+// 204, 263; 100M 2056 (32), 1967, 1954, 2007.
+int lane_seg(uint64_t nnz, int G)
 {
     if (g_seg > 0) return g_seg;
     const int lo = G / 2 > 8 ? G / 2 : 8;
-    const int hi = E >= 4 || G >= 32 ? 128 : G <= 4 ? 32 : 64;
+    const int hi = G <= 4 ? 32 : G >= 32 ? 128 : 64;
     const uint64_t want = nnz * (uint64_t)G >> 18;
     int seg = lo;
-    while (seg < hi && (uint64_t)seg * 3 / 2 < want) seg <<= 1;
+    while (seg < hi && (uint64_t)seg * 3 < want) seg <<= 1;
     return seg;
 }
 static int g_chunk = 0;
@@ -409,7 +408,7 @@ int alto_mttkrp_autotune(alto_tensor_t* t, uint64_t rank, int precision, const v
         best_ms = def_ms;
         // segment lengths within 4x of the size rule's choice (the others
         // measured slower on every tensor tried, up to 10x on large ones)
-        const int h = lane_seg(t->nnz, group_lanes(R), precision == ALTO_PREC_F64 ? 2 : 4);
+        const int h = lane_seg(t->nnz, group_lanes(R));
         for (int v : variants)
             for (int sg : segs) {
                 if (sg * 4 < h || sg > h * 4) continue;

@@ -319,6 +319,22 @@ template <int G, int L> __device__ __forceinline__ float bcast_val(float v)
     return __uint_as_float(bcast32<G, L>(__float_as_uint(v)));
 }
 
+// value of the lane before this one (of a group's first lane: not defined)
+template <int G> __device__ __forceinline__ uint32_t lane_before(uint32_t v)
+{
+    if constexpr (G <= 16) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);  // row_shr:1
+    else return (uint32_t)__shfl_up((int)v, 1);
+}
+// the lanes that hold position `src` of each group's slot
+template <int G> constexpr uint64_t position_lanes(int src)
+{
+    uint64_t m = 0;
+    for (int g = 0; g < 64; g += G) m |= 1ull << (g + src);
+    return m;
+}
+__device__ __forceinline__ float fused(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fused(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
 // First column of the E consecutive ones that lane gl of a group holds (R >= E).
 // Where E does not divide the rank the last lane moves back to the row's last
 // E columns: it shares some with its neighbour, which alone flushes them, and
@@ -327,13 +343,40 @@ template <int G, int L> __device__ __forceinline__ float bcast_val(float v)
 template <int E>
 __device__ __forceinline__ int first_col(int gl, int R) { return min(gl * E, R - E); }
 
-template <typename AT, typename OT, int E>
+// Adds the group's sums to an output row.  The sums change places through LDS
+// first (one wavefront's own, no barrier), so that each atomic instruction
+// covers G consecutive columns: the atomics' rate is that of the memory lines
+// they touch, and lanes of E columns each would touch every line E times.  3M
+// nonzeros in 262144 rows, 3 modes: BF16 rank 64 (E = 4) 469 -> 138 us, FP32 rank
+// 32 (E = 4) 258 -> 84, FP64 rank 16 (E = 2) 74 -> 62; in 512 rows, where
+// hardly anything is flushed, 61, 41 and 41 us.
+// DIRECT: without LDS (a lane that holds the whole row; kernels whose LDS is
+// taken).
+template <typename AT, typename OT, int G, int E, bool DIRECT = G == 1>
 __device__ __forceinline__ void flush_cols(OT* out, uint32_t row, int R, int gl, int cb, const AT (&acc)[E])
 {
-    OT* o = out + (uint64_t)row * R + cb;
+    OT* o = out + (uint64_t)row * R;
+    if constexpr (DIRECT) {
 #pragma unroll
-    for (int q = 0; q < E; ++q)
-        if (cb + q >= gl * E) atomic_add_hw(&o[q], (OT)acc[q]);
+        for (int q = 0; q < E; ++q)
+            if (cb + q >= gl * E) atomic_add_hw(&o[cb + q], (OT)acc[q]);
+    } else {
+        __shared__ __align__(16) AT s_row[256 * E];
+        // (the index is opaque: addresses kept in registers between the
+        // flushes cost the gathers a wavefront per SIMD)
+        int t = threadIdx.x;
+        asm volatile("" : "+v"(t));
+        AT* r = s_row + (t / G) * (G * E);
+        gl = t & (G - 1);
+#pragma unroll
+        for (int q = 0; q < E; ++q)
+            if (cb + q >= gl * E) r[cb + q] = acc[q];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int q = 0; q < E; ++q)
+            if (q * G + gl < R) atomic_add_hw(&o[q * G + gl], (OT)r[q * G + gl]);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
 }
 
 // The last row of every lane group of a workgroup, combined before it is
@@ -392,7 +435,7 @@ __device__ __forceinline__ void flush_last_rows(OT* out, uint32_t cur, int R, in
             if (!s_whole[w]) break;
         }
     }
-    flush_cols<OT, OT, E>(out, cur, R, gl, cb, sum);
+    flush_cols<OT, OT, G, E>(out, cur, R, gl, cb, sum);
 }
 
 // The MTTKRP stream kernel with 16-byte lanes: per batch of G nonzeros each
@@ -448,9 +491,11 @@ __device__ __forceinline__ void mttkrp16_body(const StreamArgs<FT, VT, OT>& a, u
         }
     }
 
+    uint32_t last = 0xffffffffu;  // the row before this batch
     for (uint64_t p = s; p < e; p += B) {
         uint32_t offs[NS][NO > 0 ? NO : 1];
-        uint32_t rown[NS];
+        uint32_t rown[NS], head[NS];
+        uint64_t heads[NS];
         VT myv[NS];
 #pragma unroll
         for (int k = 0; k < NS; ++k) {
@@ -458,20 +503,28 @@ __device__ __forceinline__ void mttkrp16_body(const StreamArgs<FT, VT, OT>& a, u
 #pragma unroll
             for (int o = 0; o < NO; ++o) offs[k][o] = (uint32_t)(field<PW>(kn[k], a.offo[o], a.bitso[o]) * (uint64_t)R);
             rown[k] = (uint32_t)field<PW>(kn[k], a.offn, a.bitsn);
+            uint32_t before = lane_before<G>(rown[k]);  // by every lane
+            before = gl == 0 ? last : before;
+            head[k] = rown[k] != before && p + k * G + gl < e;
+            heads[k] = __ballot(head[k]);
+            last = bcast32<G, G - 1>(rown[k]);
         }
         const int cnt = (int)(e - p < (uint64_t)B ? e - p : (uint64_t)B);
         static_for<0, B / J>([&](auto bi) {
             constexpr int j0 = decltype(bi)::value * J;
             if (j0 >= cnt) return;
-            AT prod[J][E];
-            uint32_t rj[J];
+            // the last mode's row stays apart for the fused multiply-add (RTNO:
+            // it is not known here which mode is the last)
+            AT prod[J][E], xl[J][E];
             static_for<0, J>([&](auto ji) {
                 constexpr int jj = decltype(ji)::value;
                 constexpr int slot = (j0 + jj) / G, src = (j0 + jj) % G;
-                rj[jj] = bcast32<G, src>(rown[slot]);
                 const AT v = (AT)bcast_val<G, src>(myv[slot]);
 #pragma unroll
-                for (int q = 0; q < E; ++q) prod[jj][q] = v;
+                for (int q = 0; q < E; ++q) {
+                    prod[jj][q] = v;
+                    xl[jj][q] = (AT)1;
+                }
             });
             static_for<0, NO>([&](auto oi) {
                 constexpr int o = decltype(oi)::value;
@@ -487,7 +540,10 @@ __device__ __forceinline__ void mttkrp16_body(const StreamArgs<FT, VT, OT>& a, u
                     if constexpr ((HM >> o) & 1) VecLoad<FT, E>::load(H + off + cb, x);
                     else VecLoad<FT, E>::load(U + off + cb, x);
 #pragma unroll
-                    for (int q = 0; q < E; ++q) prod[jj][q] *= x[q];
+                    for (int q = 0; q < E; ++q) {
+                        if constexpr (!RTNO && o == NO - 1) xl[jj][q] = x[q];
+                        else prod[jj][q] *= x[q];
+                    }
                 });
             });
             if constexpr (j0 == 0) {
@@ -505,24 +561,30 @@ __device__ __forceinline__ void mttkrp16_body(const StreamArgs<FT, VT, OT>& a, u
                     }
                 }
             }
-#pragma unroll
-            for (int jj = 0; jj < J; ++jj) {
-                if (j0 + jj < cnt) {
-                    if (rj[jj] != cur) {
-                        if (cur != 0xffffffffu) flush_cols<AT, OT, E>(a.out, cur, R, gl, cb, acc);
-                        cur = rj[jj];
+            static_for<0, J>([&](auto ji) {
+                constexpr int jj = decltype(ji)::value;
+                constexpr int slot = (j0 + jj) / G, src = (j0 + jj) % G;
+                constexpr uint64_t here = position_lanes<G>(src);
+                if (heads[slot] & here) {  // uniform
+                    if (bcast32<G, src>(head[slot])) {
+                        if (cur != 0xffffffffu)
+                            flush_cols<AT, OT, G, E, HM != 0 || G == 1>(a.out, cur, R, gl, cb, acc);
+                        cur = bcast32<G, src>(rown[slot]);
 #pragma unroll
                         for (int q = 0; q < E; ++q) acc[q] = 0;
                     }
-#pragma unroll
-                    for (int q = 0; q < E; ++q) acc[q] += prod[jj][q];
                 }
-            }
+                if (j0 + jj < cnt) {
+#pragma unroll
+                    for (int q = 0; q < E; ++q)
+                        acc[q] = RTNO ? acc[q] + prod[jj][q] : fused(prod[jj][q], xl[jj][q], acc[q]);
+                }
+            });
         });
     }
     // (the split streams' kernels keep all of their LDS for staged rows)
     if constexpr (HM == 0) flush_last_rows<AT, OT, G, E>(a.out, cur, R, gl, cb, acc);
-    else if (cur != 0xffffffffu) flush_cols<AT, OT, E>(a.out, cur, R, gl, cb, acc);
+    else if (cur != 0xffffffffu) flush_cols<AT, OT, G, E, HM != 0 || G == 1>(a.out, cur, R, gl, cb, acc);
 }
 
 template <typename FT, typename VT, typename AT, typename OT, int G, int E, int PW, int NO, int HM>
@@ -536,18 +598,24 @@ __global__ void __launch_bounds__(256) k_mttkrp16(StreamArgs<FT, VT, OT> a)
 }
 
 // MTTKRP over a fiber-ordered stream (nonzeros ordered by (row, row of the
-// fiber mode a)): as k_mttkrp16, but the fiber-mode row U_a[row_a] is read
-// only where a fiber starts.  In each block of J nonzeros of a group, a
-// position whose fiber differs from the previous position's (for the first
-// position: from the previous block's last) is a fiber head; the wave loads
-// U_a rows at the positions where any of its groups has a head -- a
-// wave-uniform branch, so every lane loads (groups without a head reload
-// the row they already hold) and nothing is merged into live registers
-// between the issues -- and every other position reuses the row of the
-// last loaded one.  On long fibers most blocks need no U_a load: a
-// 3-mode MTTKRP then gathers one row per nonzero instead of two.  The other
-// NB = N - 2 modes' rows are gathered per nonzero; products are summed per
-// output row and flushed as in k_mttkrp16.
+// fiber mode a)): a fiber's nonzeros share U_a's row, so a lane group sums the
+// products of the value and the other modes' rows over the fiber and multiplies
+// the sum by U_a's row once, at the fiber's end, into the sum of the output row,
+// which is flushed as in k_mttkrp16.
+//
+// The bound is instruction issue as much as the gathers, so the per-nonzero part
+// is kept to broadcasts, loads and one fused multiply-add per column: which
+// nonzeros start a fiber is found while a batch is decoded (each lane compares
+// its nonzero with its neighbour's), travels as one ballot per batch, and
+// positions where no group of the wavefront starts a fiber pass the fiber code
+// by a scalar branch.  U_a's rows are loaded behind the block's gathers, at the
+// positions where any group has a head (ahead of them: 8% slower); `loaded`
+// reaches the sums through an opaque copy, so that they are not folded into the
+// branches of the loads.  76.9M nonzeros, rank 32: 26 -> 17 vector
+// instructions per position and five wavefronts per SIMD, 1219 -> 1196 us per
+// MTTKRP: what is left is the gathers' way through L1 (busy 80%) and L2 (16
+// TB/s; twice the gathers in flight per wavefront at four fewer wavefronts:
+// 1311 us).
 template <typename FT, typename VT, typename AT, typename OT, int G, int E, int PW, int NB>
 __global__ void __launch_bounds__(256) k_mttkrp_fib(StreamArgs<FT, VT, OT> a, const FT* __restrict__ Ua, int offa,
                                                    int bitsa)
@@ -566,12 +634,11 @@ __global__ void __launch_bounds__(256) k_mttkrp_fib(StreamArgs<FT, VT, OT> a, co
     const int R = a.rank;
     const int cb = first_col<E>(gl, R);
 
-    AT acc[E], ua_last[E];
+    AT acc[E], fib[E], ua[E];
 #pragma unroll
-    for (int q = 0; q < E; ++q) acc[q] = ua_last[q] = 0;
+    for (int q = 0; q < E; ++q) acc[q] = fib[q] = ua[q] = 0;
     uint32_t cur = 0xffffffffu;
-    uint32_t prev_a = 0;  // fiber row offset of the previous position
-    bool have_a = false;  // ua_last holds U_a at prev_a
+    uint32_t last = 0xffffffffu, last_a = 0;  // row and fiber row offset before this batch
 
     // this lane's nonzeros of the next batch (past the segment: row 0 of
     // every mode, value 0 -- valid memory, and never accumulated)
@@ -592,7 +659,8 @@ __global__ void __launch_bounds__(256) k_mttkrp_fib(StreamArgs<FT, VT, OT> a, co
 
     for (uint64_t p = s; p < e; p += B) {
         uint32_t offs[NS][NB];
-        uint32_t aoff[NS], rown[NS];
+        uint32_t aoff[NS], rown[NS], head[NS];
+        uint64_t heads[NS];
         VT myv[NS];
 #pragma unroll
         for (int k = 0; k < NS; ++k) {
@@ -601,24 +669,26 @@ __global__ void __launch_bounds__(256) k_mttkrp_fib(StreamArgs<FT, VT, OT> a, co
             for (int o = 0; o < NB; ++o) offs[k][o] = (uint32_t)(field<PW>(kn[k], a.offo[o], a.bitso[o]) * (uint64_t)R);
             aoff[k] = (uint32_t)(field<PW>(kn[k], offa, bitsa) * (uint64_t)R);
             rown[k] = (uint32_t)field<PW>(kn[k], a.offn, a.bitsn);
+            uint32_t before = lane_before<G>(rown[k]), before_a = lane_before<G>(aoff[k]);  // by every lane
+            before = gl == 0 ? last : before;
+            before_a = gl == 0 ? last_a : before_a;
+            head[k] = (rown[k] != before || aoff[k] != before_a) && p + k * G + gl < e;
+            heads[k] = __ballot(head[k]);
+            last = bcast32<G, G - 1>(rown[k]);
+            last_a = bcast32<G, G - 1>(aoff[k]);
         }
         const int cnt = (int)(e - p < (uint64_t)B ? e - p : (uint64_t)B);
         static_for<0, B / J>([&](auto bi) {
             constexpr int j0 = decltype(bi)::value * J;
             if (j0 >= cnt) return;
-            AT prod[J][E];
-            uint32_t rj[J], aj[J];
+            AT prod[J][E], xl[J][E];  // the last mode's row stays apart for the fused multiply-add
             static_for<0, J>([&](auto ji) {
                 constexpr int jj = decltype(ji)::value;
                 constexpr int slot = (j0 + jj) / G, src = (j0 + jj) % G;
-                rj[jj] = bcast32<G, src>(rown[slot]);
-                aj[jj] = bcast32<G, src>(aoff[slot]);
                 const AT v = (AT)bcast_val<G, src>(myv[slot]);
 #pragma unroll
                 for (int q = 0; q < E; ++q) prod[jj][q] = v;
             });
-            // issue: the other modes' rows of the J nonzeros, then U_a rows
-            // at the fiber heads
             static_for<0, NB>([&](auto oi) {
                 constexpr int o = decltype(oi)::value;
                 const FT* __restrict__ U = a.Uo[o];
@@ -629,23 +699,24 @@ __global__ void __launch_bounds__(256) k_mttkrp_fib(StreamArgs<FT, VT, OT> a, co
                     AT x[E];
                     VecLoad<FT, E>::load(U + off + cb, x);
 #pragma unroll
-                    for (int q = 0; q < E; ++q) prod[jj][q] *= x[q];
+                    for (int q = 0; q < E; ++q) {
+                        if constexpr (o == NB - 1) xl[jj][q] = x[q];
+                        else prod[jj][q] *= x[q];
+                    }
                 });
             });
             AT ra[J][E];
-            uint32_t ldm = 0;  // positions loaded (uniform)
-#pragma unroll
-            for (int jj = 0; jj < J; ++jj) {
-                const bool head = jj == 0 ? (!have_a || aj[0] != prev_a) : aj[jj] != aj[jj - 1];
-                if (__any(head)) {
-                    VecLoad<FT, E>::load(Ua + aj[jj] + cb, ra[jj]);
-                    ldm |= 1u << jj;
+            uint32_t loaded = 0;  // positions loaded (uniform)
+            static_for<0, J>([&](auto ji) {
+                constexpr int jj = decltype(ji)::value;
+                constexpr int slot = (j0 + jj) / G, src = (j0 + jj) % G;
+                constexpr uint64_t here = position_lanes<G>(src);
+                if (heads[slot] & here) { // uniform; the other groups reload their fiber's row
+                    VecLoad<FT, E>::load(Ua + bcast32<G, src>(aoff[slot]) + cb, ra[jj]);
+                    loaded |= 1u << jj;
                 }
-            }
-            // the mask reaches the selection below through an opaque copy, so
-            // that the selection is not folded into the branches above (which
-            // would chain every load to the next one's registers)
-            asm volatile("" : "+s"(ldm));
+            });
+            asm volatile("" : "+s"(loaded));
             if constexpr (j0 == 0) {
                 // the next batch's nonzeros, issued behind this block's gathers
 #pragma unroll
@@ -661,34 +732,36 @@ __global__ void __launch_bounds__(256) k_mttkrp_fib(StreamArgs<FT, VT, OT> a, co
                     }
                 }
             }
-            // math: each position's U_a row is that of the last load at or
-            // before it
+            static_for<0, J>([&](auto ji) {
+                constexpr int jj = decltype(ji)::value;
+                constexpr int slot = (j0 + jj) / G, src = (j0 + jj) % G;
+                constexpr uint64_t here = position_lanes<G>(src);
+                if ((loaded >> jj) & 1u) {  // uniform
+                    if (bcast32<G, src>(head[slot])) {
 #pragma unroll
-            for (int jj = 0; jj < J; ++jj) {
-                const bool use = (ldm >> jj) & 1u;
+                        for (int q = 0; q < E; ++q) {
+                            acc[q] = fused(fib[q], ua[q], acc[q]);
+                            fib[q] = 0;
+                            ua[q] = ra[jj][q];
+                        }
+                        const uint32_t row = bcast32<G, src>(rown[slot]);
+                        if (row != cur) {
+                            if (cur != 0xffffffffu) flush_cols<AT, OT, G, E>(a.out, cur, R, gl, cb, acc);
+                            cur = row;
 #pragma unroll
-                for (int q = 0; q < E; ++q) {
-                    ua_last[q] = use ? ra[jj][q] : ua_last[q];
-                    prod[jj][q] *= ua_last[q];
-                }
-            }
-            prev_a = aj[J - 1];
-            have_a = true;
-#pragma unroll
-            for (int jj = 0; jj < J; ++jj) {
-                if (j0 + jj < cnt) {
-                    if (rj[jj] != cur) {
-                        if (cur != 0xffffffffu) flush_cols<AT, OT, E>(a.out, cur, R, gl, cb, acc);
-                        cur = rj[jj];
-#pragma unroll
-                        for (int q = 0; q < E; ++q) acc[q] = 0;
+                            for (int q = 0; q < E; ++q) acc[q] = 0;
+                        }
                     }
-#pragma unroll
-                    for (int q = 0; q < E; ++q) acc[q] += prod[jj][q];
                 }
-            }
+                if (j0 + jj < cnt) {
+#pragma unroll
+                    for (int q = 0; q < E; ++q) fib[q] = fused(prod[jj][q], xl[jj][q], fib[q]);
+                }
+            });
         });
     }
+#pragma unroll
+    for (int q = 0; q < E; ++q) acc[q] = fused(fib[q], ua[q], acc[q]);
     flush_last_rows<AT, OT, G, E>(a.out, cur, R, gl, cb, acc);
 }
 
@@ -722,13 +795,14 @@ __global__ void __launch_bounds__(256) k_mttkrp16_batch(BatchTable<FT, VT, OT> t
 // against them is that a wavefront then holds twice the lane groups, each of
 // which flushes rows and starts fibers at its own positions.
 //   FP64: two columns, 16 bytes.
-//   FP32: four columns from rank 17 on (rank 32: 20M nonzeros, 4 modes, 254 us
-//     per MTTKRP against 328 with two; 76.9M, 3 modes, 755 against 927; rank
-//     16: 205 against 174).
-//   BF16: four from rank 33 on (rank 32: 3M nonzeros 63 us against 50; rank
-//     64: 2M nonzeros 66 against 84).
-// Below 1M nonzeros a launch is bound by latency and flushes and every rank
-// takes two columns (200K nonzeros, 5 modes, rank 32: 17 us against 19).
+//   FP32: four from rank 17 on (3M nonzeros, 4 modes, rank 32: 54 us per MTTKRP
+//     against 81 with two; 20M, 3 modes, rank 16: 177 against 166).
+//   BF16: eight from rank 33 on (rank 64: 3M nonzeros 67 us against 108 with
+//     two and 74 with four, 100M, 5 modes 1952 against 2503 with four; rank 32,
+//     20M nonzeros: 190 us with two, 213 with four).
+// Below 128K nonzeros a launch is bound by latency and every rank takes two
+// columns (rank 64 in BF16: 60K nonzeros 10.5 us against 12.6, 250K 15.4 against
+// 14.5; rank 32 in FP32: 60K 9.2 against 10.4, 250K 14.4 against 11.1).
 template <typename FT, typename VT, typename OT>
 inline int lane_cols(const StreamArgs<FT, VT, OT>& a, uint64_t nnz, int R, const MttkrpTune& k)
 {
@@ -741,7 +815,7 @@ inline int lane_cols(const StreamArgs<FT, VT, OT>& a, uint64_t nnz, int R, const
     int E = 2;
     if (!F64) {
         const int narrow = k.narrow_max >= 0 ? k.narrow_max : BF16 ? 32 : 16;
-        if (R > narrow && !(k.narrow_small && nnz < (1ull << 20) && R <= 128)) E = 4;
+        if (R > narrow && !(k.narrow_small && nnz < (1ull << 17))) E = BF16 && R > 32 ? 8 : 4;
     }
     return R >= E ? E : R >= 2 ? 2 : 0;
 }
@@ -755,6 +829,9 @@ inline bool rows_aligned(const StreamArgs<FT, VT, OT>& a, int R, int bytes)
         if ((uintptr_t)a.Uo[o] % bytes != 0) return false;
     return true;
 }
+
+// the lane shapes in use (ranks up to 128; eight columns per lane above rank 32)
+constexpr bool lane_shape(int G, int E) { return G * E <= 128 && (E < 8 || G >= 8); }
 
 // lanes per nonzero with E columns per lane (R <= 128: at most 128 / E)
 inline int lanes_for(int R, int E)
@@ -803,7 +880,7 @@ int launch_fiber_tier(const alto_tensor* t, int mode, int fmode, uint64_t first,
     } while (0)
 #define KFG_(GG)                                   \
     do {                                           \
-        if constexpr (GG * E <= 128)               \
+        if constexpr (lane_shape(GG, E)) \
             if (G == GG) {                         \
                 if (t->pack.pw == 1) KFN_(GG, 1);  \
                 else KFN_(GG, 2);                  \
@@ -863,7 +940,7 @@ int launch_lanes(const alto_tensor* t, int mode, int R, const FT* const* U, Stre
 {
     const ModeStream& M = t->ms[mode];
     const int G = lanes_for(R, E);
-    if (seg <= 0) seg = lane_seg(t->nnz, G, E);
+    if (seg <= 0) seg = lane_seg(t->nnz, G);
     a.seg = (uint64_t)seg;
     const uint64_t nfib = M.nlong + M.nlong2;
     if (M.fib_mode >= 0 && nfib > 0 && a.nother >= 2) {
@@ -883,7 +960,7 @@ int launch_lanes(const alto_tensor* t, int mode, int R, const FT* const* U, Stre
     } while (0)
 #define KNG_(GG)                                     \
     do {                                             \
-        if constexpr (GG * E <= 128)                 \
+        if constexpr (lane_shape(GG, E))                 \
             if (G == GG) {                           \
                 if (t->pack.pw == 1) KN_(GG, 1);     \
                 else KN_(GG, 2);                     \
@@ -945,7 +1022,7 @@ int launch_split(const alto_tensor* t, int mode, int R, const StreamArgs<FT, VT,
     } while (0)
 #define K16_(GG)                                     \
     do {                                             \
-        if constexpr (GG * E <= 128)                 \
+        if constexpr (lane_shape(GG, E))                 \
             if (G == GG) {                           \
                 if (t->pack.pw == 1) K16N_(GG, 1);   \
                 else K16N_(GG, 2);                   \
@@ -995,6 +1072,8 @@ int launch_mttkrp(const alto_tensor* t, int mode, int R, const FT* const* U, con
         if (E == 2) return launch_lanes<FT, VT, AT, OT, 2>(t, mode, R, U, a, seg, s);
         if constexpr (E16 == 4)
             if (E == 4) return launch_lanes<FT, VT, AT, OT, 4>(t, mode, R, U, a, seg, s);
+        if constexpr (std::is_same<FT, bf16_t>::value)
+            if (E == 8) return launch_lanes<FT, VT, AT, OT, 8>(t, mode, R, U, a, seg, s);
         v = 0;
     }
     const int E = v == 1 ? 4 : 2;
@@ -1058,7 +1137,7 @@ inline void launch_batch_table(const BatchTable<FT, VT, OT>& tab, int G, int pw,
 {
 #define KB_(GG)                                                                                              \
     do {                                                                                                     \
-        if constexpr (GG * E <= 128) {                                                                       \
+        if constexpr (lane_shape(GG, E)) {                                                                       \
             if (pw == 1) hipLaunchKernelGGL((k_mttkrp16_batch<FT, VT, AT, OT, GG, E, 1>), grid, dim3(256), 0, s, tab); \
             else hipLaunchKernelGGL((k_mttkrp16_batch<FT, VT, AT, OT, GG, E, 2>), grid, dim3(256), 0, s, tab);    \
         }                                                                                                    \
@@ -1106,7 +1185,7 @@ int launch_mttkrp_batch(int n, alto_tensor* const* ts, const int* modes, int R, 
             ALTO_TRY((launch_mttkrp<FT, VT, AT, OT>(t, modes[i], R, U[i], vals[i], outs[i], seg, k, s)));
             continue;
         }
-        a.seg = (uint64_t)(seg > 0 ? seg : lane_seg(t->nnz, G, E));
+        a.seg = (uint64_t)(seg > 0 ? seg : lane_seg(t->nnz, G));
         (void)stream_grid(t->nnz, (int)a.seg, G, a);
         Group* g = nullptr;
         for (auto& x : groups)
@@ -1136,7 +1215,11 @@ int launch_mttkrp_batch(int n, alto_tensor* const* ts, const int* modes, int R, 
             }
             const dim3 grid((unsigned)((total + 7) / 8 * 8));
             if (g.E == 2) launch_batch_table<FT, VT, AT, OT, 2>(tab, g.G, g.pw, grid, s);
-            else if constexpr (E16 != 2) launch_batch_table<FT, VT, AT, OT, E16>(tab, g.G, g.pw, grid, s);
+            else if constexpr (E16 != 2) {
+                if (g.E == 4) launch_batch_table<FT, VT, AT, OT, 4>(tab, g.G, g.pw, grid, s);
+                else if constexpr (std::is_same<FT, bf16_t>::value)
+                    launch_batch_table<FT, VT, AT, OT, 8>(tab, g.G, g.pw, grid, s);
+            }
             HIP_TRY(hipGetLastError());
         }
     }

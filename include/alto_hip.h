@@ -160,13 +160,13 @@ int alto_coo_mttkrp(int nmodes, const uint64_t* dims, uint64_t nnz, const uint64
  * 32768).
  * ALTO_TUNE_NARROW_RANK: FP32 / BF16 ranks up to this value (0..128) use
  * two columns per lane in the vector-lane mapping (fewer lane groups per
- * wave, so fewer rounds of FP64 row flushes), above it four; by default 16
- * for FP32 and 32 for BF16.
+ * wave, so fewer rounds of FP64 row flushes), above it four (BF16 above rank
+ * 32: eight); by default 16 for FP32 and 32 for BF16.
  * ALTO_TUNE_PHI_VARIANT: CP-APR Phi kernel, 0 = runtime batch loop with LDS
  * permutes, 1 = compile-time batch with DPP broadcasts (default), 2 = 16-byte
  * lanes with the model row reloaded only where the row changes (even ranks
  * and 16-byte aligned factors; others take 1).
- * ALTO_TUNE_NARROW_SMALL: 1 (default) = below 1M nonzeros every FP32 / BF16
+ * ALTO_TUNE_NARROW_SMALL: 1 (default) = below 128K nonzeros every FP32 / BF16
  * rank uses two columns per lane.
  * ALTO_TUNE_FIBERS: 1 (default) = mode streams of tensors with at least
  * ALTO_TUNE_FIBER_MIN_NNZ nonzeros (default 4M) and 3+ modes are ordered by

@@ -114,3 +114,49 @@ def test_batched_odd_ranks(prec):
         for o, (cidx, vals), U in zip(got, co, Us):
             err = np.abs(o - mttkrp_numpy(cidx, vals, U, mode))
             assert (err <= _bound(A, prec, cidx, vals, U, mode)).all()
+
+
+@pytest.mark.parametrize("prec", [1, 2])
+@pytest.mark.parametrize("R", [34, 40, 64, 66, 128])
+def test_batched_wide_lanes(tune, R, prec):
+    """Four (FP32) and eight (BF16) columns per lane in the batched launch."""
+    A = _A()
+    tune(NARROW_RANK, 0)
+    tune(NARROW_SMALL, 0)
+    rng = np.random.default_rng(R)
+    ts, Us, co = [], [], []
+    for k, (dims, n) in enumerate([([30, 40, 50], 900), ([9, 300, 20, 7], 5000), ([64, 64, 64], 1)]):
+        cidx, vals = uniform_tensor(dims, n, k)
+        ts.append(A.AltoTensor(dims, cidx, vals))
+        co.append((cidx, vals))
+        U = [rng.random((d, R)).astype(np.float32).astype(np.float64) for d in dims]
+        Us.append([A.from_bf16_bits(A.to_bf16_bits(u)).astype(np.float64) for u in U] if prec == A.PREC_BF16 else U)
+    for mode in range(3):
+        got = A.mttkrp_batched(ts, [mode] * 3, Us, prec)
+        for o, (cidx, vals), U in zip(got, co, Us):
+            err = np.abs(o - mttkrp_numpy(cidx, vals, U, mode))
+            assert (err <= _bound(A, prec, cidx, vals, U, mode)).all()
+
+
+@pytest.mark.parametrize("prec", [0, 1, 2])
+def test_infinite_and_nan_entries_stay_where_they_are(tune, prec):
+    """Non-finite factor entries reach the rows of their own nonzeros and no
+    others: lanes past a segment's end read row 0 of every mode."""
+    A = _A()
+    tune(FIBER_MIN_NNZ, 0)
+    tune(NARROW_SMALL, 0)
+    dims, R = [50, 60, 40], 40
+    cidx, vals = zipf_tensor(dims, 4001, 2, s=1.1)
+    keep = (cidx[1] != 0) | (cidx[0] % 2 == 1)
+    cidx, vals = np.ascontiguousarray(cidx[:, keep]), vals[keep]
+    rng = np.random.default_rng(4)
+    U = [rng.integers(1, 9, (d, R)).astype(np.float64) for d in dims]
+    U[1][0, ::3] = np.inf
+    U[1][0, 1::3] = np.nan
+    for fibers in (0, 1):
+        tune(FIBERS, fibers)
+        got = A.AltoTensor(dims, cidx, vals).mttkrp(0, U, prec)
+        hit = np.zeros(dims[0], bool)
+        hit[cidx[0][cidx[1] == 0].astype(np.int64)] = True
+        assert np.isinf(got[hit][:, ::3]).all() and np.isnan(got[hit][:, 1::3]).all()
+        assert np.isfinite(got[~hit]).all() and np.isfinite(got[:, 2::3]).all()

@@ -116,7 +116,7 @@ static int cpd_alloc(alto_tensor* t, int R, CpdState<UT, ST, MT>& c)
     c.nb_solve = solve_blocks(maxrows_solve, R);
     ALTO_TRY(c.M.alloc(maxd * R * sizeof(MT)));
     ALTO_TRY(c.grams.alloc((size_t)t->nmode * R * R * 8));
-    ALTO_TRY(c.gpart.alloc((size_t)gram_blocks(maxd) * R * R * 8));
+    ALTO_TRY(c.gpart.alloc((size_t)mode_gram_blocks(maxd, R) * R * R * 8));
     ALTO_TRY(c.L.alloc((size_t)R * R * 8));
     ALTO_TRY(c.P.alloc((size_t)R * R * 8));
     ALTO_TRY(c.wsA.alloc((size_t)R * R * 8));
@@ -125,7 +125,7 @@ static int cpd_alloc(alto_tensor* t, int R, CpdState<UT, ST, MT>& c)
     ALTO_TRY(c.psum.alloc((size_t)c.nb_solve * R * 8));
     ALTO_TRY(c.pmax.alloc((size_t)c.nb_solve * R * 8));
     ALTO_TRY(c.pin.alloc((size_t)c.nb_solve * 8));
-    ALTO_TRY(c.pin_gram.alloc((size_t)gram_blocks(maxd) * 8));
+    ALTO_TRY(c.pin_gram.alloc((size_t)mode_gram_blocks(maxd, R) * 8));
     ALTO_TRY(c.lambda.alloc((size_t)R * 8));
     ALTO_TRY(c.ipart.alloc((size_t)64 * R * 8));
     ALTO_TRY(c.fitbuf.alloc(4 * 8));
@@ -222,7 +222,7 @@ template <typename UT, typename ST, typename MT>
 static int cpd_inner_parts(const alto_tensor* t, const CpdState<UT, ST, MT>& c)
 {
     const uint64_t rows = t->dims[c.N - 1];
-    return c.rounds ? gram_blocks(rows) : c.R <= 64 ? solve_blocks(rows, c.R) : c.nb_solve;
+    return c.rounds ? mode_gram_blocks(rows, c.R) : c.R <= 64 ? solve_blocks(rows, c.R) : c.nb_solve;
 }
 
 // whether mode j's update leaves its Gram in partials (in gpart) for the next
@@ -240,7 +240,7 @@ static PendingGram cpd_pending(const alto_tensor* t, const CpdState<UT, ST, MT>&
     if (cpd_defers(t, c, j)) {
         p.part = c.gpart.template as<double>();
         p.mode = j;
-        p.n = gram_blocks(t->dims[j]);
+        p.n = mode_gram_blocks(t->dims[j], c.R);
     }
     return p;
 }

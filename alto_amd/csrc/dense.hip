@@ -110,7 +110,7 @@ __device__ __forceinline__ void gram_rows_body(T* __restrict__ U, uint64_t I, in
 {
     constexpr int NP = T16 * (T16 + 1) / 2;
     using acc_t = typename std::conditional<F64, d4_t, f4_t>::type;
-    extern __shared__ double sG[];  // R x R
+    extern __shared__ double sG[];  // 2 x R x R
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r16 = lane & 15, kq = lane >> 4;
     acc_t acc[NP];
@@ -186,12 +186,11 @@ __device__ __forceinline__ void gram_rows_body(T* __restrict__ U, uint64_t I, in
         for (int o = 32; o > 0; o >>= 1) inacc += __shfl_xor(inacc, o);
         if (lane == 0) s_in[wave] = inacc;
     }
-    for (int k = threadIdx.x; k < R * R; k += blockDim.x) sG[k] = 0.0;
-    __syncthreads();
-    if constexpr (INNER)
-        if (Mi && threadIdx.x == 0) pin[bid] = (s_in[0] + s_in[1]) + (s_in[2] + s_in[3]);
-    for (int w = 0; w < 4; ++w) {
-        if (wave == w) {
+    // the four wavefronts' sums through two buffers: (0 + 2) + (1 + 3)
+#pragma unroll 1
+    for (int pass = 0; pass < 2; ++pass) {
+        if (wave >> 1 == pass) {
+            double* G = sG + (wave & 1) * R * R;
             int q = 0;
 #pragma unroll
             for (int ta = 0; ta < T16; ++ta)
@@ -203,17 +202,20 @@ __device__ __forceinline__ void gram_rows_body(T* __restrict__ U, uint64_t I, in
                         // v_mfma_f64_16x16x4f64: lane l, register v holds row l/16 + 4v;
                         // v_mfma_f32_16x16x4f32: row 4*(l/16) + v (both column l%16)
                         const int a = ta * 16 + (F64 ? kq + 4 * v : 4 * kq + v);
-                        if (a < R && b < R) sG[a * R + b] += (double)acc[q][v];
+                        if (a < R && b < R) G[a * R + b] = (pass ? G[a * R + b] : 0.0) + (double)acc[q][v];
                     }
                 }
         }
         __syncthreads();
     }
+    if constexpr (INNER)
+        if (Mi && threadIdx.x == 0) pin[bid] = (s_in[0] + s_in[1]) + (s_in[2] + s_in[3]);
     double* P = part + (size_t)bid * R * R;
     for (int k = threadIdx.x; k < R * R; k += blockDim.x) {
         const int a = k / R, b = k % R;
         // the upper block triangle holds the sums; mirror the lower one
-        P[k] = (a / 16 <= b / 16) ? sG[k] : sG[b * R + a];
+        const int e = a / 16 <= b / 16 ? k : b * R + a;
+        P[k] = sG[e] + sG[R * R + e];
     }
 }
 
@@ -295,6 +297,18 @@ int gram_blocks(uint64_t I)
     return b < 1 ? 1 : (int)b;
 }
 
+// blocks of a mode update's Gram launch: rank > 32 takes 64 rows per block up to
+// 128 blocks (a block of 256 rows walks them in 8 dependent steps and most CUs
+// have none: rank 64, modes of 150 to 20000 rows, with the sums in two buffers 25.1
+// -> 14.7 us)
+int mode_gram_blocks(uint64_t I, int R)
+{
+    const int b = gram_blocks(I);
+    if (R <= 32 || b >= 128) return b;
+    const uint64_t n = (I + 63) / 64;
+    return n < 128 ? (n < 1 ? 1 : (int)n) : 128;
+}
+
 template <typename T>
 int gram_device(const T* U, uint64_t I, int R, double* G, double* part, hipStream_t s, bool f64)
 {
@@ -305,7 +319,7 @@ int gram_device(const T* U, uint64_t I, int R, double* G, double* part, hipStrea
     int nb = gram_blocks(I);
     if (R <= 64) {
         const uint64_t rpb = ((I + nb - 1) / nb + 15) / 16 * 16;
-        const size_t lds = (size_t)R * R * 8;
+        const size_t lds = (size_t)R * R * 16;
     T* Uw = const_cast<T*>(U);  // read only without SCALE
 #define GR_(TT)                                                                                                  \
     do {                                                                                                         \
@@ -1485,7 +1499,7 @@ static int mode_gram(int n, const DenseModeJob* m, int R, bool f64, hipStream_t 
     gr.n = n;
     for (int k = 0; k < n; ++k) {
         const DenseModeJob& x = m[k];
-        const int gb = gram_blocks(x.I);
+        const int gb = mode_gram_blocks(x.I, R);
         const uint64_t rpb = ((x.I + gb - 1) / gb + 15) / 16 * 16;
         const bool fl = fuse_lambda(x.I, R);
         gr.a[k] = GramJob{x.U, same ? nullptr : x.S, x.lambda, x.gpart, x.Mgram, x.pin_gram, x.I, rpb,
@@ -1497,7 +1511,7 @@ static int mode_gram(int n, const DenseModeJob* m, int R, bool f64, hipStream_t 
         su.start[su.n + 1] = su.start[su.n] + (uint32_t)nsum + clear_blocks(x.zero_bytes);
         ++su.n;
     }
-    const size_t lds = (size_t)R * R * 8;
+    const size_t lds = (size_t)R * R * 16;
     // storage that rounds (BF16): the last modes' fit inner products from
     // the stored values, in the same launch
 #define GS_(TT)                                                                                                        \

@@ -7,6 +7,7 @@
 namespace alto {
 
 int gram_blocks(uint64_t I);
+int mode_gram_blocks(uint64_t I, int R);  // of a mode update (at least gram_blocks)
 template <typename T>
 int gram_device(const T* U, uint64_t I, int R, double* G, double* part, hipStream_t s, bool f64);
 int chol_device(const double* grams, int nmode, int mode, int R, double* L, double* P, double* wsA, double* wsQ,

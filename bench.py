@@ -140,9 +140,9 @@ def measure_traffic():
         mtt = [float(x["Counter_Value"]) for x in rows if "mttkrp" in x["Kernel_Name"]]
         if not copies or not mtt or len(mtt) % 3:
             return {"error": f"{counter}: {len(copies)} copy and {len(mtt)} MTTKRP dispatches"}
-        scale = (COPY_PROBE_BYTES / 1024.0) / copies[-1]
+        scale = (COPY_PROBE_BYTES / 1024.0) / copies[0]  # (building the tensor copies, too)
         last = mtt[-len(mtt) // 3:]  # the last all-mode pass
-        out[counter] = {"kib_last_pass": sum(last), "copy_kib": copies[-1], "scale": scale,
+        out[counter] = {"kib_last_pass": sum(last), "copy_kib": copies[0], "scale": scale,
                         "bytes_per_call": sum(last) * 1024.0 * scale / 3, "dispatches_per_pass": len(last)}
     rd, wr = out["FETCH_SIZE"]["bytes_per_call"], out["WRITE_SIZE"]["bytes_per_call"]
     return {"read_bytes_per_call": rd, "write_bytes_per_call": wr, "bytes_per_call": rd + wr,

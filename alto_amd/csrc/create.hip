@@ -1015,11 +1015,27 @@ static int chunk_bits(uint64_t n, int chunk_log2)
     return cb;
 }
 
-// Buffers shared by the orderings of a tensor's modes (all sized for nnz)
+// Buffers shared by the orderings of a tensor's modes (all sized for nnz; ck
+// and sort.keys, which change places in the sorts, both for the widest key)
 struct OrderSpace {
     DevBuf rec, ck, pay, cnt, nl, perm;
     SortSpace sort;
+    int hold_keys(uint64_t n, size_t key_bytes) const
+    {
+        if (ck.bytes >= n * key_bytes && pay.bytes >= n * 4) return ALTO_OK;
+        set_error("mode streams: %zu bytes for %llu sort keys of %zu", ck.bytes, (unsigned long long)n, key_bytes);
+        return ALTO_ERR_ARG;
+    }
 };
+
+// bits of the widest sort key of stream m in layout L
+static int stream_key_bits(const alto_tensor* t, int m, const StreamLayout& L)
+{
+    int a = 0;  // of the fiber mode's row
+    if (L.fib_mode >= 0) a = t->pack.bits[L.fib_mode];
+    if (L.fib_mode2 >= 0) a = std::max(a, t->pack.bits[L.fib_mode2]);
+    return chunk_bits(t->nnz, L.chunk_log2) + t->pack.bits[m] + a;
+}
 
 // One fiber split: the nonzeros at ALTO positions idx[0, n) (0..n-1 when
 // idx is null) ordered by (chunk, row_m, row_a) and split stably into the
@@ -1032,6 +1048,7 @@ static int fiber_split(alto_tensor* t, int m, int amode, int chunk_log2, int bit
                        uint64_t n, OrderSpace& w, uint32_t* nl_dev, uint32_t* perm, const StreamOut& o, hipStream_t s)
 {
     const uint64_t* rec = w.rec.as<uint64_t>();
+    ALTO_TRY(w.hold_keys(n, sizeof(K)));
     RANK_DISPATCH_PW(t->pack.pw, {
         hipLaunchKernelGGL((k_stream_key<K, PW>), dim3(grid_for(n)), dim3(256), 0, s, rec, t->pack, m, amode, chunk_log2,
                            n, idx, w.ck.as<K>(), w.pay.as<uint32_t>());
@@ -1094,6 +1111,7 @@ template <typename K>
 static int row_order(alto_tensor* t, int m, int chunk_log2, int bits, OrderSpace& w, const StreamOut& o, hipStream_t s)
 {
     const uint64_t n = t->nnz;
+    ALTO_TRY(w.hold_keys(n, sizeof(K)));
     RANK_DISPATCH_PW(t->pack.pw, {
         hipLaunchKernelGGL((k_stream_key<K, PW>), dim3(grid_for(n)), dim3(256), 0, s, w.rec.as<uint64_t>(), t->pack, m,
                            -1, chunk_log2, n, nullptr, w.ck.as<K>(), nullptr);
@@ -1144,11 +1162,16 @@ int prepare_mode_streams(alto_tensor* t, int need64, int need32, hipStream_t s)
             M.nlong = M.nlong2 = 0;
         }
     }
+    int key_bits = 0;
+    for (int m = 0; m < t->nmode; ++m) key_bits = std::max(key_bits, stream_key_bits(t, m, want[m]));
+    const size_t key_bytes = key_bits <= 32 ? 4 : 8;
     OrderSpace w;
     const Drain drain{s};  // before w goes back to the cache, whichever way out
     ALTO_TRY(w.rec.alloc(n * (t->pack.pw + 1) * 8));
-    ALTO_TRY(w.ck.alloc(n * 8));
+    ALTO_TRY(w.ck.alloc(n * key_bytes));
+    ALTO_TRY(w.sort.keys.alloc(n * key_bytes));
     ALTO_TRY(w.pay.alloc(n * 4));
+    ALTO_TRY(w.sort.pay.alloc(n * 4));
     ALTO_TRY(w.cnt.alloc((n + FS_TILE - 1) / FS_TILE * 4));
     ALTO_TRY(w.nl.alloc(ALTO_MAXN * 2 * 4));
     ALTO_TRY(fill_zero(w.nl.as<uint32_t>(), ALTO_MAXN * 2, s));

@@ -297,6 +297,13 @@ int sort_pairs(DevBuf& keys, DevBuf& pay, bool identity, uint64_t n, int bits, S
         set_error("radix sort supports fewer than 2^32 nonzeros");
         return ALTO_ERR_UNSUPPORTED;
     }
+    // (the passes swap the halves, so what a shared space holds depends on the
+    // sorts before this one)
+    if (keys.bytes < n * sizeof(K) || pay.bytes < n * 4) {
+        set_error("radix sort: %zu bytes of keys and %zu of positions for %llu pairs", keys.bytes, pay.bytes,
+                  (unsigned long long)n);
+        return ALTO_ERR_ARG;
+    }
     if (n <= 1 || bits <= 0) {
         if (identity && n) {
             hipLaunchKernelGGL(k_iota, dim3((unsigned)std::min<uint64_t>((n + 255) / 256, 4096)), dim3(256), 0, s,

@@ -12,15 +12,17 @@ struct alignas(16) Key128 {
 };
 
 // Work buffers of sort_pairs, reused from sort to sort on one stream.  Like
-// every DevBuf they must outlive the work that uses them.
+// every DevBuf they must outlive the work that uses them.  A sort may leave its
+// buffers swapped: sorts of several key types over one space need keys and
+// sp.keys both sized for the widest before the first.
 struct SortSpace {
     DevBuf keys, pay;   // the alternate halves of the double buffers
     DevBuf hist, total;
 };
 
 // Sorts n pairs by the low `bits` bits of the keys, stably and
-// asynchronously on s.  keys / pay are double-buffered with sp.keys /
-// sp.pay: on return `keys` and `pay` hold the result (the buffers may have
+// asynchronously on s.  keys / pay (refused where they are too small for n) are
+// double-buffered with sp.keys / sp.pay: on return `keys` and `pay` hold the result (the buffers may have
 // been swapped).  identity: pay is not read, the position of key i is i.
 template <typename K>
 int sort_pairs(DevBuf& keys, DevBuf& pay, bool identity, uint64_t n, int bits, SortSpace& sp, hipStream_t s);

@@ -164,6 +164,14 @@ alto_tensor::~alto_tensor()
 
 namespace alto {
 
+// Waits for a stream at the end of a scope, whichever way out: declared behind
+// the buffers that are released there and ahead of the first work that uses
+// them.
+struct Drain {
+    hipStream_t s;
+    ~Drain() { (void)hipStreamSynchronize(s); }
+};
+
 // ------------------------------------------------------------------ masks
 // setup_packed_alto(at, LSB_FIRST, SHORT_FIRST): modes ordered by bit count
 // (stable), one bit per still-active mode per level, LSB first.
@@ -231,7 +239,7 @@ int build_luts(alto_tensor* t, hipStream_t s)
                 }
             }
         ALTO_TRY(lut.dev.alloc(lut.host.size() * 8));
-        // (the table stays in `host`: no wait for the copy)
+        // (the table stays in `host`; the caller waits)
         HIP_TRY(hipMemcpyAsync(lut.dev.p, lut.host.data(), lut.host.size() * 8, hipMemcpyHostToDevice, s));
         return ALTO_OK;
     };
@@ -791,6 +799,7 @@ static int rank_streams(alto_tensor* t, hipStream_t s)
         const uint64_t d = t->dims[m];
         DevBuf cnt, keys, pay;
         SortSpace sp;
+        const Drain drain{s};
         ALTO_TRY(cnt.alloc(d * 4));
         ALTO_TRY(keys.alloc(d * 8));
         ALTO_TRY(pay.alloc(d * 4));
@@ -919,6 +928,7 @@ int split_stream(alto_tensor* t, int mode, const int* hot_k, hipStream_t s)
     for (int o = 0; o < ALTO_MAXN - 1; ++o) hk.k[o] = o < no ? hot_k[o] : 0;
     DevBuf ck, pay, cnt, pk2, v64, v32;
     SortSpace sp;
+    const Drain drain{s};
     ALTO_TRY(ck.alloc(n * 8));
     ALTO_TRY(pay.alloc(n * 4));
     ALTO_TRY(cnt.alloc(64 * 4));
@@ -999,13 +1009,6 @@ static StreamLayout wanted_layout(const alto_tensor* t, int m, int ranked)
     L.fib_min = fmin;
     return L;
 }
-
-// waits for a stream at the end of a scope: declared behind buffers that are
-// released there
-struct Drain {
-    hipStream_t s;
-    ~Drain() { (void)hipStreamSynchronize(s); }
-};
 
 static int chunk_bits(uint64_t n, int chunk_log2)
 {
@@ -1261,12 +1264,15 @@ static int create_impl(int nmode, const uint64_t* dims, uint64_t nnz, const uint
         set_error("alto_tensor_create: %d index bits exceed the %d-bit ALTO mask", total, lit_bits);
         return ALTO_ERR_ARG;
     }
+    // the tensor's own buffers (guard) and every temporary here are released
+    // only after the stream has drained: the allocator hands freed blocks to
+    // other streams
+    DevBuf dcoord[ALTO_MAXN], dvals, pay, bad, iv, lo, hi;
+    SortSpace sp;
+    const Drain drain{s};
     ALTO_TRY(build_luts(t, s));
 
-    // inputs to device (the staging buffers, like every temporary here, are
-    // released only after the stream has drained: the allocator hands freed
-    // blocks to other streams)
-    DevBuf dcoord[ALTO_MAXN], dvals;
+    // inputs to device
     CoordPtrs cp = {};
     const double* dv = vals;
     if (ptr_kind == ALTO_PTR_HOST) {
@@ -1284,9 +1290,6 @@ static int create_impl(int nmode, const uint64_t* dims, uint64_t nnz, const uint
 
     ALTO_TRY(t->key.alloc(nnz * t->W * 8));
     ALTO_TRY(t->vals.alloc(nnz * 8));
-    DevBuf pay, bad, iv;
-    SortSpace sp;
-    const Drain drain{s};
     ALTO_TRY(pay.alloc(nnz * 4));
     ALTO_TRY(bad.alloc(4));
     ALTO_TRY(fill_zero(bad.as<int>(), 1, s));
@@ -1349,7 +1352,6 @@ static int create_impl(int nmode, const uint64_t* dims, uint64_t nnz, const uint
         uint64_t cm0 = t->cr_masks[m * t->W], cm1 = t->W == 2 ? t->cr_masks[m * t->W + 1] : 0;
         // with one partition no row is shared, so no key gets the bit
         if (!(cm0 | cm1) || nprtn == 1) continue;
-        DevBuf lo, hi;
         ALTO_TRY(lo.alloc(dims[m] * 4));
         ALTO_TRY(hi.alloc(dims[m] * 4));
         hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(dims[m])), dim3(256), 0, s, lo.as<int>(), dims[m], nprtn);
@@ -1451,6 +1453,7 @@ int alto_tensor_export_oidx(const alto_tensor_t* t, int mode, uint64_t* oidx)
     uint64_t n = t->nnz;
     DevBuf ck, pay;
     SortSpace sp;
+    const Drain drain{nullptr};
     ALTO_TRY(ck.alloc(n * 8));
     ALTO_TRY(pay.alloc(n * 4));
     // a plain stable sort by row

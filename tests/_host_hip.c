@@ -19,8 +19,7 @@ typedef void (*launch_fn)(const char* name, uint32_t grid, uint32_t block, void*
 static launch_fn on_launch;
 static int mallocs, fail_from = -1; /* allocations so far; the first one that fails */
 static uint64_t live, limit = ~0ull; /* bytes allocated, and how many may be */
-static int in_flight;               /* operations nothing has waited for */
-static int released_in_flight;      /* hipFree calls that came before such a wait */
+static int in_flight;                /* operations nothing has waited for */
 
 void host_hip_on_launch(launch_fn f) { on_launch = f; }
 void host_hip_fail_from(int n) { fail_from = n < 0 ? -1 : mallocs + n; }
@@ -28,7 +27,6 @@ void host_hip_limit(uint64_t bytes) { limit = bytes; }
 uint64_t host_hip_live(void) { return live; }
 int host_hip_mallocs(void) { return mallocs; }
 int host_hip_in_flight(void) { return in_flight; }
-int host_hip_released_in_flight(void) { return released_in_flight; }
 
 enum { MAXBLOCKS = 4096 };
 static struct {
@@ -63,7 +61,6 @@ err_t hipMalloc(void** p, size_t n)
 }
 err_t hipFree(void* p)
 {
-    if (in_flight) ++released_in_flight;
     for (int i = 0; i < MAXBLOCKS; ++i)
         if (p && blocks[i].p == p) {
             munmap(p, blocks[i].n);

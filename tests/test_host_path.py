@@ -60,3 +60,55 @@ out.update(status=mttkrp(t, {dims}, 2), widths=sorted(widths), bad=bad[:4])
 ''')
     assert out["status"] == 0 and out["widths"] == [4, 8]
     assert not out["bad"]
+
+
+# out["runs"][k]: status of call() when its k-th allocation and all later ones
+# fail, and what it left in flight; up to the first k that it does not reach
+_FAILING = r'''
+def failing(setup, call):
+    runs = []
+    for k in range(64):
+        x = setup()
+        A.check(L.alto_device_synchronize(), "sync")
+        A.check(L.alto_device_trim(), "trim")
+        H.host_hip_fail_from(k)
+        status = call(x)
+        H.host_hip_fail_from(-1)
+        runs.append([status, H.host_hip_in_flight()])
+        after(x)
+        if status == 0:
+            return runs
+after = lambda x: None
+'''
+
+_CREATE = r'''
+idx = np.zeros((3, 4000), np.uint64)
+vals = np.ones(4000)
+def create(_):
+    h = C.c_void_p()
+    d = np.array([70, 50, 40], np.uint64)
+    st = L.alto_tensor_create(3, d.ctypes.data, 4000, A._ptr_array([r.ctypes.data for r in idx]), vals.ctypes.data,
+                              0, 0, 0, 4, None, C.byref(h))
+    if st == 0:
+        L.alto_tensor_destroy(h)
+    return st
+out["runs"] = failing(lambda: None, create)
+'''
+_STREAMS = r'''
+A.check(L.alto_tune_set(7, HOT), "hot rows")
+out["runs"] = failing(lambda: tensor([70, 50, 40], 200_000), lambda t: mttkrp(t, [1] * 3, 16))
+'''
+_OIDX = r'''
+o = np.zeros(200_000, np.uint64)
+out["runs"] = failing(lambda: tensor([70, 50, 40], 200_000), lambda t: L.alto_tensor_export_oidx(t.h, 1, o.ctypes.data))
+'''
+
+
+@pytest.mark.parametrize("body", [_CREATE, _STREAMS.replace("HOT", "0"), _STREAMS.replace("HOT", "1"), _OIDX],
+                         ids=["create", "streams", "hot rows", "oidx"])
+def test_nothing_in_flight_when_an_allocation_fails(host, body):
+    """A call that gives up hands its buffers back to the cache shared by all
+    streams, so nothing that it enqueued may still be running."""
+    runs = host(_FAILING + body)["runs"]
+    assert len(runs) > 3 and runs[-1][0] == 0
+    assert all(status != 0 and left == 0 for status, left in runs[:-1]), runs

@@ -797,14 +797,14 @@ static int rank_streams(alto_tensor* t, hipStream_t s)
     for (int m = 0; m < t->nmode; ++m) {
         if (t->rank_row[m].p) continue;
         const uint64_t d = t->dims[m];
-        DevBuf cnt, keys, pay;
+        DevBuf cnt, keys, pay, rank_row, row_rank;  // (the tensor gets the tables when they are written)
         SortSpace sp;
         const Drain drain{s};
         ALTO_TRY(cnt.alloc(d * 4));
         ALTO_TRY(keys.alloc(d * 8));
         ALTO_TRY(pay.alloc(d * 4));
-        ALTO_TRY(t->rank_row[m].alloc(d * 4));
-        ALTO_TRY(t->row_rank[m].alloc(d * 4));
+        ALTO_TRY(rank_row.alloc(d * 4));
+        ALTO_TRY(row_rank.alloc(d * 4));
         ALTO_TRY(fill_zero(cnt.as<uint32_t>(), d, s));
         RANK_DISPATCH_PW(t->pack.pw, {
             hipLaunchKernelGGL((k_row_counts<PW>), dim3(grid_for(n)), dim3(256), 0, s, t->ms[m].pk.as<uint64_t>(), n,
@@ -815,10 +815,11 @@ static int rank_streams(alto_tensor* t, hipStream_t s)
         HIP_TRY(hipGetLastError());
         ALTO_TRY(sort_pairs<uint64_t>(keys, pay, true, d, 32 + t->pack.bits[m], sp, s));
         hipLaunchKernelGGL(k_rank_scatter, dim3(grid_for(d)), dim3(256), 0, s, pay.as<uint32_t>(), d,
-                           t->rank_row[m].as<uint32_t>(), t->row_rank[m].as<uint32_t>());
+                           rank_row.as<uint32_t>(), row_rank.as<uint32_t>());
         HIP_TRY(hipGetLastError());
-        // the temporaries go back to the shared cache: drain first
         HIP_TRY(hipStreamSynchronize(s));
+        t->rank_row[m].swap(rank_row);
+        t->row_rank[m].swap(row_rank);
     }
     RankTabs T;
     for (int m = 0; m < ALTO_MAXN; ++m) T.row_rank[m] = m < t->nmode ? t->row_rank[m].as<uint32_t>() : nullptr;
@@ -1129,6 +1130,20 @@ static int row_order(alto_tensor* t, int m, int chunk_log2, int bits, OrderSpace
     return ALTO_OK;
 }
 
+// A stream that is being written: given up, and built anew by the next call,
+// when this one leaves before it is done
+struct StreamInWork {
+    ModeStream* M = nullptr;
+    ~StreamInWork()
+    {
+        if (!M) return;
+        M->pk.release();
+        M->val64.release();
+        M->val32.release();
+        M->chunk_log2 = -1;
+    }
+};
+
 int prepare_mode_streams(alto_tensor* t, int need64, int need32, hipStream_t s)
 {
     uint64_t n = t->nnz;
@@ -1168,8 +1183,9 @@ int prepare_mode_streams(alto_tensor* t, int need64, int need32, hipStream_t s)
     int key_bits = 0;
     for (int m = 0; m < t->nmode; ++m) key_bits = std::max(key_bits, stream_key_bits(t, m, want[m]));
     const size_t key_bytes = key_bits <= 32 ? 4 : 8;
+    StreamInWork work;
     OrderSpace w;
-    const Drain drain{s};  // before w goes back to the cache, whichever way out
+    const Drain drain{s};
     ALTO_TRY(w.rec.alloc(n * (t->pack.pw + 1) * 8));
     ALTO_TRY(w.ck.alloc(n * key_bytes));
     ALTO_TRY(w.sort.keys.alloc(n * key_bytes));
@@ -1192,6 +1208,7 @@ int prepare_mode_streams(alto_tensor* t, int need64, int need32, hipStream_t s)
         // the stream is rewritten in its base order: every value array it
         // has is rewritten with it
         const bool w64 = need64 || M.val64.p, w32 = need32 || M.val32.p;
+        work.M = &M;
         if (!M.pk.p) ALTO_TRY(M.pk.alloc(n * t->pack.pw * 8));
         if (w64 && !M.val64.p) ALTO_TRY(M.val64.alloc(n * 8));
         if (w32 && !M.val32.p) ALTO_TRY(M.val32.alloc(n * 4));
@@ -1210,6 +1227,7 @@ int prepare_mode_streams(alto_tensor* t, int need64, int need32, hipStream_t s)
         M.fib_mode2 = L.fib_mode2;
         M.fib_min = L.fib_min;
         M.nlong = M.nlong2 = 0;
+        work.M = nullptr;
     }
     if (fibers) {
         uint32_t nl[ALTO_MAXN * 2];

@@ -112,3 +112,45 @@ def test_nothing_in_flight_when_an_allocation_fails(host, body):
     runs = host(_FAILING + body)["runs"]
     assert len(runs) > 3 and runs[-1][0] == 0
     assert all(status != 0 and left == 0 for status, left in runs[:-1]), runs
+
+
+# values and rank tables that kernels read: each must have been written by a
+# kernel since the set-up
+_WRITTEN = r'''
+written, unwritten = set(), []
+def watch(x):
+    if "k_mode_gather" in x.name or "k_fiber_place" in x.name:
+        o = x.arg(3 if "k_mode_gather" in x.name else 9, C.c_uint64 * 3)
+        written.update(o[1:])
+    elif "k_rank_scatter" in x.name:
+        written.update((x.arg(2), x.arg(3)))
+    elif "k_permute_rows" in x.name and x.arg(1) not in written:
+        unwritten.append(x.name)
+    elif "k_mttkrp" in x.name and x.arg(0, C.c_uint64 * 2)[1] not in written:
+        unwritten.append(x.name)
+seen.append(watch)
+'''
+
+
+@pytest.mark.parametrize("hot", [0, 1])
+def test_a_failed_preparation_is_not_taken_for_a_finished_one(host, hot):
+    """FP32 streams of a tensor prepared for FP64 (and, with hot rows, its rank
+    tables): the call after a failed one builds what the failed one did not."""
+    runs = host(_FAILING + _WRITTEN + f'''
+dims = [70, 50, 40]
+def setup():
+    A.check(L.alto_tune_set(7, 0), "hot rows")
+    t = tensor(dims, 200_000)
+    A.check(mttkrp(t, dims, 16), "fp64")
+    A.check(L.alto_tune_set(7, {hot}), "hot rows")
+    written.clear()
+    return t
+def again(t):
+    for m in range(3):
+        A.check(mttkrp(t, dims, 16, m, A.PREC_F32), "fp32")
+after = again
+out["runs"] = failing(setup, lambda t: mttkrp(t, dims, 16, 0, A.PREC_F32))
+out["unwritten"] = unwritten
+''')
+    assert len(runs["runs"]) > 3
+    assert not runs["unwritten"]

@@ -576,20 +576,53 @@ __global__ void __launch_bounds__(256) k_records(const uint64_t* __restrict__ ke
     }
 }
 
+// Where the streams' nonzeros come from, by ALTO position: the records, or (when
+// the records' memory is not there) the keys and values themselves.
+template <int PW_>
+struct FromRecords {
+    static constexpr int PW = PW_;
+    const uint64_t* rec;
+    __device__ __forceinline__ void coords(uint64_t i, uint64_t (&pk)[PW]) const
+    {
+#pragma unroll
+        for (int w = 0; w < PW; ++w) pk[w] = rec[i * (PW + 1) + w];
+    }
+    __device__ __forceinline__ double value(uint64_t i) const
+    {
+        return __longlong_as_double((long long)rec[i * (PW + 1) + PW]);
+    }
+};
+template <int W, int PW_>
+struct FromKeys {
+    static constexpr int PW = PW_;
+    const uint64_t* keys;
+    const double* vals;
+    const uint64_t* lut;
+    int nb;
+    __device__ __forceinline__ void coords(uint64_t i, uint64_t (&pk)[PW]) const
+    {
+        uint64_t k[W];
+#pragma unroll
+        for (int w = 0; w < W; ++w) k[w] = keys[i * W + w];
+        lut_apply<W, PW>(lut, nb, k, pk);
+    }
+    __device__ __forceinline__ double value(uint64_t i) const { return vals[i]; }
+};
+
 // Sort key of a mode's stream: (chunk, row of `mode`, row of `amode`) of the
 // nonzero at ALTO position idx[j] (j itself when idx is null; the positions
 // are then left to the sort), without the last field when amode < 0.
-template <typename K, int PW>
-__global__ void __launch_bounds__(256) k_stream_key(const uint64_t* __restrict__ rec, PackLayout L, int mode, int amode,
-                                                    int chunk_log2, uint64_t n, const uint32_t* __restrict__ idx,
-                                                    K* __restrict__ ck, uint32_t* __restrict__ pay)
+template <typename K, typename S>
+__global__ void __launch_bounds__(256) k_stream_key(S from, PackLayout L, int mode, int amode, int chunk_log2,
+                                                    uint64_t n, const uint32_t* __restrict__ idx, K* __restrict__ ck,
+                                                    uint32_t* __restrict__ pay)
 {
+    constexpr int PW = S::PW;
     const int ba = amode >= 0 ? L.bits[amode] : 0, bn = L.bits[mode];
     for (uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += (uint64_t)gridDim.x * blockDim.x) {
         const uint64_t i = idx ? idx[j] : j;
         uint64_t pk[PW];
-#pragma unroll
-        for (int w = 0; w < PW; ++w) pk[w] = rec[i * (PW + 1) + w];
+        from.coords(i, pk);
         uint64_t k = ((i >> chunk_log2) << bn) | field<PW>(pk, L.off[mode], bn);
         if (amode >= 0) k = (k << ba) | field<PW>(pk, L.off[amode], ba);
         ck[j] = (K)k;
@@ -604,25 +637,24 @@ struct StreamOut {
     float* v32;
 };
 
-template <int PW>
-__device__ inline void put_nonzero(const uint64_t* __restrict__ rec, uint64_t src, uint64_t dst, const StreamOut& o)
+template <typename S>
+__device__ inline void put_nonzero(const S& from, uint64_t src, uint64_t dst, const StreamOut& o)
 {
-    uint64_t r[PW + 1];
+    constexpr int PW = S::PW;
+    uint64_t pk[PW];
+    from.coords(src, pk);
+    const double v = from.value(src);
 #pragma unroll
-    for (int w = 0; w <= PW; ++w) r[w] = rec[src * (PW + 1) + w];
-#pragma unroll
-    for (int w = 0; w < PW; ++w) o.pk[dst * PW + w] = r[w];
-    const double v = __longlong_as_double((long long)r[PW]);
+    for (int w = 0; w < PW; ++w) o.pk[dst * PW + w] = pk[w];
     if (o.v64) o.v64[dst] = v;
     if (o.v32) o.v32[dst] = (float)v;
 }
 
-template <int PW>
-__global__ void __launch_bounds__(256) k_mode_gather(const uint64_t* __restrict__ rec, const uint32_t* __restrict__ perm,
-                                                     uint64_t n, StreamOut o)
+template <typename S>
+__global__ void __launch_bounds__(256) k_mode_gather(S from, const uint32_t* __restrict__ perm, uint64_t n, StreamOut o)
 {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-        put_nonzero<PW>(rec, perm[i], i, o);
+        put_nonzero(from, perm[i], i, o);
 }
 
 // ------------------------------------------------------------------ fiber layout
@@ -665,11 +697,11 @@ __global__ void __launch_bounds__(256) k_fiber_count(const K* __restrict__ ck, u
     if (threadIdx.x == 0) cnt[blockIdx.x] = s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
 }
 
-template <typename K, int PW>
+template <typename K, typename S>
 __global__ void __launch_bounds__(256) k_fiber_place(const K* __restrict__ ck, const uint32_t* __restrict__ pay, uint64_t n,
                                                      uint32_t min_len, uint32_t top, const uint32_t* __restrict__ cnt,
                                                      const uint32_t* __restrict__ nlong, uint32_t* __restrict__ perm,
-                                                     const uint64_t* __restrict__ rec, StreamOut o)
+                                                     S from, StreamOut o)
 {
     __shared__ uint32_t s_cnt[FS_ROUNDS * 4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -700,7 +732,7 @@ __global__ void __launch_bounds__(256) k_fiber_place(const K* __restrict__ ck, c
             const uint64_t p = run + before + below[j];  // long nonzeros ahead of i
             const uint64_t dst = (in >> j) & 1 ? p : nl + (i - p);
             if (perm) perm[dst] = pay[i];
-            else put_nonzero<PW>(rec, pay[i], dst, o);
+            else put_nonzero(from, pay[i], dst, o);
         }
         run += sum;
     }
@@ -1032,6 +1064,21 @@ struct OrderSpace {
     }
 };
 
+// f(the source of the tensor's nonzeros)
+template <typename F>
+static void with_source(const alto_tensor* t, const OrderSpace& w, F&& f)
+{
+    if (w.rec.p) {
+        const uint64_t* rec = w.rec.as<uint64_t>();
+        if (t->pack.pw == 1) f(FromRecords<1>{rec});
+        else f(FromRecords<2>{rec});
+    } else {
+        DISPATCH_WPW(t->W, t->pack.pw, {
+            f((FromKeys<W, PW>{t->key.as<uint64_t>(), t->vals.as<double>(), t->delin.dev.as<uint64_t>(), t->delin.nb}));
+        });
+    }
+}
+
 // bits of the widest sort key of stream m in layout L
 static int stream_key_bits(const alto_tensor* t, int m, const StreamLayout& L)
 {
@@ -1051,11 +1098,10 @@ template <typename K>
 static int fiber_split(alto_tensor* t, int m, int amode, int chunk_log2, int bits, uint32_t min_len, const uint32_t* idx,
                        uint64_t n, OrderSpace& w, uint32_t* nl_dev, uint32_t* perm, const StreamOut& o, hipStream_t s)
 {
-    const uint64_t* rec = w.rec.as<uint64_t>();
     ALTO_TRY(w.hold_keys(n, sizeof(K)));
-    RANK_DISPATCH_PW(t->pack.pw, {
-        hipLaunchKernelGGL((k_stream_key<K, PW>), dim3(grid_for(n)), dim3(256), 0, s, rec, t->pack, m, amode, chunk_log2,
-                           n, idx, w.ck.as<K>(), w.pay.as<uint32_t>());
+    with_source(t, w, [&](auto from) {
+        hipLaunchKernelGGL((k_stream_key<K, decltype(from)>), dim3(grid_for(n)), dim3(256), 0, s, from, t->pack, m, amode,
+                           chunk_log2, n, idx, w.ck.as<K>(), w.pay.as<uint32_t>());
     });
     HIP_TRY(hipGetLastError());
     ALTO_TRY(sort_pairs<K>(w.ck, w.pay, idx == nullptr, n, bits, w.sort, s));
@@ -1066,9 +1112,9 @@ static int fiber_split(alto_tensor* t, int m, int amode, int chunk_log2, int bit
                        w.cnt.as<uint32_t>());
     HIP_TRY(hipGetLastError());
     ALTO_TRY(scan_rows(w.cnt.as<uint32_t>(), 1, nt, nl_dev, s));
-    RANK_DISPATCH_PW(t->pack.pw, {
-        hipLaunchKernelGGL((k_fiber_place<K, PW>), dim3((unsigned)nt), dim3(256), 0, s, w.ck.as<K>(),
-                           w.pay.as<uint32_t>(), n, min_len, top, w.cnt.as<uint32_t>(), nl_dev, perm, rec, o);
+    with_source(t, w, [&](auto from) {
+        hipLaunchKernelGGL((k_fiber_place<K, decltype(from)>), dim3((unsigned)nt), dim3(256), 0, s, w.ck.as<K>(),
+                           w.pay.as<uint32_t>(), n, min_len, top, w.cnt.as<uint32_t>(), nl_dev, perm, from, o);
     });
     HIP_TRY(hipGetLastError());
     return ALTO_OK;
@@ -1094,7 +1140,6 @@ static int fiber_order(alto_tensor* t, int m, const StreamLayout& L, OrderSpace&
     const uint64_t n = t->nnz;
     if (L.fib_mode2 < 0)
         return fiber_split_any(t, m, L.fib_mode, L.chunk_log2, (uint32_t)L.fib_min, nullptr, n, w, nl_dev, nullptr, o, s);
-    if (!w.perm.p) ALTO_TRY(w.perm.alloc(n * 4));
     uint32_t* perm = w.perm.as<uint32_t>();
     ALTO_TRY(fiber_split_any(t, m, L.fib_mode, L.chunk_log2, (uint32_t)L.fib_min, nullptr, n, w, nl_dev, perm, o, s));
     uint32_t nlong = 0;
@@ -1103,8 +1148,8 @@ static int fiber_order(alto_tensor* t, int m, const StreamLayout& L, OrderSpace&
     if (nlong < n)  // the short part [nlong, n) of perm holds the ALTO positions it orders
         ALTO_TRY(fiber_split_any(t, m, L.fib_mode2, L.chunk_log2, (uint32_t)L.fib_min, perm + nlong, n - nlong, w,
                                  nl_dev + 1, perm + nlong, o, s));
-    RANK_DISPATCH_PW(t->pack.pw, {
-        hipLaunchKernelGGL((k_mode_gather<PW>), dim3(grid_for(n)), dim3(256), 0, s, w.rec.as<uint64_t>(), perm, n, o);
+    with_source(t, w, [&](auto from) {
+        hipLaunchKernelGGL((k_mode_gather<decltype(from)>), dim3(grid_for(n)), dim3(256), 0, s, from, perm, n, o);
     });
     HIP_TRY(hipGetLastError());
     return ALTO_OK;
@@ -1116,41 +1161,134 @@ static int row_order(alto_tensor* t, int m, int chunk_log2, int bits, OrderSpace
 {
     const uint64_t n = t->nnz;
     ALTO_TRY(w.hold_keys(n, sizeof(K)));
-    RANK_DISPATCH_PW(t->pack.pw, {
-        hipLaunchKernelGGL((k_stream_key<K, PW>), dim3(grid_for(n)), dim3(256), 0, s, w.rec.as<uint64_t>(), t->pack, m,
-                           -1, chunk_log2, n, nullptr, w.ck.as<K>(), nullptr);
+    with_source(t, w, [&](auto from) {
+        hipLaunchKernelGGL((k_stream_key<K, decltype(from)>), dim3(grid_for(n)), dim3(256), 0, s, from, t->pack, m, -1,
+                           chunk_log2, n, nullptr, w.ck.as<K>(), nullptr);
     });
     HIP_TRY(hipGetLastError());
     ALTO_TRY(sort_pairs<K>(w.ck, w.pay, true, n, bits, w.sort, s));
-    RANK_DISPATCH_PW(t->pack.pw, {
-        hipLaunchKernelGGL((k_mode_gather<PW>), dim3(grid_for(n)), dim3(256), 0, s, w.rec.as<uint64_t>(),
+    with_source(t, w, [&](auto from) {
+        hipLaunchKernelGGL((k_mode_gather<decltype(from)>), dim3(grid_for(n)), dim3(256), 0, s, from,
                            w.pay.as<uint32_t>(), n, o);
     });
     HIP_TRY(hipGetLastError());
     return ALTO_OK;
 }
 
-// A stream that is being written: given up, and built anew by the next call,
-// when this one leaves before it is done
-struct StreamInWork {
-    ModeStream* M = nullptr;
-    ~StreamInWork()
+// What a call that leaves early takes back: the arrays that it allocated and did
+// not write, and whole streams that it was writing (bit m: stream m), so that the
+// next call builds them
+struct StreamsInWork {
+    alto_tensor* t;
+    int fresh64 = 0, fresh32 = 0, writing = 0;
+    ~StreamsInWork()
     {
-        if (!M) return;
-        M->pk.release();
-        M->val64.release();
-        M->val32.release();
-        M->chunk_log2 = -1;
+        for (int m = 0; m < t->nmode; ++m) {
+            ModeStream& M = t->ms[m];
+            if ((writing >> m) & 1) {
+                M.pk.release();
+                M.chunk_log2 = -1;
+            }
+            if (((writing | fresh64) >> m) & 1) M.val64.release();
+            if (((writing | fresh32) >> m) & 1) M.val32.release();
+        }
     }
 };
 
+// Writes every stream that lacks its coordinates or a value array, in the layout
+// want[m].  Beside the streams this takes, per nonzero, 24 bytes for the sorts
+// (16 where all keys have up to 32 bits, 4 more for a second fiber mode) and 16
+// or (two-word coordinates) 24 for the records; when those last do not fit, the
+// streams are gathered without records.  The streams' own arrays come first, so
+// that the records are what gives way.
+static int build_streams(alto_tensor* t, const StreamLayout* want, int need64, int need32, hipStream_t s)
+{
+    const uint64_t n = t->nnz;
+    StreamsInWork work{t};
+    OrderSpace w;
+    const Drain drain{s};
+    int modes = 0, key_bits = 0;
+    bool second = false;
+    for (int m = 0; m < t->nmode; ++m) {
+        ModeStream& M = t->ms[m];
+        if (M.pk.p && (!need64 || M.val64.p) && (!need32 || M.val32.p)) continue;
+        modes |= 1 << m;
+        if (!M.pk.p) {
+            work.writing |= 1 << m;
+            ALTO_TRY(M.pk.alloc(n * t->pack.pw * 8));
+        }
+        if (need64 && !M.val64.p) {
+            work.fresh64 |= 1 << m;
+            ALTO_TRY(M.val64.alloc(n * 8));
+        }
+        if (need32 && !M.val32.p) {
+            work.fresh32 |= 1 << m;
+            ALTO_TRY(M.val32.alloc(n * 4));
+        }
+        key_bits = std::max(key_bits, stream_key_bits(t, m, want[m]));
+        second = second || want[m].fib_mode2 >= 0;
+    }
+    const size_t key_bytes = key_bits <= 32 ? 4 : 8;
+    ALTO_TRY(w.ck.alloc(n * key_bytes));
+    ALTO_TRY(w.pay.alloc(n * 4));
+    ALTO_TRY(reserve_sort(n, key_bytes, w.sort));
+    if (second) ALTO_TRY(w.perm.alloc(n * 4));
+    ALTO_TRY(w.cnt.alloc((n + FS_TILE - 1) / FS_TILE * 4));
+    ALTO_TRY(w.nl.alloc(ALTO_MAXN * 2 * 4));
+    const int st = w.rec.alloc(n * (t->pack.pw + 1) * 8);
+    if (st != ALTO_OK && st != ALTO_ERR_OOM) return st;
+    ALTO_TRY(fill_zero(w.nl.as<uint32_t>(), ALTO_MAXN * 2, s));
+    if (w.rec.p)
+        DISPATCH_WPW(t->W, t->pack.pw, {
+            hipLaunchKernelGGL((k_records<W, PW>), dim3(grid_for(n)), dim3(256), lut_smem(t->delin), s,
+                               t->key.as<uint64_t>(), t->vals.as<double>(), lutref(t->delin), n, w.rec.as<uint64_t>());
+        });
+    HIP_TRY(hipGetLastError());
+    int fibers = 0;  // modes ordered by fibers here
+    for (int m = 0; m < t->nmode; ++m) {
+        if (!((modes >> m) & 1)) continue;
+        ModeStream& M = t->ms[m];
+        work.writing |= 1 << m;
+        M.ranked = 0;
+        M.split = 0;
+        M.pat_start.clear();
+        // the stream is rewritten in its base order: every value array it
+        // has is rewritten with it
+        const StreamOut o{M.pk.as<uint64_t>(), M.val64.as<double>(), M.val32.as<float>()};
+        const StreamLayout& L = want[m];
+        if (L.fib_mode >= 0) {
+            ALTO_TRY(fiber_order(t, m, L, w, w.nl.as<uint32_t>() + 2 * m, o, s));
+            fibers |= 1 << m;
+        } else {
+            const int bits = stream_key_bits(t, m, L);
+            if (bits <= 32) ALTO_TRY(row_order<uint32_t>(t, m, L.chunk_log2, bits, w, o, s));
+            else ALTO_TRY(row_order<uint64_t>(t, m, L.chunk_log2, bits, w, o, s));
+        }
+        M.chunk_log2 = L.chunk_log2;
+        M.fib_mode = L.fib_mode;
+        M.fib_mode2 = L.fib_mode2;
+        M.fib_min = L.fib_min;
+        M.nlong = M.nlong2 = 0;
+    }
+    if (fibers) {
+        uint32_t nl[ALTO_MAXN * 2];
+        HIP_TRY(hipMemcpyAsync(nl, w.nl.p, sizeof nl, hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        for (int m = 0; m < t->nmode; ++m)
+            if ((fibers >> m) & 1) {
+                t->ms[m].nlong = nl[2 * m];
+                t->ms[m].nlong2 = nl[2 * m + 1];
+            }
+    }
+    work.fresh64 = work.fresh32 = work.writing = 0;
+    return ALTO_OK;
+}
+
 int prepare_mode_streams(alto_tensor* t, int need64, int need32, hipStream_t s)
 {
-    uint64_t n = t->nnz;
     const int want_chunk = tuned_chunk_log2();
     if (want_chunk > 0 && want_chunk != t->chunk_log2) t->chunk_log2 = want_chunk;
     const int ranked = det_enabled() ? 0 : (int)rank_applicable(t);
-    int fibers = 0;  // modes ordered by fibers here
     StreamLayout want[ALTO_MAXN];
     bool any = false, reorder = false;
     for (int m = 0; m < t->nmode; ++m) {
@@ -1180,65 +1318,7 @@ int prepare_mode_streams(alto_tensor* t, int need64, int need32, hipStream_t s)
             M.nlong = M.nlong2 = 0;
         }
     }
-    int key_bits = 0;
-    for (int m = 0; m < t->nmode; ++m) key_bits = std::max(key_bits, stream_key_bits(t, m, want[m]));
-    const size_t key_bytes = key_bits <= 32 ? 4 : 8;
-    StreamInWork work;
-    OrderSpace w;
-    const Drain drain{s};
-    ALTO_TRY(w.rec.alloc(n * (t->pack.pw + 1) * 8));
-    ALTO_TRY(w.ck.alloc(n * key_bytes));
-    ALTO_TRY(w.sort.keys.alloc(n * key_bytes));
-    ALTO_TRY(w.pay.alloc(n * 4));
-    ALTO_TRY(w.sort.pay.alloc(n * 4));
-    ALTO_TRY(w.cnt.alloc((n + FS_TILE - 1) / FS_TILE * 4));
-    ALTO_TRY(w.nl.alloc(ALTO_MAXN * 2 * 4));
-    ALTO_TRY(fill_zero(w.nl.as<uint32_t>(), ALTO_MAXN * 2, s));
-    DISPATCH_WPW(t->W, t->pack.pw, {
-        hipLaunchKernelGGL((k_records<W, PW>), dim3(grid_for(n)), dim3(256), lut_smem(t->delin), s,
-                           t->key.as<uint64_t>(), t->vals.as<double>(), lutref(t->delin), n, w.rec.as<uint64_t>());
-    });
-    HIP_TRY(hipGetLastError());
-    for (int m = 0; m < t->nmode; ++m) {
-        ModeStream& M = t->ms[m];
-        if (M.pk.p && (!need64 || M.val64.p) && (!need32 || M.val32.p)) continue;
-        M.ranked = 0;
-        M.split = 0;
-        M.pat_start.clear();
-        // the stream is rewritten in its base order: every value array it
-        // has is rewritten with it
-        const bool w64 = need64 || M.val64.p, w32 = need32 || M.val32.p;
-        work.M = &M;
-        if (!M.pk.p) ALTO_TRY(M.pk.alloc(n * t->pack.pw * 8));
-        if (w64 && !M.val64.p) ALTO_TRY(M.val64.alloc(n * 8));
-        if (w32 && !M.val32.p) ALTO_TRY(M.val32.alloc(n * 4));
-        const StreamOut o{M.pk.as<uint64_t>(), w64 ? M.val64.as<double>() : nullptr, w32 ? M.val32.as<float>() : nullptr};
-        const StreamLayout& L = want[m];
-        if (L.fib_mode >= 0) {
-            ALTO_TRY(fiber_order(t, m, L, w, w.nl.as<uint32_t>() + 2 * m, o, s));
-            fibers |= 1 << m;
-        } else {
-            const int bits = t->pack.bits[m] + chunk_bits(n, L.chunk_log2);
-            if (bits <= 32) ALTO_TRY(row_order<uint32_t>(t, m, L.chunk_log2, bits, w, o, s));
-            else ALTO_TRY(row_order<uint64_t>(t, m, L.chunk_log2, bits, w, o, s));
-        }
-        M.chunk_log2 = L.chunk_log2;
-        M.fib_mode = L.fib_mode;
-        M.fib_mode2 = L.fib_mode2;
-        M.fib_min = L.fib_min;
-        M.nlong = M.nlong2 = 0;
-        work.M = nullptr;
-    }
-    if (fibers) {
-        uint32_t nl[ALTO_MAXN * 2];
-        HIP_TRY(hipMemcpyAsync(nl, w.nl.p, sizeof nl, hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
-        for (int m = 0; m < t->nmode; ++m)
-            if ((fibers >> m) & 1) {
-                t->ms[m].nlong = nl[2 * m];
-                t->ms[m].nlong2 = nl[2 * m + 1];
-            }
-    }
+    ALTO_TRY(build_streams(t, want, need64, need32, s));
     if (rank_applicable(t)) ALTO_TRY(rank_streams(t, s));
     HIP_TRY(hipStreamSynchronize(s));
     return ALTO_OK;

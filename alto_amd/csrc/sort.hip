@@ -286,6 +286,20 @@ int scan_rows(uint32_t* a, uint64_t rows, uint64_t m, uint32_t* total, hipStream
     return ALTO_OK;
 }
 
+// small inputs: shorter tiles, so that more workgroups share them
+constexpr uint64_t SMALL = 1ull << 20;
+
+int reserve_sort(uint64_t n, size_t key_bytes, SortSpace& sp)
+{
+    // (a part of n pairs may be a small input with more tiles than all of them)
+    const uint64_t tiles = std::max((std::min(n, SMALL) + RS_THREADS * 4 - 1) / (RS_THREADS * 4),
+                                    (n + RS_THREADS * 16 - 1) / (RS_THREADS * 16));
+    ALTO_TRY(sp.keys.alloc(n * key_bytes));
+    ALTO_TRY(sp.pay.alloc(n * 4));
+    ALTO_TRY(sp.hist.alloc(256 * tiles * 4));
+    return sp.total.alloc(256 * 4);
+}
+
 template <typename K>
 int sort_pairs(DevBuf& keys, DevBuf& pay, bool identity, uint64_t n, int bits, SortSpace& sp, hipStream_t s)
 {
@@ -314,9 +328,8 @@ int sort_pairs(DevBuf& keys, DevBuf& pay, bool identity, uint64_t n, int bits, S
     }
     ALTO_TRY(grow(sp.keys, n * sizeof(K), s));
     ALTO_TRY(grow(sp.pay, n * 4, s));
-    // small inputs: shorter tiles, so that more workgroups share them
-    return n < (1ull << 20) ? sort_passes<K, 4>(keys, pay, identity, n, bits, sp, s)
-                            : sort_passes<K, 16>(keys, pay, identity, n, bits, sp, s);
+    return n < SMALL ? sort_passes<K, 4>(keys, pay, identity, n, bits, sp, s)
+                     : sort_passes<K, 16>(keys, pay, identity, n, bits, sp, s);
 }
 template int sort_pairs<uint32_t>(DevBuf&, DevBuf&, bool, uint64_t, int, SortSpace&, hipStream_t);
 template int sort_pairs<uint64_t>(DevBuf&, DevBuf&, bool, uint64_t, int, SortSpace&, hipStream_t);

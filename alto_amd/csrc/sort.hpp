@@ -20,6 +20,10 @@ struct SortSpace {
     DevBuf hist, total;
 };
 
+// sizes the (unused) work buffers for up to n pairs with keys of key_bytes, so
+// that the sorts allocate nothing
+int reserve_sort(uint64_t n, size_t key_bytes, SortSpace& sp);
+
 // Sorts n pairs by the low `bits` bits of the keys, stably and
 // asynchronously on s.  keys / pay (refused where they are too small for n) are
 // double-buffered with sp.keys / sp.pay: on return `keys` and `pay` hold the result (the buffers may have

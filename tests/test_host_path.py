@@ -154,3 +154,30 @@ out["unwritten"] = unwritten
 ''')
     assert len(runs["runs"]) > 3
     assert not runs["unwritten"]
+
+
+@pytest.mark.parametrize("dims,bits,per", [
+    ([4000, 3000], 64, 24), ([4000, 1 << 30], 128, 24),
+    # fibers; the last one's coordinates take two words
+    ([4000, 3000, 5000], 64, 24), ([1 << 30, 1 << 30, 1 << 30], 128, 24),
+], ids=str)
+def test_streams_need_no_room_for_records(host, dims, bits, per):
+    """A preparation in memory that holds the streams and 24 bytes per nonzero
+    succeeds, and takes the records up where there is room for them too."""
+    n = 1 << 22  # (allocations are powers of two)
+    words = 2 if sum((d - 1).bit_length() for d in dims) > 64 else 1
+    out = host(_BOUNDS + _WRITTEN + f'''
+records = []
+seen.append(lambda x: records.append(x.name) if "k_records" in x.name else None)
+t = tensor({dims}, {n}, lit_bits={bits})
+A.check(L.alto_device_trim(), "trim")
+stream = {len(dims)} * ({words} * 8 + 8) * {n}
+H.host_hip_limit(H.host_hip_live() + stream + {per} * {n} + (8 << 20))
+out["scarce"] = [mttkrp(t, {dims}, 2), len(records)]
+H.host_hip_limit(1 << 60)
+t = tensor({dims}, {n}, lit_bits={bits})
+out["ample"] = [mttkrp(t, {dims}, 2), len(records)]
+out["bad"] = bad
+''')
+    assert out["scarce"] == [0, 0] and not out["bad"]
+    assert out["ample"] == [0, 1]

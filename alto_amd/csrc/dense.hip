@@ -440,7 +440,10 @@ int gram_noalloc(const void* U, uint64_t dim, int R, int precision, double* gram
 // everything (the buffer's previous readers have passed the barrier of step k)
 // and the division is done by one wavefront, not by all.  Rank 64: 54 -> 31 us
 // (0.48 us a step).
-__device__ __attribute__((noinline)) void pinv_body(int R, double* A, double* Q, double* Pout);
+typedef __attribute__((address_space(1))) double* global_f64;
+typedef __attribute__((address_space(3))) double* lds_f64;
+template <typename P>
+__device__ __forceinline__ void pinv_body(int R, P __restrict__ A, P __restrict__ Q, P __restrict__ Pout);
 
 __device__ __forceinline__ double lane_value(double v, int l)
 {
@@ -609,7 +612,7 @@ __device__ __forceinline__ void spd_inverse_body(const double* __restrict__ gram
             const int i = k / R, c = k % R;
             wsA[k] = gram_product(grams, nmode, mode, R, max(i, c), min(i, c));
         }
-        pinv_body(R, wsA, wsQ, W);
+        pinv_body(R, (global_f64)wsA, (global_f64)wsQ, (global_f64)W);
     }
 }
 
@@ -623,12 +626,13 @@ __global__ void __launch_bounds__(BT) k_spd_inverse(const double* __restrict__ g
 
 // Minimum-norm pseudo-inverse V^+ = Q diag(1/e) Q^T over |e| > R*eps*max|e|
 // (parallel cyclic Jacobi; runs only after a failed Cholesky).  A holds V and
-// is overwritten; A, Q and Pout (R x R, global memory or LDS) are shared
-// through work-group barriers.
-__device__ __attribute__((noinline)) void pinv_body(int R, double* A, double* Q, double* Pout)
+// is overwritten; A, Q and Pout (R x R, global memory or LDS; apart from each
+// other) are shared through work-group barriers.
+template <typename P>
+__device__ __forceinline__ void pinv_body(int R, P __restrict__ A, P __restrict__ Q, P __restrict__ Pout)
 {
     const int tid = threadIdx.x;
-    __shared__ double s_red[1024];
+    __shared__ double s_red[2][1024];
     __shared__ double s_c[64], s_s[64];
     __shared__ int s_p[64], s_q[64];
     __shared__ int s_stop;
@@ -652,28 +656,40 @@ __device__ __attribute__((noinline)) void pinv_body(int R, double* A, double* Q,
             tot += v;
             if (k / R != k % R) off += v;
         }
-        s_red[tid] = off;
+        s_red[0][tid] = off;
+        s_red[1][tid] = tot;
         __syncthreads();
-        for (int o = (int)blockDim.x / 2; o > 0; o >>= 1) {
-            if (tid < o) s_red[tid] += s_red[tid + o];
+        for (int o = (int)blockDim.x / 2; o >= 64; o >>= 1) {
+            if (tid < o) {
+                s_red[0][tid] += s_red[0][tid + o];
+                s_red[1][tid] += s_red[1][tid + o];
+            }
             __syncthreads();
         }
-        const double offs = s_red[0];
-        __syncthreads();
-        s_red[tid] = tot;
-        __syncthreads();
-        for (int o = (int)blockDim.x / 2; o > 0; o >>= 1) {
-            if (tid < o) s_red[tid] += s_red[tid + o];
-            __syncthreads();
+        if (tid < 64) {
+            off = s_red[0][tid];
+            tot = s_red[1][tid];
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) {
+                off += __shfl_down(off, o);
+                tot += __shfl_down(tot, o);
+            }
+            if (tid == 0) s_stop = off <= 1e-30 * tot || off == 0.0;
         }
-        if (tid == 0) s_stop = (offs <= 1e-30 * s_red[0]) || offs == 0.0;
         __syncthreads();
         if (s_stop) break;
         // one sweep in Rp - 1 steps of Rp / 2 disjoint rotations (round-robin
         // pairing: index Rp - 1 stays, the others circulate, so every pair
         // meets once per sweep; with R odd, index R is a dummy).  A step
         // computes all its rotations from the same A, then applies
-        // A <- A J, Q <- Q J and A <- J^T A, each in parallel.
+        // A <- J^T (A J) and Q <- Q J.  The four entries of A where the rows
+        // of one pair meet the columns of another change among themselves, so
+        // a thread takes such a block through both products and the step has
+        // two barriers.  A call with a failing pivot, against one product after
+        // the other behind three barriers in a function that is not inlined:
+        // rank 32 109 against 128 us, rank 64 423 against 650, rank 128 2.77
+        // against 4.46 ms; a CP-ALS iteration of equal columns, rank 32, three
+        // modes of 16000 rows, 480 against 585 us.
         const int Rp = R + (R & 1);
         for (int t = 0; t < Rp - 1; ++t) {
             for (int k = tid; k < Rp / 2; k += blockDim.x) {
@@ -696,28 +712,43 @@ __device__ __attribute__((noinline)) void pinv_body(int R, double* A, double* Q,
                 s_s[k] = sn;
             }
             __syncthreads();
-            for (int w = tid; w < (Rp / 2) * R; w += blockDim.x) {  // columns p, q of A and Q
+            const int half = Rp / 2;
+            for (int w = tid; w < half * half; w += blockDim.x) {  // rows of pair k, columns of pair l
+                const int k = w / half, l = w % half;
+                const double sr = s_s[k], sc = s_s[l];
+                if (sr == 0.0 && sc == 0.0) continue;
+                const double cr = s_c[k], cc = s_c[l];
+                const int p = s_p[k], q = s_q[k], u = s_p[l], v = s_q[l];
+                const bool hq = q < R, hv = v < R;
+                double pu = A[p * R + u], pv = hv ? A[p * R + v] : 0.0;
+                double qu = hq ? A[q * R + u] : 0.0, qv = hq && hv ? A[q * R + v] : 0.0;
+                if (sc != 0.0) {
+                    const double x = cc * pu - sc * pv, y = cc * qu - sc * qv;
+                    pv = sc * pu + cc * pv;
+                    qv = sc * qu + cc * qv;
+                    pu = x;
+                    qu = y;
+                }
+                if (sr != 0.0) {
+                    const double x = cr * pu - sr * qu, y = cr * pv - sr * qv;
+                    qu = sr * pu + cr * qu;
+                    qv = sr * pv + cr * qv;
+                    pu = x;
+                    pv = y;
+                }
+                A[p * R + u] = pu;
+                if (hv) A[p * R + v] = pv;
+                if (hq) A[q * R + u] = qu;
+                if (hq && hv) A[q * R + v] = qv;
+            }
+            for (int w = tid; w < half * R; w += blockDim.x) {  // columns of Q
                 const int k = w / R, r = w % R;
                 const double c = s_c[k], sn = s_s[k];
                 if (sn != 0.0) {
                     const int p = s_p[k], q = s_q[k];
-                    const double arp = A[r * R + p], arq = A[r * R + q];
-                    A[r * R + p] = c * arp - sn * arq;
-                    A[r * R + q] = sn * arp + c * arq;
                     const double qrp = Q[r * R + p], qrq = Q[r * R + q];
                     Q[r * R + p] = c * qrp - sn * qrq;
                     Q[r * R + q] = sn * qrp + c * qrq;
-                }
-            }
-            __syncthreads();
-            for (int w = tid; w < (Rp / 2) * R; w += blockDim.x) {  // rows p, q of A
-                const int k = w / R, r = w % R;
-                const double c = s_c[k], sn = s_s[k];
-                if (sn != 0.0) {
-                    const int p = s_p[k], q = s_q[k];
-                    const double apr = A[p * R + r], aqr = A[q * R + r];
-                    A[p * R + r] = c * apr - sn * aqr;
-                    A[q * R + r] = sn * apr + c * aqr;
                 }
             }
             __syncthreads();
@@ -1327,7 +1358,7 @@ __global__ void __launch_bounds__(256) k_solve_batch(BatchTab<SolveJob, N> t, in
                 s_p[e] = s_v[max(i, c) * R + min(i, c)];
             }
             __syncthreads();
-            pinv_body(R, s_p, s_q, s_v);
+            pinv_body(R, (lds_f64)s_p, (lds_f64)s_q, (lds_f64)s_v);
             __syncthreads();
             for (int e = threadIdx.x; e < R * R; e += 256) sW[(e / R) * WS + e % R] = (T)s_v[e];
         }

@@ -3,6 +3,8 @@ change: the inverse per rank class, row solves that invert V themselves (up to
 rank 16 and 32768 rows, rank 32 and 16384), lambda taken in the Gram launch (64
 rows x rank up to 2048 x 64) and Grams left in partials (256-row blocks x rank^2
 up to 2048)."""
+import ctypes
+
 import numpy as np
 import pytest
 import scipy.linalg
@@ -103,3 +105,23 @@ def test_mode_updates_reduced_precision(prec, tol, R, rows):
     Uo, lo = oracle.random_init(dims, R, 3)
     _, fo = o.cpd_als(Uo, lo, 4, 0.0)
     assert abs(fits[-1] - fo[-1]) <= tol * max(1.0, abs(fo[-1]))
+
+
+@pytest.mark.parametrize("R", [2, 3, 7, 16, 17, 31, 32, 33, 64, 65, 101, 127, 128])
+def test_pseudo_inverse_of_half_rank(R):
+    """V of rank about R / 2 with a zero row (its pivot is exactly zero), so that
+    the rotations sweep many times, against LAPACK's minimum-norm solution."""
+    A = _A()
+    rng = np.random.default_rng(R)
+    B = rng.random((R, (R + 1) // 2)) - 0.3
+    B[R // 2] = 0
+    V = B @ B.T
+    M = rng.random((50, R))
+    g, d = A.DeviceArray.from_numpy(np.stack([np.eye(R), V])), A.DeviceArray.from_numpy(M)
+    fb = ctypes.c_int(0)
+    A.check(A.lib().alto_pseudo_inverse(g.ptr, 2, 0, R, d.ptr, 50, ctypes.byref(fb), None), "pinv")
+    e = np.linalg.eigvalsh(V)
+    e = e[e > 1e-10 * e[-1]]
+    want = M @ np.linalg.pinv(V, rcond=1e-10, hermitian=True)
+    assert fb.value == 1
+    np.testing.assert_allclose(d.numpy(), want, rtol=0, atol=64 * R * EPS * e[-1] / e[0] * np.abs(want).max())

@@ -267,7 +267,7 @@ int alto_tune_set(int param, int value)
     if (param == ALTO_TUNE_SEG) return set_seg(value);
     if (param == ALTO_TUNE_CHUNK_LOG2) return set_chunk(value);
     if (param == ALTO_TUNE_NARROW_RANK) {
-        if (value < 0 || value > 128) return ALTO_ERR_ARG;
+        if (value < -1 || value > 128) return ALTO_ERR_ARG;
         g_narrow_max = value;
         return ALTO_OK;
     }

@@ -161,7 +161,7 @@ int alto_coo_mttkrp(int nmodes, const uint64_t* dims, uint64_t nnz, const uint64
  * ALTO_TUNE_NARROW_RANK: FP32 / BF16 ranks up to this value (0..128) use
  * two columns per lane in the vector-lane mapping (fewer lane groups per
  * wave, so fewer rounds of FP64 row flushes), above it four (BF16 above rank
- * 32: eight); by default 16 for FP32 and 32 for BF16.
+ * 32: eight); -1 (default) = 16 for FP32 and 32 for BF16.
  * ALTO_TUNE_PHI_VARIANT: CP-APR Phi kernel, 0 = runtime batch loop with LDS
  * permutes, 1 = compile-time batch with DPP broadcasts (default), 2 = 16-byte
  * lanes with the model row reloaded only where the row changes (even ranks

@@ -181,3 +181,22 @@ out["bad"] = bad
 ''')
     assert out["scarce"] == [0, 0] and not out["bad"]
     assert out["ample"] == [0, 1]
+
+
+def test_narrow_rank_goes_back_to_its_default(host):
+    """ALTO_TUNE_NARROW_RANK: -1 restores the rule per element type."""
+    out = host(r'''
+dims, lanes = [300, 200, 100], []
+seen.append(lambda x: lanes.append(x.name) if "k_mttkrp" in x.name else None)
+t = tensor(dims, 500_000)
+for value in (None, 64, -1):
+    if value is not None:
+        A.check(L.alto_tune_set(10, value), "narrow rank")
+    for prec in (A.PREC_F32, A.PREC_BF16):
+        for R in (16, 24, 32, 64):
+            A.check(mttkrp(t, dims, R, 0, prec), "mttkrp")
+out["lanes"], out["refused"] = lanes, [L.alto_tune_set(10, v) for v in (-2, 129)]
+''')
+    shipped, narrow, restored = out["lanes"][:8], out["lanes"][8:16], out["lanes"][16:]
+    assert len(out["lanes"]) == 24 and shipped == restored != narrow
+    assert all(v != 0 for v in out["refused"])

@@ -256,6 +256,24 @@ int mttkrp_device(alto_tensor* t, int mode, int R, const void* const* U, void* o
     return mttkrp_device_shape(t, mode, R, U, out, precision, accumulate, s, seg, -2);
 }
 
+// the segment length that lane mapping v takes by itself for this tensor and mode
+template <typename FT, typename VT>
+static int own_seg(const alto_tensor* t, int mode, int R, const void* const* U, int v)
+{
+    if (v == 2) {
+        StreamArgs<FT, VT, double> a;
+        fill_stream_args(t, mode, R, 0, a);
+        for (int m = 0; m < t->nmode; ++m)
+            if (m != mode) a.Uo[a.nother++] = (const FT*)U[m];
+        MttkrpTune k;
+        k.narrow_max = g_narrow_max;
+        k.narrow_small = g_narrow_small;
+        int G = 0, E = 0;
+        if (vector_lane_shape(t, mode, R, a, k, G, E)) return lane_seg(t->nnz, G);
+    }
+    return tuned_seg(t->nnz, group_lanes(R), (int)sizeof(VT));  // (32-bit values are summed in 32 bits)
+}
+
 }  // namespace alto
 
 using namespace alto;
@@ -406,10 +424,12 @@ int alto_mttkrp_autotune(alto_tensor_t* t, uint64_t rank, int precision, const v
         st = time_cfg(mode, -2, 0, &def_ms);
         int bv = -1, bs = 0;
         best_ms = def_ms;
-        // segment lengths within 4x of the size rule's choice (the others
-        // measured slower on every tensor tried, up to 10x on large ones)
-        const int h = lane_seg(t->nnz, group_lanes(R));
-        for (int v : variants)
+        // segment lengths within 4x of what the mapping takes by itself (the
+        // others measured slower on every tensor tried, up to 10x on large ones)
+        for (int v : variants) {
+            const int h = precision == ALTO_PREC_F64   ? own_seg<double, double>(t, mode, R, factors, v)
+                          : precision == ALTO_PREC_F32 ? own_seg<float, float>(t, mode, R, factors, v)
+                                                       : own_seg<bf16_t, float>(t, mode, R, factors, v);
             for (int sg : segs) {
                 if (sg * 4 < h || sg > h * 4) continue;
                 if (st != ALTO_OK) break;
@@ -421,6 +441,7 @@ int alto_mttkrp_autotune(alto_tensor_t* t, uint64_t rank, int precision, const v
                     bs = sg;
                 }
             }
+        }
         if (st != ALTO_OK) break;
         if (bv >= 0) t->tuned.push_back({mode, R, precision, bv, bs});
         if (result) {

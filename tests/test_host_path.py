@@ -200,3 +200,28 @@ out["lanes"], out["refused"] = lanes, [L.alto_tune_set(10, v) for v in (-2, 129)
     shipped, narrow, restored = out["lanes"][:8], out["lanes"][8:16], out["lanes"][16:]
     assert len(out["lanes"]) == 24 and shipped == restored != narrow
     assert all(v != 0 for v in out["refused"])
+
+
+@pytest.mark.parametrize("R,prec,nnz,kernel", [(1, 0, 20_000_000, "k_mttkrp<"), (25, 2, 20_000_000, "k_mttkrp<"),
+                                               (16, 0, 20_000_000, "k_mttkrp<"), (16, 0, 10_000, "k_mttkrp16<"),
+                                               (64, 2, 20_000_000, "k_mttkrp16<")])
+def test_autotune_tries_each_mapping_around_its_own_rule(host, R, prec, nnz, kernel):
+    """Segment lengths from a quarter to four times the length each kernel takes
+    by itself are among the ones tried (the first two launches are the default's)."""
+    strided = kernel == "k_mttkrp<"
+    out = host(f'''
+dims, tried = [3000, 2000, 1000], []
+seen.append(lambda x: tried.append(x.arg(0, C.c_uint64 * 15)[14]) if "{'8k_mttkrpI' if strided else '10k_mttkrp16I'}" in x.name
+            else None)
+A.check(L.alto_tune_set(13, 0), "no fibers")
+A.check(L.alto_tune_set(4, {0 if strided else -1}), "variant")
+t = tensor(dims, {nnz})
+A.check(mttkrp(t, dims, {R}, 0, {prec}), "mttkrp")
+A.check(L.alto_tune_set(4, -1), "variant")
+out["own"] = tried.pop()
+tried.clear()
+A.check(L.alto_mttkrp_autotune(t.h, {R}, {prec}, A._ptr_array([1 << 20] * 3), 1 << 20, 1, None, None), "autotune")
+out["tried"] = sorted(set(tried))
+''')
+    window = [s for s in (16 << k for k in range(9)) if out["own"] <= 4 * s and s <= 4 * out["own"]]
+    assert set(window) <= set(out["tried"]), out

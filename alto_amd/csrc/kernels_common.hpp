@@ -273,6 +273,9 @@ inline int fill_zero(T* p, uint64_t n, hipStream_t s) { return fill_value<T>(p, 
 // entry points implemented in mttkrp.hip and phi.hip
 int check_offsets(const alto_tensor* t, int R);
 int phi_variant();
+// a `variant` of phi_device_cached beside the knob's values: as 1, but with the
+// lane groups' kernel (and its unpadded product cache) at every rank
+constexpr int PHI_LANE_GROUPS = 3;
 int mttkrp_device(alto_tensor* t, int mode, int R, const void* const* U, void* out, int precision, int accumulate,
                   hipStream_t s, int seg);
 int phi_device(alto_tensor* t, int mode, int R, const double* const* U, double* phi, double eps, hipStream_t s, int seg);

@@ -19,11 +19,13 @@ typedef void (*launch_fn)(const char* name, uint32_t grid, uint32_t block, void*
 static launch_fn on_launch;
 static int mallocs, fail_from = -1; /* allocations so far; the first one that fails */
 static uint64_t live, limit = ~0ull; /* bytes allocated, and how many may be */
+static uint64_t said_free = 288ull << 30; /* what hipMemGetInfo says */
 static int in_flight;                /* operations nothing has waited for */
 
 void host_hip_on_launch(launch_fn f) { on_launch = f; }
 void host_hip_fail_from(int n) { fail_from = n < 0 ? -1 : mallocs + n; }
 void host_hip_limit(uint64_t bytes) { limit = bytes; }
+void host_hip_say_free(uint64_t bytes) { said_free = bytes; }
 uint64_t host_hip_live(void) { return live; }
 int host_hip_mallocs(void) { return mallocs; }
 int host_hip_in_flight(void) { return in_flight; }
@@ -71,7 +73,12 @@ err_t hipFree(void* p)
 }
 err_t hipHostMalloc(void** p, size_t n, unsigned flags) { return (*p = calloc(1, n)) ? OK : OOM; }
 err_t hipHostFree(void* p) { free(p); return OK; }
-err_t hipMemGetInfo(size_t* fr, size_t* total) { *fr = *total = 288ull << 30; return OK; }
+err_t hipMemGetInfo(size_t* fr, size_t* total)
+{
+    *total = 288ull << 30;
+    *fr = said_free;
+    return OK;
+}
 static void copy(void* dst, const void* src, size_t n, int kind)
 {
     /* device memory that nothing was copied to reads as zeros */

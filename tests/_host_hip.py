@@ -15,7 +15,7 @@ import ctypes as C, json, sys
 sys.path.insert(0, sys.argv[2])
 H = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)  # ahead of the real runtime for every later library
 H.host_hip_room.restype = H.host_hip_live.restype = C.c_uint64
-H.host_hip_room.argtypes = H.host_hip_limit.argtypes = [C.c_uint64]
+H.host_hip_room.argtypes = H.host_hip_limit.argtypes = H.host_hip_say_free.argtypes = [C.c_uint64]
 import numpy as np
 import alto_amd as A
 L = A.lib()

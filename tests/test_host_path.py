@@ -225,3 +225,25 @@ out["tried"] = sorted(set(tried))
 ''')
     window = [s for s in (16 << k for k in range(9)) if out["own"] <= 4 * s and s <= 4 * out["own"]]
     assert set(window) <= set(out["tried"]), out
+
+
+@pytest.mark.parametrize("R", [3, 5, 8, 13])
+def test_cp_apr_keeps_products_where_they_fit_unpadded(host, R):
+    """The one-nonzero-per-lane Phi pads odd ranks and the last nonzeros in its
+    product cache; where only nnz x rank doubles fit half the free memory, the
+    products are kept all the same."""
+    out = host(f'''
+n, dims = 1_000_003, [300, 200, 100]
+launched = []
+seen.append(lambda x: launched.append(x.name) if "k_phi_" in x.name else None)
+t = tensor(dims, n)
+for key, room in (("tight", n * {R}), ("ample", (n + 64) * {R + 1}), ("none", n * {R} - 1)):
+    H.host_hip_say_free(2 * 8 * room)
+    launched.clear()
+    t.cp_apr([np.ones((d, {R})) for d in dims], np.ones({R}), 1, 10)
+    out[key] = sorted(set(launched))
+''')
+    # (the last template argument: 0 = no products, 1 = stored)
+    assert len(out["tight"]) == 1 and "k_phi_b" in out["tight"][0] and "ELi1EEEv" in out["tight"][0]
+    assert len(out["ample"]) == 1 and "k_phi_cols" in out["ample"][0] and "ELi1EEEv" in out["ample"][0]
+    assert len(out["none"]) == 1 and "ELi0EEEv" in out["none"][0]

@@ -1,7 +1,8 @@
 // ALTO format construction on gfx950: linearization (bit deposit) and
 // delinearization (bit extract) as byte-LUT bit permutations, the sort by key
-// (sort.hip), line-balanced partition pointers, partition intervals, conflict-resolution (CR) bits, and the per-mode
-// chunk-ordered nonzero streams consumed by MTTKRP / Phi.
+// (sort.hip), line-balanced partition pointers, partition intervals,
+// conflict-resolution (CR) bits, and the per-mode chunk-ordered nonzero streams
+// consumed by MTTKRP / Phi.
 //
 // Reference behaviour followed: create_alto (include/alto.hpp:108-294),
 // setup_packed_alto (:669-770), sort_alto (:772-803), prtn_alto (:805-1028).

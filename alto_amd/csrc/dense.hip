@@ -1212,7 +1212,7 @@ int normsq_device(const double* v, uint64_t n, double* part, double* out, hipStr
 //   - up to rank 32 every row-solve block inverts V for itself while its rows
 //     of M are on their way (fuse_inverse),
 //   - every Gram block takes lambda from the row solves' partials itself
-//     (fuse_lambda: at most 2048 of each, 16 KB per block),
+//     (fuse_lambda: at most 2048 sums and 2048 maxima, 32 KB per block),
 //   - the Gram stays in partials, which the blocks of the next mode's row
 //     solves (and the fit) add up for themselves, in the same order, and the
 //     Gram launch clears the next M in blocks of its own,

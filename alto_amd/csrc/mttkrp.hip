@@ -3,13 +3,17 @@
 //
 // Layout: the nonzeros of each ALTO chunk (2^chunk_log2 consecutive nonzeros
 // in ALTO order) are stored, per target mode, sorted by that mode's row
-// (stable), as packed coordinates + value.  A lane group of G lanes (G =
-// power of two >= rank, up to 64; E elements per lane) walks a contiguous
-// range of the stream: batches of G nonzeros are loaded coalesced (one per
-// lane) and broadcast with ds_bpermute; the Hadamard product of the input
-// factor rows is formed with row-contiguous gathers (lane r reads column r);
-// contributions are reduced in registers while the output row stays the same
-// and flushed with one hardware FP atomic per column when it changes.
+// (stable), as packed coordinates + value; with the fiber layout by row and
+// fiber row.  A lane group of G lanes (a power of two; E columns of the rank
+// per lane) walks a contiguous range of the stream: batches of G nonzeros are
+// loaded coalesced and decoded (one per lane) and their fields broadcast
+// through DPP or readlane; the Hadamard product of the input factor rows is
+// formed with one vector load per lane and row; contributions are summed in
+// registers while the output row stays the same.  When it changes, the sums
+// change places in LDS, so that hardware FP atomics go to consecutive columns,
+// and a workgroup's last rows are combined before they are flushed.  (Mappings
+// 0 and 1 of launch_mttkrp broadcast through LDS permutes and flush each
+// group's rows directly.)
 // Workgroups are mapped XCD-aware: the 8 XCDs each walk one contiguous eighth
 // of the stream so that each XCD's L2 holds the factor rows of its region.
 //

@@ -22,7 +22,7 @@ struct MttkrpTune {
     int hot_block = 512;    // threads per workgroup of the ranked-stream kernel
     int hot_lds = 49152;    // LDS bytes per workgroup for hot rows
     int narrow_max = -1;    // FP32 / BF16 ranks that use two columns per lane, -1 = per element type
-    int narrow_small = 1;   // ... and every rank below 1M nonzeros
+    int narrow_small = 1;   // ... and every rank below 128K nonzeros
 };
 
 // Column mapping of a lane group: strided (lane gl holds c = gl + q*G, so

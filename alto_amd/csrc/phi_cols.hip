@@ -1,5 +1,5 @@
 // CP-APR Phi with one nonzero per lane and the rank's columns in registers
-// (ranks 2 to 32), over the per-mode nonzero streams (layout: mttkrp.hip).
+// (ranks 2 to 16), over the per-mode nonzero streams (layout: mttkrp.hip).
 //
 // Reference semantics: CalculatePhi_alto_par (include/apr.hpp:295-303,
 // :383-501); the products kept per nonzero are its PRE mode

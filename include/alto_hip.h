@@ -163,9 +163,12 @@ int alto_coo_mttkrp(int nmodes, const uint64_t* dims, uint64_t nnz, const uint64
  * wave, so fewer rounds of FP64 row flushes), above it four (BF16 above rank
  * 32: eight); -1 (default) = 16 for FP32 and 32 for BF16.
  * ALTO_TUNE_PHI_VARIANT: CP-APR Phi kernel, 0 = runtime batch loop with LDS
- * permutes, 1 = compile-time batch with DPP broadcasts (default), 2 = 16-byte
- * lanes with the model row reloaded only where the row changes (even ranks
- * and 16-byte aligned factors; others take 1).
+ * permutes, 1 (default) = one nonzero per lane with the columns in registers
+ * (ranks 2-16 with the products kept, 2-10 without; it has no segments, so
+ * ALTO_TUNE_SEG does not apply to it), else a compile-time batch with DPP
+ * broadcasts, 2 = 16-byte lanes with the model row reloaded only where the row
+ * changes (even ranks and 16-byte aligned factors; others take the
+ * compile-time batch).
  * ALTO_TUNE_NARROW_SMALL: 1 (default) = below 128K nonzeros every FP32 / BF16
  * rank uses two columns per lane.
  * ALTO_TUNE_FIBERS: 1 (default) = mode streams of tensors with at least
@@ -190,7 +193,7 @@ int alto_coo_mttkrp(int nmodes, const uint64_t* dims, uint64_t nnz, const uint64
  * ALTO_TUNE_APR_PI_CACHE: 1 (default) = CP-APR stores, at the first inner
  * iteration of each mode, the product of the other modes' factor rows for
  * every nonzero (nnz x rank doubles, when that fits in half the free device
- * memory and 64 GiB) and streams it in the mode's later inner iterations
+ * memory and 64 GiB; padded to even ranks where that fits too) and streams it in the mode's later inner iterations
  * instead of gathering those rows again (the reference's precomputed rows,
  * include/apr.hpp:1049-1165); 0 = gather them every time.
  * ALTO_TUNE_LOCKSTEP_DENSE_BATCH: 1 (default) = alto_cpd_sessions_iterate

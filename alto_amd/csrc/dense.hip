@@ -1209,7 +1209,7 @@ int normsq_device(const double* v, uint64_t n, double* part, double* out, hipStr
 // In general five launches: inverse, row solves, lambda, scaling + Gram,
 // partial sums + clearing of the next M.  Small modes are bound by the launches
 // themselves (2 to 8 us each and a gap behind it), so there
-//   - up to rank 32 every row-solve block inverts V for itself while its rows
+//   - up to rank 16 every row-solve block inverts V for itself while its rows
 //     of M are on their way (fuse_inverse),
 //   - every Gram block takes lambda from the row solves' partials itself
 //     (fuse_lambda: at most 2048 sums and 2048 maxima, 32 KB per block),
@@ -1220,17 +1220,32 @@ int normsq_device(const double* v, uint64_t n, double* part, double* out, hipStr
 // 16: the dense kernels of a mode step 31 -> 23 us in 2 launches instead of 5;
 // 1000 rows, rank 16, one model: 23 -> 16.5 us.  (A single workgroup doing the
 // whole update took 18.6 us for those 1000 rows, bound by what one CU can load
-// and store.)  Where the lines lie, whole mode updates of three equal modes
-// just below and above each: inverse in the row solves, rank 16, 32768 rows 59
-// against 63 us, rank 32, 16384 rows 80.5 and 32768 rows 90 against 82 us;
-// lambda in the Gram launch, rank 16, 8192 rows 52.3 against 52.1 us, rank 64,
-// 2048 rows 112 against 111 us (so it ends there); Gram in partials, rank 16,
-// 2048 rows 48 us, 4096 rows 51.5 against 50.4 us.
-static bool fuse_inverse(uint64_t I, int R) { return R <= 32 && solve_blocks(I, R) <= (R <= 16 ? 512 : 256); }
-static bool fuse_lambda(uint64_t I, int R) { return solve_blocks(I, R) * R <= 2048; }
+// and store.)  Where the lines lie:
+//   - inverse in the row solves.  Above rank 16 it takes all four wavefronts of
+//     a block longer than one workgroup of sixteen and a launch: iterations of
+//     three modes (3000, 5000, 200 rows) at rank 25 206 against 191 us, rank 32
+//     217 against 199.  At rank 16 it holds up to 32768 rows (181 against 191 us,
+//     three equal modes).  Many models at once are bound by the inverses
+//     themselves: 16 models of three modes of 16000 rows (4000 blocks), rank 16,
+//     557 against 541 us, 8000 rows (2000 blocks) 358, 359: above 2048 blocks in
+//     all the batch takes the inverse's own launch (the values are the same).
+//   - lambda in the Gram launch, rank 16: 8192 rows 52.3 against 52.1 us (whole
+//     update); rank 64, 2048 rows 112 against 111; rank 4 and 8, iterations,
+//     8000 rows 148 against 146 and 149, 147, 16000 rows 161, 150 and 164, 154:
+//     128 partials of at most 2048 numbers.
+//   - Gram in partials, rank 16: 2048 rows 48 us, 4096 rows 51.5 against 50.4.  A
+//     block adds them one behind the other, so their number counts and not their
+//     size: at rank 4, 32 partials (8000 rows) 168 against 148 us an iteration,
+//     125 (32000 rows) 275 against 192, 16 models 1032 against 532.
+static bool fuse_inverse(uint64_t I, int R) { return R <= 16 && solve_blocks(I, R) <= 512; }
+static bool fuse_lambda(uint64_t I, int R)
+{
+    const int nb = solve_blocks(I, R);
+    return nb <= 128 && nb * R <= 2048;
+}
 bool gram_can_stay_partial(uint64_t I, int R, uint64_t next_I)
 {
-    return fuse_inverse(next_I, R) && (uint64_t)gram_blocks(I) * R * R <= 2048;
+    return fuse_inverse(next_I, R) && gram_blocks(I) <= 8;
 }
 
 template <typename J, int N>
@@ -1320,13 +1335,13 @@ __global__ void __launch_bounds__(256) k_apply_batch(BatchTab<ApplyJob, N> t, in
                                   t.start[k + 1] - t.start[k]);
 }
 
-// Row solves that invert V themselves (R <= 32).  V is put together in LDS by
+// Row solves that invert V themselves (R <= 16).  V is put together in LDS by
 // all threads; the model's first block leaves a pending Gram's sum in its place.
 // The pseudo-inverse of a failed pivot is every block's own too, in LDS.
-template <typename UT, int T16, bool LOWP, int N>
+template <typename UT, bool LOWP, int N>
 __global__ void __launch_bounds__(256) k_solve_batch(BatchTab<SolveJob, N> t, int R)
 {
-    constexpr int C = 16 * T16;
+    constexpr int C = 16;
     __shared__ double s_v[C * C], s_p[C * C], s_q[C * C];
     const int k = batch_job(t, blockIdx.x);
     const SolveJob& j = t.a[k];
@@ -1349,7 +1364,7 @@ __global__ void __launch_bounds__(256) k_solve_batch(BatchTab<SolveJob, N> t, in
             }
         }
         __syncthreads();
-        const bool ok = spd_inverse<T16 == 1 ? 0 : 4 * T16, 1>(
+        const bool ok = spd_inverse<0, 1>(
             R, [&](int i, int c) { return s_v[i * R + c]; }, [&](int i, int c, double v) { sW[i * WS + c] = (T)v; });
         if (threadIdx.x == 0 && bid == 0) *j.status = ok ? 0 : 1;
         if (!ok) {  // uniform
@@ -1364,8 +1379,8 @@ __global__ void __launch_bounds__(256) k_solve_batch(BatchTab<SolveJob, N> t, in
         }
         __syncthreads();
     };
-    apply_body<double, UT, T16, LOWP>(j.x.M, j.x.I, R, prepare, (UT*)j.x.U, j.x.psum, j.x.pmax, j.x.pin, bid,
-                                      t.start[k + 1] - t.start[k]);
+    apply_body<double, UT, 1, LOWP>(j.x.M, j.x.I, R, prepare, (UT*)j.x.U, j.x.psum, j.x.pmax, j.x.pin, bid,
+                                    t.start[k + 1] - t.start[k]);
 }
 
 template <int N>
@@ -1446,18 +1461,17 @@ static int mode_solve(int n, const DenseModeJob* m, int R, hipStream_t s)
     BatchTab<SpdJob, N> sp{};
     BatchTab<ApplyJob, N> ap{};
     BatchTab<SolveJob, N> so{};
+    int blocks = 0;
+    for (int k = 0; k < n; ++k) blocks += m[k].nb;
+    const bool few = blocks <= 2048;  // (a Gram in partials needs the row solves' sum all the same)
     for (int k = 0; k < n; ++k) {
         const DenseModeJob& x = m[k];
         const ApplyJob a{x.M, x.P, x.U, x.psum, x.pmax, x.pin, x.I};
-        if (fuse_inverse(x.I, R)) {
+        if (x.pend.mode >= 0 || (few && fuse_inverse(x.I, R))) {
             so.a[so.n] = SolveJob{x.pend, a, x.grams, x.status, x.nmode, x.mode};
             so.start[so.n + 1] = so.start[so.n] + (uint32_t)x.nb;
             ++so.n;
             continue;
-        }
-        if (x.pend.mode >= 0) {
-            set_error("mode update: a Gram in partials before a mode of %llu rows", (unsigned long long)x.I);
-            return ALTO_ERR_UNSUPPORTED;
         }
         sp.a[sp.n++] = SpdJob{x.grams, x.P, x.wsA, x.wsQ, x.status, x.nmode, x.mode};
         ap.a[ap.n] = a;
@@ -1467,19 +1481,13 @@ static int mode_solve(int n, const DenseModeJob* m, int R, hipStream_t s)
     const size_t lds = (size_t)R * (R + 2) * 8;
     const bool lowp = std::is_same<UT, float>::value && !dense_f64_enabled();
     if (so.n) {
-#define SO_(TT, L) hipLaunchKernelGGL((k_solve_batch<UT, TT, L, N>), dim3(so.start[so.n]), dim3(256), lds, s, so, R)
-#define SOT_(TT)                                         \
-    do {                                                 \
-        if constexpr (std::is_same<UT, float>::value) {  \
-            if (lowp) SO_(TT, true);                     \
-            else SO_(TT, false);                         \
-        } else {                                         \
-            SO_(TT, false);                              \
-        }                                                \
-    } while (0)
-        if (R <= 16) SOT_(1);
-        else SOT_(2);
-#undef SOT_
+#define SO_(L) hipLaunchKernelGGL((k_solve_batch<UT, L, N>), dim3(so.start[so.n]), dim3(256), lds, s, so, R)
+        if constexpr (std::is_same<UT, float>::value) {
+            if (lowp) SO_(true);
+            else SO_(false);
+        } else {
+            SO_(false);
+        }
 #undef SO_
     }
     if (ap.n) {

@@ -125,3 +125,30 @@ def test_pseudo_inverse_of_half_rank(R):
     want = M @ np.linalg.pinv(V, rcond=1e-10, hermitian=True)
     assert fb.value == 1
     np.testing.assert_allclose(d.numpy(), want, rtol=0, atol=64 * R * EPS * e[-1] / e[0] * np.abs(want).max())
+
+
+@pytest.mark.parametrize("R,prec", [(3, 0), (16, 0), (16, 1), (9, 2)])
+def test_many_row_solve_blocks_equal_one_model(R, prec):
+    """Five models in lockstep, whose modes of 32768 rows together pass the number
+    of blocks up to which row solves invert V themselves, against the same models
+    one by one (512 blocks each, which do): the same bits, MTTKRPs in a fixed
+    order."""
+    A = _A()
+    L = A.lib()
+    dims = [32768, 60, 32768]
+    tensors = [A.AltoTensor(dims, *uniform_tensor(dims, 5000, k)) for k in range(5)]
+    U = [oracle.random_init(dims, R, 3 + k)[0] for k in range(5)]
+    A.check(L.alto_tune_set(18, 1), "deterministic")
+    try:
+        one = [A.CpdSession(t, u, prec) for t, u in zip(tensors, U)]
+        for s in one:
+            s.iterate(3)
+        many = [A.CpdSession(t, u, prec) for t, u in zip(tensors, U)]
+        A.cpd_sessions_iterate(many, 3, 0.0)
+    finally:
+        A.check(L.alto_tune_set(18, 0), "deterministic")
+    for a, b in zip(one, many):
+        (Ua, la, fa, _), (Ub, lb, fb, _) = a.get(), b.get()
+        assert fa == fb and np.array_equal(la, lb)
+        for x, y in zip(Ua, Ub):
+            np.testing.assert_array_equal(x, y)

@@ -1160,7 +1160,14 @@ inline void launch_batch_table(const BatchTable<FT, VT, OT>& tab, int G, int pw,
 // lane shape (G in 2..64, E, key width) share launches of up to
 // MTTKRP_BATCH_MAX jobs; the others are launched one by one through
 // launch_mttkrp.  Segment lengths: `seg` when positive, else the size rule
-// of each tensor.
+// of each tensor, which gives a launch of its own enough wavefronts; many
+// tensors together have them anyway, and what a short segment costs is the
+// flush at its end.  So above rank 16 segments are lengthened, to 64 at most,
+// while the launch has more than 2^15 wavefronts: 16 tensors of three modes, FP64,
+// 4000 rows and 100K nonzeros at ranks 32, 48, 64 137, 187, 198 -> 124, 168, 182
+// us; 16000 rows, 200K 235, 402, 460 -> 220, 354, 440; FP32 181, 248, 296 -> 181,
+// 220, 264.  (Up to rank 16 it depends on the rows: uniform 16000, 200K, rank 16
+// 156 at 16 against 151; Zipf 1M, rank 8 262 at 32 against 222.)
 template <typename FT, typename VT, typename AT, typename OT>
 int launch_mttkrp_batch(int n, alto_tensor* const* ts, const int* modes, int R, const FT* const* const* U,
                         const VT* const* vals, OT* const* outs, int seg, const MttkrpTune& k, hipStream_t s)
@@ -1198,16 +1205,26 @@ int launch_mttkrp_batch(int n, alto_tensor* const* ts, const int* modes, int R, 
         }
         g->jobs.push_back(a);
     }
-    for (const auto& g : groups) {
+    for (auto& g : groups) {
         for (size_t j0 = 0; j0 < g.jobs.size(); j0 += MTTKRP_BATCH_MAX) {
             BatchTable<FT, VT, OT> tab;
             tab.n = (int)std::min<size_t>(MTTKRP_BATCH_MAX, g.jobs.size() - j0);
-            uint64_t total = 0;
+            uint64_t total = 0, nnz = 0;
+            for (int j = 0; j < tab.n; ++j) nnz += g.jobs[j0 + j].nnz;
+            uint64_t least = 1;  // segment length
+            if (seg <= 0 && R > 16)
+                while (least < 64 && nnz * (uint64_t)g.G / (64 * least) > (1u << 15)) least <<= 1;
+            for (int j = 0; j < tab.n; ++j) {
+                StreamArgs<FT, VT, OT>& a = g.jobs[j0 + j];
+                if (a.seg >= least) continue;
+                a.seg = least;
+                (void)stream_grid(a.nnz, (int)least, g.G, a);
+            }
             for (int j = 0; j < MTTKRP_BATCH_MAX; ++j) {
                 if (j < tab.n) tab.a[j] = g.jobs[j0 + j];
                 else tab.a[j] = g.jobs[j0];  // unused entries
                 tab.start[j] = (uint32_t)total;
-                if (j < tab.n) total += g.jobs[j0 + j].nblocks_real;
+                if (j < tab.n) total += tab.a[j].nblocks_real;
             }
             tab.start[MTTKRP_BATCH_MAX] = (uint32_t)total;
             for (int j = tab.n; j <= MTTKRP_BATCH_MAX; ++j) tab.start[j] = (uint32_t)total;

@@ -123,3 +123,31 @@ def test_batched_arguments():
         A.mttkrp_batched([g], [3], [U], 0)
     with pytest.raises(A.AltoError):
         A.mttkrp_batched([g], [0], [U], 7)
+
+
+@pytest.fixture(scope="module")
+def sixteen():
+    """Tensors whose launch together takes longer segments than theirs alone."""
+    return [(d, *uniform_tensor(d, 80_000, 40 + k)) for k, d in
+            enumerate([[400 + 7 * k, 900, 3000] if k % 2 else [50 + k, 60, 70, 300] for k in range(16)])]
+
+
+@pytest.mark.parametrize("prec", [0, 1, 2])
+@pytest.mark.parametrize("R", [17, 33, 48, 64])
+def test_batched_longer_segments(sixteen, prec, R):
+    A = _alto()
+    rng = np.random.default_rng(R)
+    ts = [A.AltoTensor(*x) for x in sixteen]
+    Us = [[rng.random((d, R)) for d in dims] for dims, _, _ in sixteen]
+    if prec == A.PREC_F32:
+        Us = [[u.astype(np.float32).astype(np.float64) for u in U] for U in Us]
+    elif prec == A.PREC_BF16:
+        Us = [[A.from_bf16_bits(A.to_bf16_bits(u)).astype(np.float64) for u in U] for U in Us]
+    eps = 2.0 ** -52 if prec == A.PREC_F64 else 2.0 ** -23
+    got = A.mttkrp_batched(ts, [k % 3 for k in range(16)], Us, prec)
+    for k, ((dims, cidx, vals), U, x) in enumerate(zip(sixteen, Us, got)):
+        want = mttkrp_numpy(cidx, vals, U, k % 3)
+        # positive terms: value, factors and products rounded on each one's way;
+        # 32-bit sums run over at most 4096 terms before they go on in 64 bits
+        bound = want * eps * (len(dims) + 2 + (len(vals) if prec == A.PREC_F64 else 4096))
+        assert (np.abs(x - want) <= bound).all(), (k, dims)

@@ -247,3 +247,30 @@ for key, room in (("tight", n * {R}), ("ample", (n + 64) * {R + 1}), ("none", n 
     assert len(out["tight"]) == 1 and "k_phi_b" in out["tight"][0] and "ELi1EEEv" in out["tight"][0]
     assert len(out["ample"]) == 1 and "k_phi_cols" in out["ample"][0] and "ELi1EEEv" in out["ample"][0]
     assert len(out["none"]) == 1 and "ELi0EEEv" in out["none"][0]
+
+
+@pytest.mark.parametrize("R,prec,n,nnz,knob,segs", [
+    (48, 0, 4, 100_000, 0, 16), (48, 0, 16, 100_000, 0, 32), (48, 0, 16, 200_000, 0, 64), (48, 0, 16, 3_000_000, 0, 128),
+    (48, 0, 16, 100_000, 24, 24), (16, 0, 16, 100_000, 0, 8), (32, 0, 16, 100_000, 0, 16), (64, 1, 16, 200_000, 0, 32),
+    (64, 2, 16, 200_000, 0, 16), (64, 0, 16, 5_000, 0, 16)])
+def test_batched_segments(host, R, prec, n, nnz, knob, segs):
+    """Segment lengths of a launch of many tensors: each tensor's own rule until
+    the launch has more wavefronts than it needs, then longer ones."""
+    out = host(f'''
+dims, found, left = [300, 200, 100], [], []
+def look(x):
+    if "k_mttkrp16_batch" in x.name:
+        a = x.arg(0, C.c_uint64 * (22 * 16 + 9))
+        found.extend(a[22 * j + 14] for j in range({n}))
+        # every nonzero has a lane group
+        G = int(x.name.split("Li")[1].split("E")[0])
+        left.extend(-(-a[22 * j + 13] // a[22 * j + 14]) * G > a[22 * j + 15] * 256 for j in range({n}))
+seen.append(look)
+A.check(L.alto_tune_set(1, {knob}), "segments")
+ts = [tensor(dims, {nnz}) for _ in range({n})]
+f = A._ptr_array([1 << 20] * 3)
+st = L.alto_mttkrp_batched({n}, A._ptr_array([t.h for t in ts]), (C.c_int * {n})(*([0] * {n})), {R},
+                           A._ptr_array([C.addressof(f)] * {n}), A._ptr_array([1 << 20] * {n}), {prec}, 0, None)
+out.update(status=st, segs=sorted(set(found)), count=len(found), left=sum(left))
+''')
+    assert out == dict(status=0, segs=[segs], count=n, left=0)

@@ -60,6 +60,18 @@ struct DevBuf {
     template <class T> T* as() const { return reinterpret_cast<T*>(p); }
 };
 
+// Waits for a stream at the end of a scope, whichever way out: declared behind
+// the buffers that are released there and ahead of the first work that uses
+// them.  (on = false: nothing to wait for.)
+struct Drain {
+    hipStream_t s;
+    bool on = true;
+    ~Drain()
+    {
+        if (on) (void)hipStreamSynchronize(s);
+    }
+};
+
 // ---------------------------------------------------------------- tensor layout
 // Packed-coordinate layout used by the per-mode streams: mode n occupies bits
 // [off[n], off[n]+bits[n]) of a 64-bit word (pw==1) or of a 128-bit pair (pw==2).

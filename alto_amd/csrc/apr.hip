@@ -272,6 +272,7 @@ int cp_apr_impl(alto_tensor* t, int R, int max_iters, int max_inner, double epsi
     }
     const double tp0 = now_s();
     AprState c;
+    const Drain drain{s};
     c.N = t->nmode;
     c.R = R;
     const int N = c.N;
@@ -566,6 +567,7 @@ extern "C" int alto_kruskal_normalize(int nmodes, const uint64_t* dims, uint64_t
     const int R = (int)rank;
     const bool host = ptr_kind == ALTO_PTR_HOST;
     DevBuf part, norm, lam, Ud[ALTO_MAXN];
+    const Drain drain{s};
     ALTO_TRY(part.alloc((size_t)COL_BLOCKS * R * 8));
     ALTO_TRY(norm.alloc((size_t)R * 8));
     double* ld = lambda;
@@ -586,7 +588,7 @@ extern "C" int alto_kruskal_normalize(int nmodes, const uint64_t* dims, uint64_t
         if (host) HIP_TRY(hipMemcpyAsync(U[m], u, dims[m] * R * 8, hipMemcpyDeviceToHost, s));
     }
     if (host) HIP_TRY(hipMemcpyAsync(lambda, ld, (size_t)R * 8, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));  // temporaries are released below
+    HIP_TRY(hipStreamSynchronize(s));
     return ALTO_OK;
 }
 

@@ -80,6 +80,7 @@ extern "C" int alto_coo_mttkrp(int nmodes, const uint64_t* dims, uint64_t nnz, c
     for (int m = 0; m < nmodes; ++m) a.dims[m] = dims[m];
     const bool host = ptr_kind == ALTO_PTR_HOST;
     DevBuf ci[ALTO_MAXN], Ud[ALTO_MAXN], vd, od;
+    const Drain drain{s, host};
     if (host) {
         // host coordinates are checked here; on the device a nonzero with a
         // coordinate out of range is skipped
@@ -129,7 +130,7 @@ extern "C" int alto_coo_mttkrp(int nmodes, const uint64_t* dims, uint64_t nnz, c
     }
     if (host) {
         HIP_TRY(hipMemcpyAsync(out, od.p, dims[mode] * rank * 8, hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));  // temporaries are released below
+        HIP_TRY(hipStreamSynchronize(s));
     }
     return ALTO_OK;
 }

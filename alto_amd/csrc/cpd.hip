@@ -144,13 +144,13 @@ static int cpd_upload(alto_tensor* t, CpdState<UT, ST, MT>& c, double* const* Uh
 {
     const int R = c.R;
     std::vector<UT> tmp;
-    DevBuf ones;
+    DevBuf ones, d64;
+    Drain drain{s};
     ALTO_TRY(ones.alloc(R * 8));
     ALTO_TRY(fill_value<double>(ones.as<double>(), R, 1.0, s));
     for (int m = 0; m < c.N; ++m) {
         uint64_t n = t->dims[m] * R;
         if (!Uh) {  // seeded on the device (counter-based), then converted
-            DevBuf d64;
             double* dst = std::is_same<UT, double>::value ? reinterpret_cast<double*>(c.U[m].p) : nullptr;
             if (!dst) {
                 ALTO_TRY(d64.alloc(n * 8));
@@ -174,6 +174,7 @@ static int cpd_upload(alto_tensor* t, CpdState<UT, ST, MT>& c, double* const* Uh
                                  c.gpart.template as<double>(), s, gram_f64(c.prec)));
     }
     HIP_TRY(hipStreamSynchronize(s));
+    drain.on = false;
     return ALTO_OK;
 }
 

@@ -165,14 +165,6 @@ alto_tensor::~alto_tensor()
 
 namespace alto {
 
-// Waits for a stream at the end of a scope, whichever way out: declared behind
-// the buffers that are released there and ahead of the first work that uses
-// them.
-struct Drain {
-    hipStream_t s;
-    ~Drain() { (void)hipStreamSynchronize(s); }
-};
-
 // ------------------------------------------------------------------ masks
 // setup_packed_alto(at, LSB_FIRST, SHORT_FIRST): modes ordered by bit count
 // (stable), one bit per still-active mode per level, LSB first.

@@ -193,9 +193,10 @@ int alto_coo_mttkrp(int nmodes, const uint64_t* dims, uint64_t nnz, const uint64
  * ALTO_TUNE_APR_PI_CACHE: 1 (default) = CP-APR stores, at the first inner
  * iteration of each mode, the product of the other modes' factor rows for
  * every nonzero (nnz x rank doubles, when that fits in half the free device
- * memory and 64 GiB; padded to even ranks where that fits too) and streams it in the mode's later inner iterations
- * instead of gathering those rows again (the reference's precomputed rows,
- * include/apr.hpp:1049-1165); 0 = gather them every time.
+ * memory and 64 GiB; padded to even ranks where that fits too) and streams it
+ * in the mode's later inner iterations instead of gathering those rows again
+ * (the reference's precomputed rows, include/apr.hpp:1049-1165); 0 = gather
+ * them every time.
  * ALTO_TUNE_LOCKSTEP_DENSE_BATCH: 1 (default) = alto_cpd_sessions_iterate
  * at rank <= 64 runs each mode's R x R solves, row solves, normalisations and
  * Gram updates of all its sessions in one launch per kernel, and their fits

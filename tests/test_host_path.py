@@ -103,9 +103,32 @@ o = np.zeros(200_000, np.uint64)
 out["runs"] = failing(lambda: tensor([70, 50, 40], 200_000), lambda t: L.alto_tensor_export_oidx(t.h, 1, o.ctypes.data))
 '''
 
+_SEEDED = r'''
+def seeded(t):
+    h = C.c_void_p()
+    st = L.alto_cpd_session_create_seeded(t.h, 16, A.PREC_BF16, 3, None, C.byref(h))
+    if st == 0:
+        L.alto_cpd_session_destroy(h)
+    return st
+out["runs"] = failing(lambda: tensor([70, 50, 40], 200_000), seeded)
+'''
+_HOST = r'''
+dims = np.array([70, 50, 40], np.uint64)
+U, lam, res = [np.ones((d, 10)) for d in dims], np.ones(10), A.AprResult()
+up = A._ptr_array([u.ctypes.data for u in U])
+idx, vals = [np.zeros(4000, np.uint64) for d in dims], np.ones(4000)
+calls = dict(
+    apr=lambda t: L.alto_cp_apr(t.h, 10, 2, 3, 1e-5, 1e-10, 1e-10, 1e-2, 0, up, lam.ctypes.data, C.byref(res), 0, None),
+    coo=lambda t: L.alto_coo_mttkrp(3, dims.ctypes.data, 4000, A._ptr_array([i.ctypes.data for i in idx]),
+                                    vals.ctypes.data, 0, 10, up, U[0].ctypes.data, 1, 0, None),
+    kruskal=lambda t: L.alto_kruskal_normalize(3, dims.ctypes.data, 10, up, lam.ctypes.data, -1, 0, 0, None))
+out["runs"] = failing(lambda: tensor([70, 50, 40], 200_000), calls["CALL"])
+'''
 
-@pytest.mark.parametrize("body", [_CREATE, _STREAMS.replace("HOT", "0"), _STREAMS.replace("HOT", "1"), _OIDX],
-                         ids=["create", "streams", "hot rows", "oidx"])
+
+@pytest.mark.parametrize("body", [_CREATE, _STREAMS.replace("HOT", "0"), _STREAMS.replace("HOT", "1"), _OIDX, _SEEDED,
+                                  *(_HOST.replace("CALL", x) for x in ("apr", "coo", "kruskal"))],
+                         ids=["create", "streams", "hot rows", "oidx", "seeded", "apr", "coo", "kruskal"])
 def test_nothing_in_flight_when_an_allocation_fails(host, body):
     """A call that gives up hands its buffers back to the cache shared by all
     streams, so nothing that it enqueued may still be running."""

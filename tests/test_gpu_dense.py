@@ -1,8 +1,8 @@
 """GPU parity of the CP-ALS mode updates at the sizes where their launches
 change: the inverse per rank class, row solves that invert V themselves (up to
-rank 16 and 32768 rows, rank 32 and 16384), lambda taken in the Gram launch (64
-rows x rank up to 2048 x 64) and Grams left in partials (256-row blocks x rank^2
-up to 2048)."""
+rank 16 and 32768 rows), lambda taken in the Gram launch (up to 128 row blocks
+and row blocks x rank 2048) and Grams left in partials (up to 8 row blocks of
+the Gram), with sizes on both sides of those lines."""
 import ctypes
 
 import numpy as np
